@@ -141,6 +141,7 @@ def test_hip_platform_symmetric_matches_reference_platform(gpu, which, lncc):
 
 
 @pytest.mark.gpu
+@needs_plugin
 @pytest.mark.parametrize("which", ["cube", "oblique"])
 def test_hip_platform_symmetric_with_affine_matches_reference_platform(gpu, which):
     """The same calls with an input affine: the half affines in the grids' extensions (read by
