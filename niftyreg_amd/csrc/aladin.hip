@@ -990,12 +990,15 @@ void launch_symmetric_update(nrh_aladin *fw, nrh_aladin *bw) {
 
 void destroy(nrh_aladin *h);
 
-nrh_aladin *create(const nrh_geom *ref, const float *ref_data, const nrh_geom *flo, const float *flo_data,
-                   const int *mask, const nrh_aladin_params *params, hipStream_t sharedStream = nullptr) {
+// A handle over the two images, which it takes over (device) or, where a buffer is empty, uploads
+// from ref_data / flo_data (host).
+nrh_aladin *create(const nrh_geom *ref, DevBuf<float>&& refImg, const float *ref_data, const nrh_geom *flo,
+                   DevBuf<float>&& floImg, const float *flo_data, const int *mask, const nrh_aladin_params *params,
+                   hipStream_t sharedStream = nullptr) {
     check_geom(ref, "reference");
     check_geom(flo, "floating");
     check_aladin_params(params);
-    NRH_REQUIRE(ref_data && flo_data, NRH_ERR_ARG, "null image data");
+    NRH_REQUIRE((ref_data || !refImg.empty()) && (flo_data || !floImg.empty()), NRH_ERR_ARG, "null image data");
     NRH_REQUIRE(ref->nz > 1, NRH_ERR_UNSUPPORTED, "2-D images are not supported");
     std::unique_ptr<nrh_aladin> h(new nrh_aladin);
     h->ref = *ref;
@@ -1011,11 +1014,16 @@ nrh_aladin *create(const nrh_geom *ref, const float *ref_data, const nrh_geom *f
         NRH_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     }
     NRH_HIP(hipHostMalloc((void **)&h->pinned, 4 * sizeof(int), hipHostMallocDefault));
-    h->refImg.alloc(h->N);
-    h->floImg.alloc(h->Nf);
+    auto image = [&](DevBuf<float>& img, DevBuf<float>&& from, const float *data, size_t n) {
+        NRH_REQUIRE(from.empty() || from.n == n, NRH_ERR_ARG, "image sizes differ from the geometries");
+        img = std::move(from);
+        if (!img.empty()) return;
+        img.alloc(n);
+        NRH_HIP(hipMemcpyAsync(img.p, data, n * sizeof(float), hipMemcpyHostToDevice, h->stream));
+    };
+    image(h->refImg, std::move(refImg), ref_data, h->N);
+    image(h->floImg, std::move(floImg), flo_data, h->Nf);
     h->warped.alloc(h->N);
-    NRH_HIP(hipMemcpyAsync(h->refImg.p, ref_data, h->N * sizeof(float), hipMemcpyHostToDevice, h->stream));
-    NRH_HIP(hipMemcpyAsync(h->floImg.p, flo_data, h->Nf * sizeof(float), hipMemcpyHostToDevice, h->stream));
     NRH_HIP(hipMemsetAsync(h->warped.p, 0, h->warped.bytes(), h->stream));
     if (mask) {
         bool any = false;
@@ -1093,16 +1101,26 @@ void aladin_register(const nrh_geom& refG, const float *refData, const nrh_geom&
     }
     float Mb[16];
     mat44_inverse(M, Mb);
-    std::vector<Level> rp = pyramid(refG, refData, cfg.levels, toPerform);
-    std::vector<Level> fp = pyramid(floG, floData, cfg.levels, toPerform);
+    std::vector<DevLevel> rp, fp;
+    {
+        ScopedStream st;
+        rp = device_pyramid(refG, refData, cfg.levels, toPerform, st.s);
+        fp = device_pyramid(floG, floData, cfg.levels, toPerform, st.s);
+    }
     const nrh_aladin_params params{ cfg.block_percent, cfg.inlier_lts, std::numeric_limits<float>::quiet_NaN() };
     for (int level = 0; level < toPerform; ++level) {
         AladinHandle ah, bh;  // bh (sharing ah's stream) is destroyed first
-        ah.h = create(&rp[level].geom, rp[level].data.data(), &fp[level].geom, fp[level].data.data(), nullptr, &params);
+        ah.h = create(&rp[level].geom, std::move(rp[level].img), nullptr, &fp[level].geom, std::move(fp[level].img),
+                      nullptr, nullptr, &params);
         nrh_aladin *h = ah.h, *b = nullptr;
         set_matrix(h, M);
         if (cfg.symmetric) {
-            bh.h = create(&fp[level].geom, fp[level].data.data(), &rp[level].geom, rp[level].data.data(), nullptr,
+            DevBuf<float> ri, fi;
+            ri.alloc(h->N);
+            fi.alloc(h->Nf);
+            NRH_HIP(hipMemcpyAsync(ri.p, h->refImg.p, ri.bytes(), hipMemcpyDeviceToDevice, h->stream));
+            NRH_HIP(hipMemcpyAsync(fi.p, h->floImg.p, fi.bytes(), hipMemcpyDeviceToDevice, h->stream));
+            bh.h = create(&fp[level].geom, std::move(fi), nullptr, &rp[level].geom, std::move(ri), nullptr, nullptr,
                           &params, h->stream);
             b = bh.h;
             set_matrix(b, Mb);
@@ -1152,17 +1170,25 @@ void aladin_register_batch(int n, const nrh_geom *refs, const float *const *refD
     const auto t0 = std::chrono::steady_clock::now();
     const int toPerform = cfg.levels_to_perform > 0 ? std::min(cfg.levels_to_perform, cfg.levels) : cfg.levels;
     std::vector<std::array<float, 16>> M(n);
-    std::vector<std::vector<Level>> rp(n), fp(n);
+    std::vector<std::vector<DevLevel>> rp(n), fp(n);
     std::vector<std::string> errs(n);
+    std::vector<int> codes(n, NRH_ERR_ARG);
     {
+        int device = 0;
+        NRH_HIP(hipGetDevice(&device));
         std::vector<std::thread> pool;
         const int T = std::max(1, std::min(n, (int)std::thread::hardware_concurrency()));
         for (int t = 0; t < T; ++t)
             pool.emplace_back([&, t] {
                 for (int q = t; q < n; q += T) {
                     try {
-                        rp[q] = pyramid(refs[q], refData[q], cfg.levels, toPerform);
-                        fp[q] = pyramid(flos[q], floData[q], cfg.levels, toPerform);
+                        NRH_HIP(hipSetDevice(device));
+                        ScopedStream st;
+                        rp[q] = device_pyramid(refs[q], refData[q], cfg.levels, toPerform, st.s);
+                        fp[q] = device_pyramid(flos[q], floData[q], cfg.levels, toPerform, st.s);
+                    } catch (const Error& e) {
+                        errs[q] = e.what();
+                        codes[q] = e.code;
                     } catch (const std::exception& e) {
                         errs[q] = e.what();
                     }
@@ -1171,7 +1197,7 @@ void aladin_register_batch(int n, const nrh_geom *refs, const float *const *refD
         for (auto& th : pool) th.join();
     }
     for (int q = 0; q < n; ++q) {
-        NRH_REQUIRE(errs[q].empty(), NRH_ERR_ARG, "pair " + std::to_string(q) + ": " + errs[q]);
+        NRH_REQUIRE(errs[q].empty(), codes[q], "pair " + std::to_string(q) + ": " + errs[q]);
         float m[16] = { 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1 };
         if (cfg.align_centre) {
             auto centre = [](const nrh_geom& g, float c[3]) {
@@ -1206,8 +1232,8 @@ void aladin_register_batch(int n, const nrh_geom *refs, const float *const *refD
         for (int q = 0; q < n; ++q) {
             if (status[q] != NRH_OK) continue;
             try {
-                hs[q].h = create(&rp[q][level].geom, rp[q][level].data.data(), &fp[q][level].geom,
-                                 fp[q][level].data.data(), nullptr, &params, stream);
+                hs[q].h = create(&rp[q][level].geom, std::move(rp[q][level].img), nullptr, &fp[q][level].geom,
+                                 std::move(fp[q][level].img), nullptr, nullptr, &params, stream);
                 set_matrix(hs[q].h, M[q].data());
                 live.push_back(hs[q].h);
                 liveIdx.push_back(q);
@@ -1312,7 +1338,7 @@ int nrh_aladin_create(const nrh_geom *ref, const float *ref_data, const nrh_geom
     return guard([&] {
         NRH_REQUIRE(out, NRH_ERR_ARG, "null output handle");
         *out = nullptr;
-        *out = create(ref, ref_data, flo, flo_data, mask, params);
+        *out = create(ref, DevBuf<float>(), ref_data, flo, DevBuf<float>(), flo_data, mask, params);
     });
 }
 

@@ -123,6 +123,62 @@ void check_params(const nrh_f3d_params *p) {
                 "field_order must be NRH_FIELD_ORDER_SCALAR or NRH_FIELD_ORDER_SSE");
 }
 
+// The handle without its images: geometries, stream and result buffers.
+static std::unique_ptr<nrh_f3d> f3d_begin(const nrh_geom& ref, const nrh_geom& flo, const nrh_geom& cpp,
+                                          const nrh_f3d_params& params) {
+    NRH_REQUIRE(ref.nz > 1, NRH_ERR_UNSUPPORTED, "2-D images are not supported");
+    std::unique_ptr<nrh_f3d> h(new nrh_f3d);
+    h->ref = ref; h->flo = flo; h->cpp = cpp; h->params = params;
+    h->N = voxels(ref); h->Nf = voxels(flo); h->G = voxels(cpp);
+    NRH_HIP(hipGetDevice(&h->device));
+    NRH_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
+    NRH_HIP(hipHostMalloc((void **)&h->pinned, 16 * sizeof(double), hipHostMallocDefault));
+    NRH_HIP(hipHostMalloc((void **)&h->published, 16 * sizeof(double), hipHostMallocCoherent | hipHostMallocMapped));
+    NRH_HIP(hipHostGetDevicePointer((void **)&h->publishedDev, h->published, 0));
+    std::memset(h->published, 0, 16 * sizeof(double));  // published[15]: no sequence number yet
+    return h;
+}
+
+// The mask, control points and optimiser arrays, histogram and reduction scratch.
+static nrh_f3d *f3d_finish(std::unique_ptr<nrh_f3d> h, const int *mask) {
+    if (mask) {
+        bool any = false;
+        for (size_t i = 0; i < h->N && !any; ++i) any = mask[i] < 0;
+        if (any) {
+            h->mask.alloc(h->N);
+            NRH_HIP(hipMemcpyAsync(h->mask.p, mask, h->N * sizeof(int), hipMemcpyHostToDevice, h->stream));
+        }
+    }
+    h->cppPos.alloc(3 * h->G);
+    h->best.alloc(3 * h->G);
+    h->nodeGrad.alloc(3 * h->G);
+    h->cgG.alloc(3 * h->G);
+    h->cgH.alloc(3 * h->G);
+    NRH_HIP(hipMemsetAsync(h->cppPos.p, 0, h->cppPos.bytes(), h->stream));
+    NRH_HIP(hipMemsetAsync(h->nodeGrad.p, 0, h->nodeGrad.bytes(), h->stream));
+    alloc_histogram(h.get());
+    h->ent.alloc(8);
+    h->scalars.alloc(16);
+    h->maxBits.alloc(8);
+    NRH_HIP(hipMemsetAsync(h->maxBits.p, 0, h->maxBits.bytes(), h->stream));  // [6]: BE reduction ticket
+    h->partials.alloc(4096);
+    NRH_HIP(hipStreamSynchronize(h->stream));
+    return h.release();
+}
+
+nrh_f3d *f3d_create(const nrh_geom& ref, DevBuf<float>&& refImg, const nrh_geom& flo, DevBuf<float>&& floImg,
+                    const int *mask, const nrh_geom& cpp, const nrh_f3d_params& params) {
+    check_geom(&ref, "reference");
+    check_geom(&flo, "floating");
+    check_geom(&cpp, "control point grid");
+    check_params(&params);
+    NRH_REQUIRE(refImg.n == voxels(ref) && floImg.n == voxels(flo), NRH_ERR_ARG, "image sizes differ from the geometries");
+    std::unique_ptr<nrh_f3d> h = f3d_begin(ref, flo, cpp, params);
+    h->refImg = std::move(refImg);
+    h->floImg = std::move(floImg);
+    return f3d_finish(std::move(h), mask);
+}
+
 }  // namespace nrh
 
 using namespace nrh;
@@ -176,45 +232,14 @@ int nrh_f3d_create(const nrh_geom *ref, const float *ref_data, const nrh_geom *f
         check_geom(cpp, "control point grid");
         check_params(params);
         NRH_REQUIRE(ref_data && flo_data && out, NRH_ERR_ARG, "null image data or output");
-        NRH_REQUIRE(ref->nz > 1, NRH_ERR_UNSUPPORTED, "2-D images are not supported");
-        std::unique_ptr<nrh_f3d> h(new nrh_f3d);
-        h->ref = *ref; h->flo = *flo; h->cpp = *cpp; h->params = *params;
-        h->N = voxels(*ref); h->Nf = voxels(*flo); h->G = voxels(*cpp);
-        NRH_HIP(hipGetDevice(&h->device));
-        NRH_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-        NRH_HIP(hipHostMalloc((void **)&h->pinned, 16 * sizeof(double), hipHostMallocDefault));
-        NRH_HIP(hipHostMalloc((void **)&h->published, 16 * sizeof(double), hipHostMallocCoherent | hipHostMallocMapped));
-        NRH_HIP(hipHostGetDevicePointer((void **)&h->publishedDev, h->published, 0));
-        std::memset(h->published, 0, 16 * sizeof(double));  // published[15]: no sequence number yet
+        std::unique_ptr<nrh_f3d> h = f3d_begin(*ref, *flo, *cpp, *params);
         // Images: float32 always kept (per-operation path); float16 copies added for the fused
         // path when requested.
         h->refImg.alloc(h->N);
         h->floImg.alloc(h->Nf);
         NRH_HIP(hipMemcpyAsync(h->refImg.p, ref_data, h->N * sizeof(float), hipMemcpyHostToDevice, h->stream));
         NRH_HIP(hipMemcpyAsync(h->floImg.p, flo_data, h->Nf * sizeof(float), hipMemcpyHostToDevice, h->stream));
-        if (mask) {
-            bool any = false;
-            for (size_t i = 0; i < h->N && !any; ++i) any = mask[i] < 0;
-            if (any) {
-                h->mask.alloc(h->N);
-                NRH_HIP(hipMemcpyAsync(h->mask.p, mask, h->N * sizeof(int), hipMemcpyHostToDevice, h->stream));
-            }
-        }
-        h->cppPos.alloc(3 * h->G);
-        h->best.alloc(3 * h->G);
-        h->nodeGrad.alloc(3 * h->G);
-        h->cgG.alloc(3 * h->G);
-        h->cgH.alloc(3 * h->G);
-        NRH_HIP(hipMemsetAsync(h->cppPos.p, 0, h->cppPos.bytes(), h->stream));
-        NRH_HIP(hipMemsetAsync(h->nodeGrad.p, 0, h->nodeGrad.bytes(), h->stream));
-        alloc_histogram(h.get());
-        h->ent.alloc(8);
-        h->scalars.alloc(16);
-        h->maxBits.alloc(8);
-        NRH_HIP(hipMemsetAsync(h->maxBits.p, 0, h->maxBits.bytes(), h->stream));  // [6]: BE reduction ticket
-        h->partials.alloc(4096);
-        NRH_HIP(hipStreamSynchronize(h->stream));
-        *out = h.release();
+        *out = f3d_finish(std::move(h), mask);
     });
 }
 

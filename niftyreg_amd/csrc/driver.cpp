@@ -1,4 +1,4 @@
-// Host side of a full F3D registration: image pyramid, control-point grid creation and
+// Host side of a full F3D registration: image levels, control-point grid creation and
 // refinement, and the conjugate-gradient / line-search loop of reg_base<T>::Run
 // (reg-lib/_reg_base.cpp:727-819, reg-lib/Optimiser.cpp:129-317, reg-lib/_reg_f3d.cpp:92-159).
 // Every objective and gradient evaluation runs on the device through the F3D handle.
@@ -83,13 +83,8 @@ void gaussian_smooth(const nrh_geom& g, std::vector<float>& img, float sigmaVox)
 
 }  // namespace
 
-// reg_downsampleImage<float>(image, 1, axes) (reg-lib/cpu/_reg_tools.cpp:1343-1467): Gaussian
-// smoothing (sigma 0.7355 voxel) then nearest-neighbour decimation by 2 along the flagged axes.
-// The new voxel -> mm map doubles the flagged columns and keeps the origin.
-void downsample(const nrh_geom& g, const std::vector<float>& in, const bool axes[3], nrh_geom& out,
-                std::vector<float>& res) {
-    std::vector<float> img(in);
-    gaussian_smooth(g, img, -0.7355f);
+// The new voxel -> mm map of reg_downsampleImage doubles the flagged columns and keeps the origin.
+void downsampled_geometry(const nrh_geom& g, const bool axes[3], nrh_geom& out) {
     const int od[3] = { g.nx, g.ny, g.nz };
     int nd[3];
     float pd[3] = { g.dx, g.dy, g.dz };
@@ -105,6 +100,17 @@ void downsample(const nrh_geom& g, const std::vector<float>& in, const bool axes
         if (axes[c])
             for (int r = 0; r < 3; ++r) out.xyz[r * 4 + c] = g.xyz[r * 4 + c] * 2.f;
     mat44_inverse(out.xyz, out.ijk);
+}
+
+// reg_downsampleImage<float>(image, 1, axes) (reg-lib/cpu/_reg_tools.cpp:1343-1467) on the host:
+// Gaussian smoothing (sigma 0.7355 voxel) then nearest-neighbour decimation by 2 along the flagged
+// axes.  Registrations build their pyramids on the device with the same sums (pyramid.hip).
+void downsample(const nrh_geom& g, const std::vector<float>& in, const bool axes[3], nrh_geom& out,
+                std::vector<float>& res) {
+    std::vector<float> img(in);
+    gaussian_smooth(g, img, -0.7355f);
+    downsampled_geometry(g, axes, out);
+    const int od[3] = { g.nx, g.ny, g.nz }, nd[3] = { out.nx, out.ny, out.nz };
     const float *m = out.xyz, *r2v = g.ijk;
     auto round_int = [](float x) { return (int)(x + (x >= 0 ? 0.5f : -0.5f)); };
     res.assign(voxels(out), 0.f);
@@ -210,32 +216,6 @@ static void subdivide(const nrh_geom& old, const std::vector<float>& oldData, co
     }
 }
 
-// reg_createImagePyramid<float> (reg-lib/cpu/_reg_tools.cpp:1705-1733): the finest level is the
-// input; each coarser level halves the axes whose half-size is still >= 32 voxels.
-std::vector<Level> pyramid(const nrh_geom& g, const float *data, int levels, int toPerform) {
-    std::vector<Level> p(toPerform);
-    Level cur{ g, std::vector<float>(data, data + voxels(g)) };
-    auto axes_of = [](const nrh_geom& q, bool ax[3]) {
-        ax[0] = q.nx / 2 >= 32;
-        ax[1] = q.ny / 2 >= 32;
-        ax[2] = q.nz / 2 >= 32;
-    };
-    for (int l = toPerform; l < levels; ++l) {
-        bool ax[3];
-        axes_of(cur.geom, ax);
-        Level nxt;
-        downsample(cur.geom, cur.data, ax, nxt.geom, nxt.data);
-        cur = std::move(nxt);
-    }
-    p[toPerform - 1] = cur;
-    for (int l = toPerform - 2; l >= 0; --l) {
-        bool ax[3];
-        axes_of(p[l + 1].geom, ax);
-        downsample(p[l + 1].geom, p[l + 1].data, ax, p[l].geom, p[l].data);
-    }
-    return p;
-}
-
 namespace {
 
 struct Handle {
@@ -249,13 +229,15 @@ void check(int rc) {
 
 }  // namespace
 
-// The host side of one reg_f3d registration that does not depend on the device: weights,
-// pyramids, the control-point grid of every level, and the iteration budget.
+// One reg_f3d registration outside its levels' handles: weights, pyramids (on the device), the
+// control-point grid of every level, and the iteration budget.
 struct PairRun {
     nrh_f3d_config cfg;
     int levels = 1, toPerform = 1;
     float be = 0, le = 0, simW = 0;
-    std::vector<Level> rp, fp;
+    nrh_geom refG{}, floG{};
+    const float *refData = nullptr, *floData = nullptr;  // the caller's full-resolution images
+    std::vector<DevLevel> rp, fp;  // with use_pyramid; a level's handle takes its images over
     nrh_geom grid;
     std::vector<float> cpp;
     size_t maxIter = 0;
@@ -284,13 +266,15 @@ void pair_begin(PairRun& r, const nrh_geom& refG, const float *refData, const nr
     }
     r.be = be;
     r.le = le;
-    // pyramids (or the full-resolution images at every level with -nopy)
+    // pyramids (or the full-resolution images, uploaded anew for each level, with -nopy)
+    r.refG = refG;
+    r.floG = floG;
+    r.refData = refData;
+    r.floData = floData;
     if (cfg.use_pyramid) {
-        r.rp = pyramid(refG, refData, levels, toPerform);
-        r.fp = pyramid(floG, floData, levels, toPerform);
-    } else {
-        r.rp.assign(1, Level{ refG, std::vector<float>(refData, refData + voxels(refG)) });
-        r.fp.assign(1, Level{ floG, std::vector<float>(floData, floData + voxels(floG)) });
+        ScopedStream st;
+        r.rp = device_pyramid(refG, refData, levels, toPerform, st.s);
+        r.fp = device_pyramid(floG, floData, levels, toPerform, st.s);
     }
     // control-point grid at the coarsest level (reg-lib/_reg_f3d.cpp:161-195)
     float spmm = cfg.spacing < 0 ? -cfg.spacing * refG.dx : cfg.spacing;
@@ -298,7 +282,7 @@ void pair_begin(PairRun& r, const nrh_geom& refG, const float *refData, const nr
     float spz = cfg.spacing < 0 ? -cfg.spacing * refG.dz : cfg.spacing;
     const float scale = std::pow(2.f, (float)(levels - 1));
     const float gsp[3] = { spmm * scale, spy * scale, spz * scale };
-    const nrh_geom& g0 = r.rp[0].geom;
+    const nrh_geom& g0 = cfg.use_pyramid ? r.rp[0].geom : r.refG;
     create_grid(g0, gsp, r.grid, nullptr);
     r.cpp.resize(3 * voxels(r.grid));
     create_grid(g0, gsp, r.grid, r.cpp.data());
@@ -328,8 +312,7 @@ void pair_begin(PairRun& r, const nrh_geom& refG, const float *refData, const nr
 // reg_f3d::InitCurrentLevel (reg-lib/_reg_f3d.cpp:92-133): the level's penalty weights and grid
 // (refined after the first level), and the handle parameters and largest step of the level.
 void pair_level(PairRun& r, int level, nrh_f3d_params& p, float& maxStep) {
-    const int idx = r.cfg.use_pyramid ? level : 0;
-    const nrh_geom& lr = r.rp[idx].geom;
+    const nrh_geom& lr = r.cfg.use_pyramid ? r.rp[level].geom : r.refG;
     maxStep = std::max(lr.dx, lr.dy);
     maxStep = std::max(maxStep, lr.dz);
     if (level == 0) {
@@ -361,10 +344,13 @@ void pair_level(PairRun& r, int level, nrh_f3d_params& p, float& maxStep) {
 // (reg_nmi::InitialiseMeasure to [2, bins - 3], reg-lib/cpu/_reg_nmi.cpp:115-129; reg_lncc to [0, 1],
 // reg-lib/cpu/_reg_lncc.cpp:99-104).
 nrh_f3d *pair_handle(PairRun& r, int level, const nrh_f3d_params& p) {
-    const int idx = r.cfg.use_pyramid ? level : 0;
     nrh_f3d *h = nullptr;
-    check(nrh_f3d_create(&r.rp[idx].geom, r.rp[idx].data.data(), &r.fp[idx].geom, r.fp[idx].data.data(), nullptr,
-                         &r.grid, &p, &h));
+    if (r.cfg.use_pyramid) {
+        DevLevel &lr = r.rp[level], &lf = r.fp[level];
+        h = f3d_create(lr.geom, std::move(lr.img), lf.geom, std::move(lf.img), nullptr, r.grid, p);
+    } else {
+        check(nrh_f3d_create(&r.refG, r.refData, &r.floG, r.floData, nullptr, &r.grid, &p, &h));
+    }
     Handle H;
     H.h = h;
     check(nrh_f3d_set_control_points(h, r.cpp.data()));
@@ -458,28 +444,35 @@ void register_pair(const nrh_geom& refG, const float *refData, const nrh_geom& f
 // Many reg_f3d registrations at once: every pair runs register_pair's levels and decisions, but
 // all pairs' evaluations share the batch launches of f3d_batch.hip, and each level's iterations
 // replay one captured HIP graph (gradient, conjugate gradient, twelve lockstep line-search steps,
-// restore and stopping rule) until every pair has stopped.  The pyramids are built on host threads.
+// restore and stopping rule) until every pair has stopped.  The pyramids are built from host threads, several uploads at a time.
 void register_batch(int n, const nrh_geom *refs, const float *const *refData, const nrh_geom *flos,
                     const float *const *floData, const nrh_f3d_config& cfg, std::vector<PairRun>& runs,
                     nrh_batch_stats *stats) {
     const auto t0 = std::chrono::steady_clock::now();
-    runs.assign(n, PairRun{});
+    runs = std::vector<PairRun>(n);
     {
         std::vector<std::thread> pool;
         std::vector<std::string> errs(n);
+        std::vector<int> codes(n, NRH_ERR_ARG);
+        int device = 0;
+        NRH_HIP(hipGetDevice(&device));
         const int T = std::max(1, std::min(n, (int)std::thread::hardware_concurrency()));
         for (int t = 0; t < T; ++t)
             pool.emplace_back([&, t] {
                 for (int q = t; q < n; q += T) {
                     try {
+                        NRH_HIP(hipSetDevice(device));
                         pair_begin(runs[q], refs[q], refData[q], flos[q], floData[q], cfg);
+                    } catch (const Error& e) {
+                        errs[q] = e.what();
+                        codes[q] = e.code;
                     } catch (const std::exception& e) {
                         errs[q] = e.what();
                     }
                 }
             });
         for (auto& th : pool) th.join();
-        for (int q = 0; q < n; ++q) NRH_REQUIRE(errs[q].empty(), NRH_ERR_ARG, "pair " + std::to_string(q) + ": " + errs[q]);
+        for (int q = 0; q < n; ++q) NRH_REQUIRE(errs[q].empty(), codes[q], "pair " + std::to_string(q) + ": " + errs[q]);
     }
     const int toPerform = runs[0].toPerform;
     double deviceSeconds = 0.0;
@@ -587,13 +580,11 @@ void register_pair_sym(const nrh_geom& refG, const float *refData, const nrh_geo
     } else {
         simW = 1 - penalty;
     }
-    std::vector<Level> rp, fp;
+    std::vector<DevLevel> rp, fp;
     if (cfg.use_pyramid) {
-        rp = pyramid(refG, refData, levels, toPerform);
-        fp = pyramid(floG, floData, levels, toPerform);
-    } else {
-        rp.assign(1, Level{ refG, std::vector<float>(refData, refData + voxels(refG)) });
-        fp.assign(1, Level{ floG, std::vector<float>(floData, floData + voxels(floG)) });
+        ScopedStream st;
+        rp = device_pyramid(refG, refData, levels, toPerform, st.s);
+        fp = device_pyramid(floG, floData, levels, toPerform, st.s);
     }
     // reg_f3d2::Initialise (reg-lib/_reg_f3d2.cpp:536-590): spacing in voxels of the mean voxel size
     const float pd[3][2] = { { refG.dx, floG.dx }, { refG.dy, floG.dy }, { refG.dz, floG.dz } };
@@ -616,18 +607,18 @@ void register_pair_sym(const nrh_geom& refG, const float *refData, const nrh_geo
     }
     nrh_geom grid;
     std::vector<float> fw, bw;
-    symmetric_grids(rp[0].geom, fp[0].geom, gsp, grid, nullptr, nullptr, halfF, halfB);
+    const nrh_geom &r0 = cfg.use_pyramid ? rp[0].geom : refG, &f0 = cfg.use_pyramid ? fp[0].geom : floG;
+    symmetric_grids(r0, f0, gsp, grid, nullptr, nullptr, halfF, halfB);
     fw.resize(3 * voxels(grid));
     bw.resize(3 * voxels(grid));
-    symmetric_grids(rp[0].geom, fp[0].geom, gsp, grid, fw.data(), bw.data(), halfF, halfB);
+    symmetric_grids(r0, f0, gsp, grid, fw.data(), bw.data(), halfF, halfB);
     int steps = 6;  // intent_p2 of both grids
     size_t maxIter = (size_t)cfg.max_iterations * (size_t)std::pow(2.0, toPerform - 1);
     totalIterations = 0;
     finalNmi = 0;
     for (int level = 0; level < toPerform; ++level) {
-        const int idx = cfg.use_pyramid ? level : 0;
-        const nrh_geom& lr = rp[idx].geom;
-        const nrh_geom& lf = fp[idx].geom;
+        const nrh_geom& lr = cfg.use_pyramid ? rp[level].geom : refG;
+        const nrh_geom& lf = cfg.use_pyramid ? fp[level].geom : floG;
         // reg_f3d2::InitCurrentLevel (reg-lib/_reg_f3d2.cpp:55-100): the largest voxel size of both
         float maxStep = std::max(lr.dx, lr.dy);
         maxStep = std::max(maxStep, lf.dx);
@@ -660,8 +651,21 @@ void register_pair_sym(const nrh_geom& refG, const float *refData, const nrh_geo
         p.lncc_sigma = cfg.lncc_sigma;
         p.field_order = cfg.field_order;
         Handle F, B;
-        check(nrh_f3d_create(&lr, rp[idx].data.data(), &lf, fp[idx].data.data(), nullptr, &grid, &p, &F.h));
-        check(nrh_f3d_create(&lf, fp[idx].data.data(), &lr, rp[idx].data.data(), nullptr, &grid, &p, &B.h));
+        if (cfg.use_pyramid) {
+            // the backward handle rescales its own copies of the images
+            DevBuf<float> ri, fi;
+            ri.alloc(voxels(lr));
+            fi.alloc(voxels(lf));
+            ScopedStream st;
+            NRH_HIP(hipMemcpyAsync(ri.p, rp[level].img.p, ri.bytes(), hipMemcpyDeviceToDevice, st.s));
+            NRH_HIP(hipMemcpyAsync(fi.p, fp[level].img.p, fi.bytes(), hipMemcpyDeviceToDevice, st.s));
+            NRH_HIP(hipStreamSynchronize(st.s));
+            F.h = f3d_create(lr, std::move(rp[level].img), lf, std::move(fp[level].img), nullptr, grid, p);
+            B.h = f3d_create(lf, std::move(fi), lr, std::move(ri), nullptr, grid, p);
+        } else {
+            check(nrh_f3d_create(&lr, refData, &lf, floData, nullptr, &grid, &p, &F.h));
+            check(nrh_f3d_create(&lf, floData, &lr, refData, nullptr, &grid, &p, &B.h));
+        }
         nrh_f3d *hf = F.h, *hb = B.h;
         check(nrh_f3d_set_control_points(hf, fw.data()));
         check(nrh_f3d_set_control_points(hb, bw.data()));

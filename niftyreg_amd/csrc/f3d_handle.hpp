@@ -98,6 +98,11 @@ struct nrh_f3d {
 
 namespace nrh {
 
+// A handle over images that are on the device already (the handle takes them over); otherwise as
+// nrh_f3d_create.
+nrh_f3d *f3d_create(const nrh_geom& ref, DevBuf<float>&& refImg, const nrh_geom& flo, DevBuf<float>&& floImg,
+                    const int *mask, const nrh_geom& cpp, const nrh_f3d_params& params);
+
 void ensure_field(nrh_f3d *h);
 void ensure_warped(nrh_f3d *h);
 void ensure_warped_grad(nrh_f3d *h);
