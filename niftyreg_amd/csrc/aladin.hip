@@ -835,47 +835,164 @@ __global__ void k_zero_int(int *p) {
 // reference evaluates logm / expm with Eigen in double; here they are computed in double by
 // inverse scaling and squaring (Denman-Beavers square roots, then the [8/8] Pade approximant of
 // log(I + X) in Gauss-Legendre form) and by Taylor scaling and squaring, with the reference's
-// float roundings between the steps.  One thread: 4x4 matrices, once per iteration.
-// Mat44Avg2: the logarithms rounded to float with zero bottom rows, summed in double and
-// rounded to float, halved, exponentiated in double, rounded to float.
-__device__ bool mat44_avg2(const float *A, const float *B, const GaussLegendre8& gl, float *out) {
-    double a[16], b[16], la[16], lb[16], h[16], e[16];
-    for (int i = 0; i < 16; ++i) {
-        a[i] = A[i];
-        b[i] = B[i];
+// float roundings between the steps.
+//
+// One wave: 16 lanes hold one 4x4 matrix, an element each, so the four logarithms of an update run
+// beside one another, and every product and elimination step is one instruction per lane where a
+// single thread makes 16 to 32 and keeps the pivoted rows in scratch memory.  The arithmetic of each
+// element and the order of every sum are those of m44.hpp's functions (d4_inverse, d4_logm, d4_expm),
+// which the host and the oracle use, so the results are equal.  Latency-bound, a chain of FP64
+// divisions and lane exchanges: 75 us an update, 395 with one thread (181 x 217 x 181 pair).
+struct WaveMat {
+    int i, j, base;  // row, column, first lane of the group
+    __device__ WaveMat(): i((threadIdx.x >> 2) & 3), j(threadIdx.x & 3), base(threadIdx.x & 48) {}
+    __device__ double get(double v, int r, int c) const { return __shfl(v, base + 4 * r + c, 64); }
+    __device__ double eye() const { return i == j ? 1.0 : 0.0; }
+    __device__ double mul(double a, double b) const {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc = fma(get(a, i, k), get(b, k, j), acc);
+        return acc;
     }
-    if (!d4_logm(a, gl, la) || !d4_logm(b, gl, lb)) return false;
-    for (int i = 0; i < 16; ++i) {
-        float fa = (float)la[i], fb = (float)lb[i];
-        if (i >= 12) fa = fb = 0.f;
-        const float sum = (float)((double)fa + (double)fb);
-        h[i] = (double)(sum * 0.5f);
+    // the largest column sum of absolute values, the same in every lane of the group
+    __device__ double norm1(double a) const {
+        const double m = fabs(a);
+        const double c = get(m, 0, j) + get(m, 1, j) + get(m, 2, j) + get(m, 3, j);
+        double best = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double v = get(c, 0, q);
+            best = v > best ? v : best;
+        }
+        return best;
     }
-    d4_expm(h, e);
-    for (int i = 0; i < 16; ++i) out[i] = (float)e[i];
-    return true;
+    // the sum over the 16 elements, row by row
+    __device__ double sum(double a) const {
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s += __shfl(a, base + q, 64);
+        return s;
+    }
+    // Gauss-Jordan with partial pivoting; *singular is set for the group on a zero pivot
+    __device__ double inverse(double a, bool *singular) const {
+        double m0 = a, m1 = eye();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            double v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = get(m0, r, c);
+            int p = c;
+            double vp = v[c];
+#pragma unroll
+            for (int r = c + 1; r < 4; ++r)
+                if (fabs(v[r]) > fabs(vp)) {
+                    p = r;
+                    vp = v[r];
+                }
+            if (vp == 0.0) *singular = true;
+            // row c of the exchanged matrix is the pivot row, scaled; the lane's own row and its
+            // factor follow the exchange
+            const double inv = 1.0 / vp;
+            const double p0 = get(m0, p, j) * inv, p1 = get(m1, p, j) * inv;
+            const int src = i == p ? c : i;
+            const double o0 = get(m0, src, j), o1 = get(m1, src, j);
+            const double f = src == 0 ? v[0] : src == 1 ? v[1] : src == 2 ? v[2] : v[3];
+            m0 = i == c ? p0 : fma(-f, p0, o0);
+            m1 = i == c ? p1 : fma(-f, p1, o1);
+        }
+        return m1;
+    }
+};
+
+// Every lane of the wave calls these; loops end when no group of 16 lanes needs another turn.
+// *failed is set for the group where d4_logm returns false.
+__device__ double wave_logm(const WaveMat& w, double a, const GaussLegendre8& gl, bool *failed) {
+    double y = a, x = 0.0;
+    int k = 0;
+    bool settled = false;  // the group's matrix is near enough to the identity, or has failed
+    for (;;) {
+        if (!settled) x = y - w.eye();
+        if (w.norm1(x) <= 0.25) settled = true;
+        if (!settled && k >= 60) *failed = settled = true;
+        if (__all(settled)) break;
+        double z = w.eye();
+        bool done = settled;
+        for (int it = 0; it < 100; ++it) {
+            bool singular = false;
+            const double yi = w.inverse(y, &singular), zi = w.inverse(z, &singular);
+            if (singular && !done) *failed = settled = done = true;
+            const double yn = 0.5 * (y + zi);
+            const double diff = w.sum(fabs(yn - y)), zn = 0.5 * (z + yi);
+            const double norm = w.norm1(done ? y : yn);
+            if (!done) {
+                z = zn;
+                y = yn;
+                if (diff <= 1e-15 * norm) done = true;
+            }
+            if (__all(done)) break;
+        }
+        if (!settled) ++k;
+    }
+    double s = 0.0;
+    for (int q = 0; q < 8; ++q) {
+        bool singular = false;
+        const double ti = w.inverse(fma(gl.x[q], x, w.eye()), &singular);
+        if (singular) *failed = true;
+        s = fma(gl.w[q], w.mul(x, ti), s);
+    }
+    return ldexp(1.0, k) * s;
+}
+
+__device__ double wave_expm(const WaveMat& w, double a) {
+    const double n = w.norm1(a);
+    int s = 0;
+    if (n > 0.5) s = (int)ceil(log2(n / 0.5));
+    const double b = a * ldexp(1.0, -s);
+    double term = w.eye(), sum = term;
+    for (int k = 1; k <= 20; ++k) {
+        term = w.mul(term, b);
+        term /= k;
+        sum += term;
+    }
+    for (int q = 0; !__all(q >= s); ++q) {
+        const double sq = w.mul(sum, sum);
+        if (q < s) sum = sq;
+    }
+    return sum;
 }
 
 __global__ void __launch_bounds__(64)
 k_symmetric_update(float *__restrict__ fw, float *__restrict__ bw, GaussLegendre8 gl, int *__restrict__ status) {
-    if (threadIdx.x != 0) return;
-    float F[16], B[16], fi[16], bi[16], nf[16], nb[16];
-    for (int i = 0; i < 16; ++i) {
-        F[i] = fw[i];
-        B[i] = bw[i];
+    // the groups' matrices: forward, inverse of backward, inverse of forward, backward; each pair
+    // is averaged (Mat44Avg2: the logarithms rounded to float with zero bottom rows, summed in
+    // double and rounded to float, halved, exponentiated in double, rounded to float)
+    __shared__ float M[4][16];
+    if (threadIdx.x < 2) {
+        float a[16], inv[16];
+        const float *src = threadIdx.x == 0 ? fw : bw;
+        for (int q = 0; q < 16; ++q) a[q] = src[q];
+        nifti_inverse(a, inv);
+        for (int q = 0; q < 16; ++q) {
+            M[threadIdx.x == 0 ? 0 : 3][q] = a[q];
+            M[threadIdx.x == 0 ? 2 : 1][q] = inv[q];
+        }
     }
-    nifti_inverse(F, fi);
-    nifti_inverse(B, bi);
-    if (!mat44_avg2(F, bi, gl, nf) || !mat44_avg2(fi, B, gl, nb)) {
-        *status = 3;  // matrices left unchanged
+    __syncthreads();
+    const int group = threadIdx.x >> 4, e = threadIdx.x & 15;
+    const WaveMat w;
+    bool failed = false;
+    const double l = wave_logm(w, (double)M[group][e], gl, &failed);
+    if (__any(failed)) {
+        if (threadIdx.x == 0) *status = 3;  // matrices left unchanged
         return;
     }
-    for (int i = 12; i < 15; ++i) nf[i] = nb[i] = 0.f;
-    nf[15] = nb[15] = 1.f;
-    for (int i = 0; i < 16; ++i) {
-        fw[i] = nf[i];
-        bw[i] = nb[i];
-    }
+    const float own = e >= 12 ? 0.f : (float)l;
+    const float other = __shfl_xor(own, 16, 64);
+    const float sum = (float)((double)own + (double)other);
+    float r = (float)wave_expm(w, (double)(sum * 0.5f));
+    if (e >= 12) r = e == 15 ? 1.f : 0.f;
+    if (group == 0) fw[e] = r;
+    if (group == 2) bw[e] = r;
 }
 
 // ------------------------------------------------------------------ host side

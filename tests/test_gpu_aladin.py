@@ -10,6 +10,7 @@ import pytest
 
 import oracles as O
 from niftyreg_amd import aladin, phantoms
+from niftyreg_amd._lib import NiftyRegError
 from niftyreg_amd.aladin import AladinContent
 from niftyreg_amd.geometry import Geom
 
@@ -237,6 +238,41 @@ def test_symmetric_update_matches_reference(gpu):
             wf, wb = O.orc_symmetric_update(F, B)
         _ulp_or_abs_close(fw.get_matrix(), wf)
         _ulp_or_abs_close(bw.get_matrix(), wb)
+    fw.close()
+    bw.close()
+
+
+def _rot_z(deg, t=(0, 0, 0)):
+    c, s = np.cos(np.deg2rad(deg)), np.sin(np.deg2rad(deg))
+    return np.array([[c, -s, 0, t[0]], [s, c, 0, t[1]], [0, 0, 1, t[2]], [0, 0, 0, 1]], np.float32)
+
+
+# no square root at all, different numbers of them in the four logarithms, a zero on the diagonal
+# (a pivot in another row), a large translation
+@pytest.mark.parametrize("F,B", [
+    (np.eye(4, dtype=np.float32), np.eye(4, dtype=np.float32)),
+    (np.eye(4, dtype=np.float32), _rot_z(0, (80, -60, 40))),
+    (_rot_z(90, (3, 0, 0)), _rot_z(-89)),
+    (_rot_z(20, (150, 90, -70)), _rot_z(-21, (-160, -40, 75))),
+    (np.diag([0.02, 40, 1, 1]).astype(np.float32), np.diag([45, 0.03, 1.1, 1]).astype(np.float32)),
+])
+def test_symmetric_update_edges(gpu, F, B):
+    g = Geom.identity((32, 32, 32))
+    ref = phantoms.blob_phantom(g.dims, 1).ravel()
+    fw, bw = AladinContent(g, ref, g, ref), AladinContent(g, ref, g, ref)
+    fw.set_matrix(F)
+    bw.set_matrix(B)
+    aladin.symmetric_update(fw, bw)
+    wf, wb = O.orc_symmetric_update(F, B)
+    _ulp_or_abs_close(fw.get_matrix(), wf)
+    _ulp_or_abs_close(bw.get_matrix(), wb)
+    # a matrix without a real logarithm: an error, and both matrices unchanged
+    bad = np.diag([-1, 1, 1, 1]).astype(np.float32)
+    fw.set_matrix(bad)
+    bw.set_matrix(B)
+    with pytest.raises(NiftyRegError):
+        aladin.symmetric_update(fw, bw)
+    assert np.array_equal(fw.get_matrix(), bad) and np.array_equal(bw.get_matrix(), B)
     fw.close()
     bw.close()
 
