@@ -267,6 +267,7 @@ int nrh_f3d_set_params(nrh_f3d *h, const nrh_f3d_params *params) {
     return guard([&] {
         NRH_REQUIRE(h, NRH_ERR_ARG, "null handle");
         check_params(params);
+        if (params->field_order != h->params.field_order) settle_voxel_gradient(h);  // in the order it was asked in
         const bool bins = params->ref_bins != h->params.ref_bins || params->flo_bins != h->params.flo_bins;
         h->params = *params;
         if (bins) { alloc_histogram(h); h->histVersion = 0; }
@@ -323,10 +324,13 @@ NRH_HANDLE_OP(nrh_f3d_deformation_field(nrh_f3d *h), op_spline_field(h))
 NRH_HANDLE_OP(nrh_f3d_resample(nrh_f3d *h), op_resample(h))
 NRH_HANDLE_OP(nrh_f3d_image_gradient(nrh_f3d *h), op_image_gradient(h))
 NRH_HANDLE_OP(nrh_f3d_zero_voxel_gradient(nrh_f3d *h),
-              ensure_voxel_grad(h); NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream)))
-NRH_HANDLE_OP(nrh_f3d_nmi_voxel_gradient(nrh_f3d *h, double weight), op_nmi_voxel_gradient(h, weight))
-NRH_HANDLE_OP(nrh_f3d_convolve_voxel_gradient(nrh_f3d *h), op_convolve_voxel_gradient(h))
-NRH_HANDLE_OP(nrh_f3d_voxel_to_node(nrh_f3d *h, float weight), op_voxel_to_node(h, weight))
+              zero_voxel_gradient(h))
+NRH_HANDLE_OP(nrh_f3d_nmi_voxel_gradient(nrh_f3d *h, double weight), settle_voxel_gradient(h);
+              op_nmi_voxel_gradient(h, weight))
+NRH_HANDLE_OP(nrh_f3d_convolve_voxel_gradient(nrh_f3d *h), settle_voxel_gradient(h);
+              op_convolve_voxel_gradient(h))
+NRH_HANDLE_OP(nrh_f3d_voxel_to_node(nrh_f3d *h, float weight), settle_voxel_gradient(h);
+              op_voxel_to_node(h, weight))
 NRH_HANDLE_OP(nrh_f3d_zero_node_gradient(nrh_f3d *h),
               NRH_HIP(hipMemsetAsync(h->nodeGrad.p, 0, h->nodeGrad.bytes(), h->stream)))
 NRH_HANDLE_OP(nrh_f3d_bending_energy_gradient(nrh_f3d *h, float weight), op_bending_energy_gradient(h, weight))
@@ -395,7 +399,7 @@ int nrh_f3d_download_warped_gradient(nrh_f3d *h, float *p) {
     return guard([&] { NRH_REQUIRE(h, NRH_ERR_ARG, "null handle"); download(h, h->warpedGrad.p, p, 3 * h->N * sizeof(float), "warped gradient"); });
 }
 int nrh_f3d_download_voxel_gradient(nrh_f3d *h, float *p) {
-    return guard([&] { NRH_REQUIRE(h, NRH_ERR_ARG, "null handle"); download(h, h->voxelGrad.p, p, 3 * h->N * sizeof(float), "voxel-based gradient"); });
+    return guard([&] { NRH_REQUIRE(h, NRH_ERR_ARG, "null handle"); settle_voxel_gradient(h); download(h, h->voxelGrad.p, p, 3 * h->N * sizeof(float), "voxel-based gradient"); });
 }
 int nrh_f3d_download_node_gradient(nrh_f3d *h, float *p) {
     return guard([&] { NRH_REQUIRE(h, NRH_ERR_ARG, "null handle"); download(h, h->nodeGrad.p, p, 3 * h->G * sizeof(float), "node gradient"); });

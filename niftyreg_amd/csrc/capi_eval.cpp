@@ -111,14 +111,12 @@ int nrh_f3d_similarity_gradient(nrh_f3d *h, float weight) {
             op_spline_field(h);
             op_resample(h);
             op_image_gradient(h);
-            ensure_voxel_grad(h);
-            NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream));
+            zero_voxel_gradient(h);
             op_lncc_voxel_gradient(h, 1.0);
             if (fused_projection_supported(h)) {
                 fused_project(h, h->voxelGrad.p, weight);
             } else {
-                op_convolve_voxel_gradient(h);
-                op_voxel_to_node(h, weight);
+                op_voxel_gradient_to_nodes(h, weight);
             }
         } else if (fused_supported(h)) {
             if (h->histVersion != h->cppVersion) fused_histogram(h);
@@ -126,11 +124,9 @@ int nrh_f3d_similarity_gradient(nrh_f3d *h, float weight) {
         } else {
             histogram_at_current_points(h);
             op_image_gradient(h);
-            ensure_voxel_grad(h);
-            NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream));
+            zero_voxel_gradient(h);
             op_nmi_voxel_gradient(h, 1.0);
-            op_convolve_voxel_gradient(h);
-            op_voxel_to_node(h, weight);
+            op_voxel_gradient_to_nodes(h, weight);
         }
     });
 }
@@ -147,16 +143,14 @@ static void gradient_body(nrh_f3d *h, double *max_length) {
             op_spline_field(h);
             op_resample(h);
             op_image_gradient(h);
-            ensure_voxel_grad(h);
-            NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream));
+            zero_voxel_gradient(h);
             op_lncc_voxel_gradient(h, 1.0);
             // convolution + node extraction: the separable projection when the nodes lie on
             // voxels at an integer spacing, else the reference-order convolution
             if (fused_projection_supported(h)) {
                 fused_project(h, h->voxelGrad.p, p.similarity_weight);
             } else {
-                op_convolve_voxel_gradient(h);
-                op_voxel_to_node(h, p.similarity_weight);
+                op_voxel_gradient_to_nodes(h, p.similarity_weight);
             }
         } else if (p.similarity_weight > 0) {
             if (fused_supported(h)) {
@@ -175,11 +169,9 @@ static void gradient_body(nrh_f3d *h, double *max_length) {
                 op_nmi_finalize(h);
                 h->histVersion = h->cppVersion;
                 op_image_gradient(h);
-                ensure_voxel_grad(h);
-                NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream));
+                zero_voxel_gradient(h);
                 op_nmi_voxel_gradient(h, 1.0);
-                op_convolve_voxel_gradient(h);
-                op_voxel_to_node(h, p.similarity_weight);
+                op_voxel_gradient_to_nodes(h, p.similarity_weight);
             }
         } else {
             op_fill_f32(h->nodeGrad.p, 3 * h->G, 0.f, h->stream);

@@ -115,6 +115,7 @@ int nrh_f3d2_gradient(nrh_f3d *fw, nrh_f3d *bw, double *max_length) {
             for (nrh_f3d *h : { fw, bw }) {
                 ensure_voxel_grad(h);
                 op_fill_f32(h->voxelGrad.p, 3 * h->N, 0.f, h->stream);
+                h->voxelGradPending = false;
                 op_image_gradient(h);
             }
             for (nrh_f3d *h : { fw, bw }) {
@@ -133,8 +134,7 @@ int nrh_f3d2_gradient(nrh_f3d *fw, nrh_f3d *bw, double *max_length) {
                 if (fused_projection_supported(h)) {
                     fused_project(h, h->voxelGrad.p, p.similarity_weight);
                 } else {
-                    op_convolve_voxel_gradient(h);
-                    op_voxel_to_node(h, p.similarity_weight);
+                    op_voxel_gradient_to_nodes(h, p.similarity_weight);
                 }
             }
         } else {

@@ -197,6 +197,7 @@ int nrh_f3d_def_field_from_velocity(nrh_f3d *h, int update_step_number) {
 int nrh_f3d_exponentiate_gradient(nrh_f3d *h, nrh_f3d *bw) {
     return guard([&] {
         NRH_REQUIRE(h && bw, NRH_ERR_ARG, "null handle");
+        settle_voxel_gradient(h);
         op_exponentiate_gradient(h, bw);
         NRH_HIP(hipStreamSynchronize(h->stream));
     });
@@ -241,6 +242,7 @@ int nrh_f3d_resample_gradient(nrh_f3d *h, int interpolation, float padding, floa
     return guard([&] {
         NRH_REQUIRE(h && out, NRH_ERR_ARG, "null argument");
         NRH_REQUIRE(interpolation == 1, NRH_ERR_UNSUPPORTED, "only linear interpolation is supported");
+        settle_voxel_gradient(h);
         h->velTmp.alloc(3 * h->N);
         op_resample_gradient(h, padding, h->velTmp.p);
         NRH_HIP(hipMemcpyAsync(out, h->velTmp.p, 3 * h->N * sizeof(float), hipMemcpyDeviceToHost, h->stream));
@@ -263,6 +265,7 @@ int nrh_f3d_upload_voxel_gradient(nrh_f3d *h, const float *planar) {
     return guard([&] {
         NRH_REQUIRE(h && planar, NRH_ERR_ARG, "null argument");
         ensure_voxel_grad(h);
+        h->voxelGradPending = false;
         NRH_HIP(hipMemcpyAsync(h->voxelGrad.p, planar, 3 * h->N * sizeof(float), hipMemcpyHostToDevice, h->stream));
         NRH_HIP(hipStreamSynchronize(h->stream));
     });

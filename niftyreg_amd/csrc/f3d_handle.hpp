@@ -4,6 +4,20 @@
 #include <hip/hip_fp16.h>
 #include "common.hpp"
 
+namespace nrh {
+// The node-only convolution's plan (f3d_nodeconv.hip): for each axis the positions that the nodes
+// read, each voxel's place among them, the kernel and the density at those positions; two scratch
+// arrays.  Made for one grid-to-image transform and summation order.
+struct NodeConv {
+    bool built = false, ok = false;
+    Affine T;
+    int order = 0;
+    int n[3], radius[3];
+    DevBuf<int> list[3], map[3];
+    DevBuf<float> kern[3], dens[3], a, b;
+};
+}  // namespace nrh
+
 struct nrh_f3d {
     nrh_geom ref{}, flo{}, cpp{};
     nrh_f3d_params params{};
@@ -29,6 +43,10 @@ struct nrh_f3d {
     nrh::DevBuf<float> field, warped, warpedGrad, voxelGrad;
     nrh::DevBuf<float> convTmp, convDens, convDensTmp, convKernel;
     nrh::DevBuf<uint8_t> convNan;
+    nrh::NodeConv nodeConv;
+    // the evaluation sampled the convolved voxel gradient at the nodes only: voxelGrad still holds
+    // the gradient before the convolution, which settle_voxel_gradient carries out for a reader
+    bool voxelGradPending = false;
     nrh::DevBuf<float> leDiag;      // per-node rotation-free displacement Jacobian diagonal [3][G]
     uint64_t leDiagVersion = 0;     // cppVersion leDiag was computed at (0: none)
 
@@ -120,6 +138,17 @@ void op_nmi_finalize(nrh_f3d *h, float *kTab = nullptr, const double *pubS1 = nu
 void op_nmi_voxel_gradient(nrh_f3d *h, double weight);
 void op_convolve_voxel_gradient(nrh_f3d *h);
 void op_voxel_to_node(nrh_f3d *h, float weight);
+// op_convolve_voxel_gradient + op_voxel_to_node, convolving only what the nodes read where that is
+// less (f3d_nodeconv.hip); voxelGrad is then left for settle_voxel_gradient
+void op_voxel_gradient_to_nodes(nrh_f3d *h, float weight);
+// the convolution of voxelGrad if the last evaluation left it out; before any other use of voxelGrad
+void settle_voxel_gradient(nrh_f3d *h);
+// voxelGrad all zero
+void zero_voxel_gradient(nrh_f3d *h);
+// the cubic B-spline kernel of the node spacing (returns the radius); the grid's voxel -> image
+// voxel transform and the reorientation of op_voxel_to_node
+int convolution_kernel(float spacing, float pixdim, std::vector<float>& kern);
+void node_transforms(const nrh_f3d *h, Affine& T, Affine& R);
 // stream: where the launch goes (null: the handle's stream)
 void op_bending_energy(nrh_f3d *h, double *out_device, hipStream_t stream = nullptr);
 // the bending-energy gradient's gathered sums alone into h->beGrad (no weight, no round trip),

@@ -1256,6 +1256,27 @@ void op_nmi_voxel_gradient(nrh_f3d *h, double weight) {
     NRH_HIP(hipGetLastError());
 }
 
+// Cubic B-spline kernel of reg_tools_kernelConvolution (reg-lib/cpu/_reg_tools.cpp:868-904)
+int convolution_kernel(float spacing, float pixdim, std::vector<float>& kern) {
+    const double temp = (double)(spacing / pixdim);
+    const int radius = (int)(temp * 2.0f);
+    kern.resize(2 * radius + 1);
+    for (int i = -radius; i <= radius; ++i) {
+        const double rel = std::fabs(i / temp);
+        float kv = 0.f;
+        if (rel < 1.0) kv = (float)(2.0 / 3.0 - rel * rel + 0.5 * rel * rel * rel);
+        else if (rel < 2.0) kv = (float)(-((rel - 2.0) * (rel - 2.0) * (rel - 2.0)) / 6.0);
+        kern[i + radius] = kv;
+    }
+    return radius;
+}
+
+void zero_voxel_gradient(nrh_f3d *h) {
+    ensure_voxel_grad(h);
+    NRH_HIP(hipMemsetAsync(h->voxelGrad.p, 0, h->voxelGrad.bytes(), h->stream));
+    h->voxelGradPending = false;
+}
+
 void op_convolve_voxel_gradient(nrh_f3d *h) {
     NRH_REQUIRE(!h->voxelGrad.empty(), NRH_ERR_STATE, "no voxel-based gradient to convolve");
     const size_t N = h->N;
@@ -1267,17 +1288,8 @@ void op_convolve_voxel_gradient(nrh_f3d *h) {
     const float pix[3] = { h->ref.dx, h->ref.dy, h->ref.dz };
     const float sp[3] = { h->cpp.dx, h->cpp.dy, h->cpp.dz };
     for (int axis = 0; axis < 3; ++axis) {
-        // Cubic B-spline kernel of reg_tools_kernelConvolution (reg-lib/cpu/_reg_tools.cpp:868-904)
-        const double temp = (double)(sp[axis] / pix[axis]);
-        const int radius = (int)(temp * 2.0f);
-        std::vector<float> kern(2 * radius + 1);
-        for (int i = -radius; i <= radius; ++i) {
-            const double rel = std::fabs(i / temp);
-            float kv = 0.f;
-            if (rel < 1.0) kv = (float)(2.0 / 3.0 - rel * rel + 0.5 * rel * rel * rel);
-            else if (rel < 2.0) kv = (float)(-((rel - 2.0) * (rel - 2.0) * (rel - 2.0)) / 6.0);
-            kern[i + radius] = kv;
-        }
+        std::vector<float> kern;
+        const int radius = convolution_kernel(sp[axis], pix[axis], kern);
         if (radius > 0) {
             h->convKernel.alloc(std::max<size_t>(kern.size(), 64));
             NRH_HIP(hipMemcpyAsync(h->convKernel.p, kern.data(), kern.size() * sizeof(float), hipMemcpyHostToDevice, h->stream));
@@ -1328,10 +1340,9 @@ float node_weight_ratio(const nrh_f3d *h, float weight) {
     return weight;
 }
 
-void op_voxel_to_node(nrh_f3d *h, float weight) {
-    NRH_REQUIRE(!h->voxelGrad.empty(), NRH_ERR_STATE, "no voxel-based gradient");
-    Affine T = mat_mul_affine(h->ref.ijk, h->cpp.xyz);
-    Affine R = to_affine(h->flo.ijk);
+void node_transforms(const nrh_f3d *h, Affine& T, Affine& R) {
+    T = mat_mul_affine(h->ref.ijk, h->cpp.xyz);
+    R = to_affine(h->flo.ijk);
     if (h->velocity && h->velExt0) {
         // the grid's extension 0 maps the grid into the reference space (reg-lib/cpu/
         // _reg_localTrans.cpp:1568-1592): inverse(A) between the grid and the image, and
@@ -1350,6 +1361,12 @@ void op_voxel_to_node(nrh_f3d *h, float weight) {
         for (int i = 0; i < 3; ++i)
             for (int j = 0; j < 3; ++j) R.m[i * 4 + j] = r.m[i][j];
     }
+}
+
+void op_voxel_to_node(nrh_f3d *h, float weight) {
+    NRH_REQUIRE(!h->voxelGrad.empty(), NRH_ERR_STATE, "no voxel-based gradient");
+    Affine T, R;
+    node_transforms(h, T, R);
     const float w = node_weight_ratio(h, weight);
     hipLaunchKernelGGL(k_voxel_to_node, dim3(blocks_for(h->G)), dim3(kBlock), 0, h->stream, h->voxelGrad.p, h->ref.nx,
                        h->ref.ny, h->ref.nz, h->cpp.nx, h->cpp.ny, h->cpp.nz, T, R, w, h->nodeGrad.p);

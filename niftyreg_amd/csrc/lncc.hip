@@ -436,6 +436,7 @@ int nrh_f3d_lncc_value(nrh_f3d *h, double *value) {
 int nrh_f3d_lncc_voxel_gradient(nrh_f3d *h, double weight) {
     return guard([&] {
         NRH_REQUIRE(h, NRH_ERR_ARG, "null handle");
+        settle_voxel_gradient(h);
         op_lncc_voxel_gradient(h, weight);
     });
 }
