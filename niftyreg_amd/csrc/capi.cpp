@@ -270,6 +270,7 @@ int nrh_f3d_set_params(nrh_f3d *h, const nrh_f3d_params *params) {
         if (params->field_order != h->params.field_order) settle_voxel_gradient(h);  // in the order it was asked in
         const bool bins = params->ref_bins != h->params.ref_bins || params->flo_bins != h->params.flo_bins;
         h->params = *params;
+        h->touch();
         if (bins) { alloc_histogram(h); h->histVersion = 0; }
     });
 }
@@ -298,6 +299,7 @@ int nrh_f3d_rescale_intensities(nrh_f3d *h, float ref_lo, float ref_hi, float fl
         op_rescale(h, h->floImg.p, h->Nf, flo_lo, flo_hi);
         NRH_HIP(hipStreamSynchronize(h->stream));
         h->histVersion = 0;
+        h->touch();
         h->halfDirty = true;
     });
 }

@@ -15,7 +15,42 @@ static void histogram_at_current_points(nrh_f3d *h) {
         op_joint_histogram(h, h->warped.p);
         op_nmi_finalize(h);
         h->histVersion = h->cppVersion;
+        h->evalVersion = h->cppVersion;
     }
+}
+
+// reg_f3d::WarpFloatingImage and reg_lncc's convolved sums
+static void lncc_at_current_points(nrh_f3d *h) {
+    if (fused_warp_supported(h)) {
+        fused_warp(h);
+    } else {
+        op_spline_field(h);
+        op_resample(h);
+    }
+    op_lncc_eval(h);
+    h->evalVersion = h->cppVersion;
+}
+
+// reg_f3d::GetSimilarityMeasureGradient with reg_lncc (reg-lib/_reg_f3d.cpp:353-362,
+// reg-lib/_reg_base.cpp:497-549) into the node gradient.  A gradient at the points of the last
+// objective finds the warp and the sums in place, as the NMI one finds its histogram.
+static void lncc_gradient(nrh_f3d *h, float weight) {
+    if (h->evalVersion != h->cppVersion) lncc_at_current_points(h);
+    op_image_gradient(h);
+    op_lncc_eval_voxel_gradient(h, 1.0);
+    // convolution + node extraction: the separable projection when the nodes lie on voxels at an
+    // integer spacing, else the reference-order convolution
+    if (fused_projection_supported(h)) fused_project(h, h->voxelGrad.p, weight);
+    else op_voxel_gradient_to_nodes(h, weight);
+}
+
+// The same with reg_nmi where the fused sweeps do not apply.
+static void nmi_chain_gradient(nrh_f3d *h, float weight) {
+    if (h->evalVersion != h->cppVersion) histogram_at_current_points(h);
+    op_image_gradient(h);
+    zero_voxel_gradient(h);
+    op_nmi_voxel_gradient(h, 1.0);
+    op_voxel_gradient_to_nodes(h, weight);
 }
 
 }  // namespace nrh
@@ -39,10 +74,8 @@ static void enqueue_objective(nrh_f3d *h) {
     const bool beFused = p.be_weight > 0 && p.similarity_weight > 0 && !lncc && fused_supported(h);
     if (p.similarity_weight > 0) {
         if (lncc) {
-            // reg_f3d::WarpFloatingImage then reg_lncc::GetSimilarityMeasureValueFw
-            op_spline_field(h);
-            op_resample(h);
-            op_lncc_value(h, h->scalars.p + 4);
+            lncc_at_current_points(h);
+            op_lncc_eval_value(h, h->scalars.p + 4);
         } else if (beFused) {
             // with no linear energy to wait for, the finalisation publishes the results itself
             if (p.le_weight > 0) fused_histogram(h, nullptr, true);
@@ -89,10 +122,8 @@ int nrh_f3d_similarity_value(nrh_f3d *h, double *value) {
         NRH_REQUIRE(!h->velocity, NRH_ERR_UNSUPPORTED, "velocity grids are evaluated with nrh_f3d2_objective");
         const bool lncc = h->params.measure == NRH_MEASURE_LNCC;
         if (lncc) {
-            // reg_f3d::WarpFloatingImage then reg_lncc::GetSimilarityMeasureValueFw
-            op_spline_field(h);
-            op_resample(h);
-            op_lncc_value(h, h->scalars.p + 4);
+            lncc_at_current_points(h);
+            op_lncc_eval_value(h, h->scalars.p + 4);
         } else {
             histogram_at_current_points(h);
         }
@@ -108,25 +139,12 @@ int nrh_f3d_similarity_gradient(nrh_f3d *h, float weight) {
         NRH_REQUIRE(h, NRH_ERR_ARG, "null handle");
         NRH_REQUIRE(!h->velocity, NRH_ERR_UNSUPPORTED, "velocity grids are evaluated with nrh_f3d2_gradient");
         if (h->params.measure == NRH_MEASURE_LNCC) {
-            op_spline_field(h);
-            op_resample(h);
-            op_image_gradient(h);
-            zero_voxel_gradient(h);
-            op_lncc_voxel_gradient(h, 1.0);
-            if (fused_projection_supported(h)) {
-                fused_project(h, h->voxelGrad.p, weight);
-            } else {
-                op_voxel_gradient_to_nodes(h, weight);
-            }
+            lncc_gradient(h, weight);
         } else if (fused_supported(h)) {
             if (h->histVersion != h->cppVersion) fused_histogram(h);
             fused_gradient(h, weight, 0.f, nullptr);
         } else {
-            histogram_at_current_points(h);
-            op_image_gradient(h);
-            zero_voxel_gradient(h);
-            op_nmi_voxel_gradient(h, 1.0);
-            op_voxel_gradient_to_nodes(h, weight);
+            nmi_chain_gradient(h, weight);
         }
     });
 }
@@ -138,20 +156,7 @@ static void gradient_body(nrh_f3d *h, double *max_length) {
         const bool be = p.be_weight > 0, le = p.le_weight > 0;
         bool beDone = false;
         if (p.similarity_weight > 0 && p.measure == NRH_MEASURE_LNCC) {
-            // reg_f3d::GetSimilarityMeasureGradient with reg_lncc (reg-lib/_reg_f3d.cpp:353-362,
-            // reg-lib/_reg_base.cpp:497-549)
-            op_spline_field(h);
-            op_resample(h);
-            op_image_gradient(h);
-            zero_voxel_gradient(h);
-            op_lncc_voxel_gradient(h, 1.0);
-            // convolution + node extraction: the separable projection when the nodes lie on
-            // voxels at an integer spacing, else the reference-order convolution
-            if (fused_projection_supported(h)) {
-                fused_project(h, h->voxelGrad.p, p.similarity_weight);
-            } else {
-                op_voxel_gradient_to_nodes(h, p.similarity_weight);
-            }
+            lncc_gradient(h, p.similarity_weight);
         } else if (p.similarity_weight > 0) {
             if (fused_supported(h)) {
                 // the bending-energy gradient sums run on the side stream beside the projection
@@ -162,16 +167,7 @@ static void gradient_body(nrh_f3d *h, double *max_length) {
                 fused_gradient(h, p.similarity_weight, be ? p.be_weight : 0.f, trackMax ? h->maxBits.p : nullptr);
                 beDone = be;
             } else {
-                // reg_f3d::GetSimilarityMeasureGradient chain (reg-lib/_reg_f3d.cpp:353-362)
-                op_spline_field(h);
-                op_resample(h);
-                op_joint_histogram(h, h->warped.p);
-                op_nmi_finalize(h);
-                h->histVersion = h->cppVersion;
-                op_image_gradient(h);
-                zero_voxel_gradient(h);
-                op_nmi_voxel_gradient(h, 1.0);
-                op_voxel_gradient_to_nodes(h, p.similarity_weight);
+                nmi_chain_gradient(h, p.similarity_weight);
             }
         } else {
             op_fill_f32(h->nodeGrad.p, 3 * h->G, 0.f, h->stream);
@@ -230,6 +226,7 @@ int nrh_f3d_fused_field(nrh_f3d *h) {
         NRH_REQUIRE(fused_supported(h), NRH_ERR_UNSUPPORTED, "fused path unavailable for this geometry");
         ensure_field(h);
         h->velFieldVersion = 0;
+        h->touch();
         fused_histogram(h, h->field.p);
         NRH_HIP(hipStreamSynchronize(h->stream));
         collect_sweep_times(h);

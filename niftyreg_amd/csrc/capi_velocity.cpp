@@ -158,7 +158,7 @@ int nrh_f3d_set_velocity_affines(nrh_f3d *h, const float *ext0, const float *ext
         if (transformation) std::memcpy(h->velTransM, transformation, sizeof h->velTransM);
         h->velFieldVersion = 0;
         h->velChainVersion = 0;
-        h->pairStateVersion = 0;
+        h->touch();
     });
 }
 
@@ -255,7 +255,7 @@ int nrh_f3d_upload_field(nrh_f3d *h, const float *planar) {
         NRH_REQUIRE(h && planar, NRH_ERR_ARG, "null argument");
         ensure_field(h);
         h->velFieldVersion = 0;
-        h->pairStateVersion = 0;
+        h->touch();
         NRH_HIP(hipMemcpyAsync(h->field.p, planar, 3 * h->N * sizeof(float), hipMemcpyHostToDevice, h->stream));
         NRH_HIP(hipStreamSynchronize(h->stream));
     });

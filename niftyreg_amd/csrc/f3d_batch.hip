@@ -188,7 +188,7 @@ void batch_touch(nrh_batch *b, bool pointsChanged) {
             h->histVersion = h->cppVersion;
         }
         h->kTabCurrent = false;  // the batch's finalisation leaves the pair's own table as it was
-        h->pairStateVersion = 0;
+        h->touch();
         h->velFieldVersion = 0;
     }
 }

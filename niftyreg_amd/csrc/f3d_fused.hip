@@ -1,8 +1,8 @@
 // Fused F3D evaluation for gfx950.
 //
-// One objective evaluation is one sweep over the reference grid (k_sweep<false>): B-spline
+// One objective evaluation is one sweep over the reference grid (k_sweep<T, kSweepHist>): B-spline
 // field, trilinear warp and joint-histogram fill, with no field or warped image written to HBM.
-// One gradient evaluation is a second sweep (k_sweep<true>): the field and warp are recomputed
+// One gradient evaluation is a second sweep (k_sweep<T, kSweepGrad>): the field and warp are recomputed
 // together with the image gradient and the NMI voxel gradient, which is written once (planar
 // [3][N]); three separable passes then project it onto the control points.
 //
@@ -66,7 +66,9 @@ struct FusedArgs {
     const double *ent;
     const float *kTab;  // gradient sweep: K[r + w rb] = log p_r + log p_w - NMI log p_rw (padded to 4)
     float *gvox;      // gradient sweep: the NMI voxel gradient (planar [3][N])
-    float *fieldOut;  // optional: the deformation field of the sweep (planar [3][N]), for checking
+    float *fieldOut;  // the deformation field of the sweep (planar [3][N]): warp sweep; optional in the
+                      // histogram sweep, for checking
+    float *warpOut;   // warp sweep: the warped image
     // voxels left to the exact pass: positions within ambTol (floating voxels) of a voxel plane;
     // tile t lists its voxels in ambList[t * kTileVoxels ..] and their number in ambCounts[t]
     uint32_t *ambList;
@@ -76,6 +78,10 @@ struct FusedArgs {
     int lut;         // 5-voxel spacing on every axis (the reference's table path)
     const double *logh;  // the reference's jointHistogramLog (exact pass of the gradient sweep)
 };
+
+// What a sweep makes of its voxels: the joint histogram, the NMI voxel gradient, or the warped image
+// (with the field in fieldOut).
+enum { kSweepHist = 0, kSweepGrad = 1, kSweepWarp = 2 };
 
 template<class T> __device__ __forceinline__ float ld(const T *p, size_t i);
 template<> __device__ __forceinline__ float ld<float>(const float *p, size_t i) { return p[i]; }
@@ -190,12 +196,12 @@ __device__ __forceinline__ void load_taps(const FusedArgs& a, const TImg *__rest
     }
 }
 
-// GRAD = false: counts the voxel's (reference, warped) bin, or, when the warped value lies within
+// Histogram sweep: counts the voxel's (reference, warped) bin, or, when the warped value lies within
 // its error bound of an integer (where the reference's bin index (int)war, and the in-range test,
 // flip with the last bits), lists the voxel for the exact pass instead.  The bound: a position
 // error of up to ambTol floating voxels per axis moves the trilinear value by at most the taps'
 // spread per axis, plus eight ulps for the interpolation's own rounding.  Called by every lane.
-template<bool GRAD>
+template<int MODE>
 __device__ __forceinline__ void sweep_finish(const FusedArgs& a, VoxelTaps t, float *dyn, double coef, float& g0,
                                              float& g1, float& g2, uint32_t idx, uint32_t *ambList,
                                              uint32_t *ambCount) {
@@ -210,7 +216,9 @@ __device__ __forceinline__ void sweep_finish(const FusedArgs& a, VoxelTaps t, fl
     const float f0 = e00 * y0b + e01 * ry, f1 = e10 * y0b + e11 * ry;
     const float war = f0 * z0b + f1 * rz;
     const float rv = t.rv;
-    if (!GRAD) {
+    if (MODE == kSweepWarp) {
+        if (t.active) a.warpOut[idx] = war;
+    } else if (MODE == kSweepHist) {
         bool edge = false;
         if (t.active && rv == rv && war == war) {
             float lo = t.v[0][0][0], hi = lo;
@@ -353,8 +361,8 @@ __device__ __forceinline__ float3 gradient_taps(const float v[2][2][2], float3 p
 }
 
 // One listed voxel idx of pair a: the histogram pass counts it into the tile's LDS histogram h,
-// the gradient pass writes its voxel gradient.
-template<class TImg, bool GRAD>
+// the gradient pass writes its voxel gradient, the warp pass its field and warped value.
+template<class TImg, int MODE>
 __device__ __forceinline__ void fixup_voxel(const FusedArgs& a, const uint32_t idx, uint32_t *h) {
     const TImg *__restrict__ ref = (const TImg *)a.ref;
     const TImg *__restrict__ flo = (const TImg *)a.flo;
@@ -371,7 +379,13 @@ __device__ __forceinline__ void fixup_voxel(const FusedArgs& a, const uint32_t i
     exact_taps(flo, a.fnx, a.fny, a.fnz, px, py, pz, a.pad, v);
     const float rv = ld(ref, idx);
     const float war = sample_taps(v, p, px, py, pz);
-    if (!GRAD) {
+    if (MODE == kSweepWarp) {
+        const uint32_t N = (uint32_t)a.nx * a.ny * a.nz;
+        a.fieldOut[idx] = w.x;
+        a.fieldOut[idx + N] = w.y;
+        a.fieldOut[idx + 2 * N] = w.z;
+        a.warpOut[idx] = war;
+    } else if (MODE == kSweepHist) {
         if (rv == rv && war == war && rv >= 0.f && rv < (float)a.rb && war >= 0.f && war < (float)a.fb)
             atomicAdd(&h[(int)rv + (int)war * a.rb], 1u);
     } else {
@@ -393,7 +407,7 @@ __device__ __forceinline__ void fixup_voxel(const FusedArgs& a, const uint32_t i
 // the histogram pass counts them in one LDS histogram h per workgroup and merges it once.
 constexpr int kFixChunk = 8;  // tiles per exact-pass workgroup
 
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __device__ __forceinline__ void fixup_tiles(const FusedArgs& a, const int t0, const int nt, uint32_t *h) {
     __shared__ uint32_t sOff[kFixChunk + 1];
     const int tid = threadIdx.x;
@@ -408,7 +422,7 @@ __device__ __forceinline__ void fixup_tiles(const FusedArgs& a, const int t0, co
     __syncthreads();
     const uint32_t total = sOff[kFixChunk];
     if (total == 0) return;  // uniform over the workgroup
-    if (!GRAD) {
+    if (MODE == kSweepHist) {
         for (int i = tid; i < a.rb * a.fb; i += blockDim.x) h[i] = 0u;
         __syncthreads();
     }
@@ -416,20 +430,20 @@ __device__ __forceinline__ void fixup_tiles(const FusedArgs& a, const int t0, co
         int k = 0;
         while (i >= sOff[k + 1]) ++k;
         const uint32_t idx = a.ambList[(size_t)(t0 + k) * kTileVoxels + (i - sOff[k])];
-        fixup_voxel<TImg, GRAD>(a, idx, h);
+        fixup_voxel<TImg, MODE>(a, idx, h);
     }
-    if (!GRAD) {
+    if (MODE == kSweepHist) {
         __syncthreads();
         for (int i = tid; i < a.rb * a.fb; i += blockDim.x)
             if (h[i]) atomicAdd(&a.hist[i], h[i]);
     }
 }
 
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __global__ void __launch_bounds__(256) k_sweep_fixup(FusedArgs a) {
     extern __shared__ __align__(16) uint32_t fixLds[];  // histogram counts (objective pass)
     const int t0 = blockIdx.x * kFixChunk;
-    fixup_tiles<TImg, GRAD>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
+    fixup_tiles<TImg, MODE>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
 }
 
 // The histogram pass's exact pass with the bending energy in the same launch: workgroups
@@ -456,17 +470,17 @@ __global__ void __launch_bounds__(256) k_sweep_fixup_be(FusedArgs a, BeValueArgs
         return;
     }
     const int t0 = ((int)blockIdx.x - be.nb) * kFixChunk;
-    fixup_tiles<TImg, false>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
+    fixup_tiles<TImg, kSweepHist>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
 }
 
 // Batched: one workgroup per chunk (pair, first tile, tiles) of the exact-pass chunk list.
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __global__ void __launch_bounds__(256)
 k_sweep_fixup_batch(const FusedArgs *__restrict__ A, const int4 *__restrict__ chunks, const int *active) {
     extern __shared__ __align__(16) uint32_t fixLds[];
     const int4 c = chunks[blockIdx.x];
     if (active && !active[c.x]) return;
-    fixup_tiles<TImg, GRAD>(A[c.x], c.y, c.z, fixLds);
+    fixup_tiles<TImg, MODE>(A[c.x], c.y, c.z, fixLds);
 }
 
 // A 64 x 8 x 8 tile per workgroup.  The control-point window is staged in LDS and contracted
@@ -483,7 +497,7 @@ struct SweepShared {
 
 // One tile t of the pair described by a; dyn: the dynamic LDS (window [3][WZM][WYM][WXM], then
 // the histogram or the table K).  Called by every thread of the workgroup.
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, SweepShared& S, float *dyn) {
     auto& sAyz = S.sAyz;
     auto& sIdYZ = S.sIdYZ;
@@ -578,7 +592,7 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
     }
     __syncthreads();
     double coef = 0.0;
-    if (GRAD) {
+    if (MODE == kSweepGrad) {
         // the table K of k_nmi_table: the voxel NMI derivative is the bicubic contraction
         // sum_r sum_w B(ref - r) B'(war - w) K[r, w]; four float4 loads in flight per thread
         const int n4 = (a.rb * a.fb + 3) / 4;
@@ -596,7 +610,7 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
             }
         }
         coef = 1.0 / (a.ent[2] * a.ent[3]);
-    } else {
+    } else if (MODE == kSweepHist) {
         uint32_t *h = (uint32_t *)dyn;
         for (int i = tid; i < a.rb * a.fb; i += kThreads) h[i] = 0u;
     }
@@ -611,7 +625,7 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
         const double ux = (double)px + (double)(b.y + 2.f * b.z + 3.f * b.w);
         const double idX[3] = { (double)a.cppXyz.m[0] * ux, (double)a.cppXyz.m[4] * ux, (double)a.cppXyz.m[8] * ux };
         const uint32_t N = (uint32_t)a.nx * a.ny * a.nz;
-        float *fieldOut = GRAD ? nullptr : a.fieldOut;
+        float *fieldOut = MODE == kSweepGrad ? nullptr : a.fieldOut;
         constexpr int kRowsPerWave = TY / (kThreads / 64);
         for (int z = 0; z < nZ; ++z) {
             // the rows of this wave in slice z: every tap is loaded before any is used
@@ -642,15 +656,15 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
                 t[k].rx = pos[k].rx;
                 t[k].ry = pos[k].ry;
                 t[k].rz = pos[k].rz;
-                t[k].rv = ld(ref, idx[k]);
+                t[k].rv = MODE == kSweepWarp ? 0.f : ld(ref, idx[k]);
             }
 #pragma unroll
             for (int k = 0; k < kRowsPerWave; ++k) {
                 const int y = wave + k * (kThreads / 64);
                 if (y >= nY) continue;  // uniform over the wave
                 float g0, g1, g2;
-                sweep_finish<GRAD>(a, t[k], dyn, coef, g0, g1, g2, idx[k], ambList, &S.ambCount);
-                if (GRAD) {
+                sweep_finish<MODE>(a, t[k], dyn, coef, g0, g1, g2, idx[k], ambList, &S.ambCount);
+                if (MODE == kSweepGrad) {
                     a.gvox[idx[k]] = g0;
                     a.gvox[idx[k] + N] = g1;
                     a.gvox[idx[k] + 2 * N] = g2;
@@ -660,20 +674,20 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
     }
     __syncthreads();
     if (tid == 0) a.ambCounts[t] = S.ambCount;
-    if (!GRAD) {
+    if (MODE == kSweepHist) {
         const uint32_t *h = (const uint32_t *)dyn;
         for (int i = tid; i < a.rb * a.fb; i += kThreads)
             if (h[i]) atomicAdd(&a.hist[i], h[i]);
     }
 }
 
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __global__ void __launch_bounds__(kThreads) k_sweep(FusedArgs a) {
     __shared__ SweepShared S;
     extern __shared__ __align__(16) float dyn[];
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     if (t >= a.numTiles) return;
-    sweep_tile<TImg, GRAD>(a, t, S, dyn);
+    sweep_tile<TImg, MODE>(a, t, S, dyn);
 }
 
 // Persistent sweep over the (pair, tile) work list of a batch of pairs: item = pair << 20 | tile,
@@ -681,7 +695,7 @@ __global__ void __launch_bounds__(kThreads) k_sweep(FusedArgs a) {
 // b % 8), so a pair's tiles, which read overlapping floating-image lines, share one L2; the
 // workgroups of an XCD take the items of its range in turn.  Items of pairs whose flag in
 // `active` is 0 are skipped (a line search that has ended for that pair).
-template<class TImg, bool GRAD>
+template<class TImg, int MODE>
 __global__ void __launch_bounds__(kThreads)
 k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ items, int nItems,
               const int *__restrict__ active) {
@@ -694,7 +708,7 @@ k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ i
         const uint32_t it = __builtin_amdgcn_readfirstlane(items[i]);  // uniform: scalar loads of the arguments
         const int pair = (int)(it >> 20);
         if (active && !active[pair]) continue;  // uniform over the workgroup
-        sweep_tile<TImg, GRAD>(args[pair], (int)(it & 0xfffffu), S, dyn);
+        sweep_tile<TImg, MODE>(args[pair], (int)(it & 0xfffffu), S, dyn);
         __syncthreads();  // the next tile reuses the LDS
     }
 }
@@ -1253,9 +1267,9 @@ void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pu
     const bool timed = h->profile && h->profileSeen[0]++ % h->profilePeriod == 0;
     if (timed) NRH_HIP(hipEventRecord(h->ev[0], h->stream));
     if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep<__half, false>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep<__half, kSweepHist>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
     else
-        hipLaunchKernelGGL((k_sweep<float, false>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep<float, kSweepHist>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
     NRH_HIP(hipGetLastError());
     if (timed) {
         NRH_HIP(hipEventRecord(h->ev[1], h->stream));
@@ -1282,15 +1296,42 @@ void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pu
         else
             hipLaunchKernelGGL(k_sweep_fixup_be<float>, grid, dim3(256), fixLds, h->stream, a, be, be_basis());
     } else if (h->params.image_storage == 1) {
-        hipLaunchKernelGGL((k_sweep_fixup<__half, false>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepHist>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
     } else {
-        hipLaunchKernelGGL((k_sweep_fixup<float, false>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep_fixup<float, kSweepHist>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
     }
     NRH_HIP(hipGetLastError());
     // the finalisation also writes the gradient sweep's NMI table
     p->kTab.alloc((size_t)(a.rb * a.fb + 3) / 4 * 4);
     op_nmi_finalize(h, p->kTab.p, pubS1, pubN1);
     h->histVersion = h->cppVersion;
+}
+
+// The warped image and the field of the current points (the exact pass's voxels in the reference's
+// order, as everywhere on the fused path): one sweep without histogram in place of a kernel for the
+// field's 64 sums per voxel and one for the resampling.  float32 images, whatever the storage.
+bool fused_warp_supported(nrh_f3d *h) {
+    return plan_of(h)->ok && 3 * (size_t)h->N <= 0xffffffffull && (size_t)h->Nf <= 0xffffffffull;
+}
+
+void fused_warp(nrh_f3d *h) {
+    FusedPlan *p = plan_of(h);
+    NRH_REQUIRE(fused_warp_supported(h), NRH_ERR_UNSUPPORTED, "fused path unavailable for this geometry");
+    ensure_field(h);
+    ensure_warped(h);
+    h->velFieldVersion = 0;
+    h->touch();
+    FusedArgs a = make_args(h, p);
+    a.ref = h->refImg.p;
+    a.flo = h->floImg.p;
+    a.fieldOut = h->field.p;
+    a.warpOut = h->warped.p;
+    const size_t lds = (size_t)3 * (WZM + TZ) * WYM * WXM * sizeof(float);
+    hipLaunchKernelGGL((k_sweep<float, kSweepWarp>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
+    NRH_HIP(hipGetLastError());
+    hipLaunchKernelGGL((k_sweep_fixup<float, kSweepWarp>), dim3((unsigned)((p->numTiles + kFixChunk - 1) / kFixChunk)),
+                       dim3(256), 0, h->stream, a);
+    NRH_HIP(hipGetLastError());
 }
 
 // Arguments of the three projection passes of the voxel gradient g (planar [3][N]) onto the
@@ -1389,9 +1430,9 @@ void fused_gradient(nrh_f3d *h, float weight, float beWeight, uint32_t *maxBits)
     const bool timed = h->profile && h->profileSeen[1]++ % h->profilePeriod == 0;
     if (timed) NRH_HIP(hipEventRecord(h->ev[2], h->stream));
     if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep<__half, true>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep<__half, kSweepGrad>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
     else
-        hipLaunchKernelGGL((k_sweep<float, true>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
+        hipLaunchKernelGGL((k_sweep<float, kSweepGrad>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
     NRH_HIP(hipGetLastError());
     if (timed) {
         NRH_HIP(hipEventRecord(h->ev[3], h->stream));
@@ -1399,9 +1440,9 @@ void fused_gradient(nrh_f3d *h, float weight, float beWeight, uint32_t *maxBits)
     }
     const dim3 fixGrid((unsigned)((p->numTiles + kFixChunk - 1) / kFixChunk));
     if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep_fixup<__half, true>), fixGrid, dim3(256), 0, h->stream, a);
+        hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepGrad>), fixGrid, dim3(256), 0, h->stream, a);
     else
-        hipLaunchKernelGGL((k_sweep_fixup<float, true>), fixGrid, dim3(256), 0, h->stream, a);
+        hipLaunchKernelGGL((k_sweep_fixup<float, kSweepGrad>), fixGrid, dim3(256), 0, h->stream, a);
     NRH_HIP(hipGetLastError());
     project_to_nodes(h, p, p->gvox.p, weight, beWeight, maxBits);
     if (beWeight > 0.f) h->cppVersion++;  // the round trip may have changed the last bit of some points
@@ -1499,14 +1540,14 @@ void batch_histogram(nrh_batch *b, const int *active) {
     // the pairs' counts are zero here: allocation zeroes them and every finalisation consumes them
     const bool half = b->pairs[0]->params.image_storage == 1;
     if (half) {
-        hipLaunchKernelGGL((k_sweep_batch<__half, false>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_batch<__half, kSweepHist>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
                            A, b->sweepItems.p, b->nSweepItems, active);
-        hipLaunchKernelGGL((k_sweep_fixup_batch<__half, false>), dim3(b->nFixChunks), dim3(256), b->fixLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_fixup_batch<__half, kSweepHist>), dim3(b->nFixChunks), dim3(256), b->fixLds, b->stream,
                            A, b->fixChunks.p, active);
     } else {
-        hipLaunchKernelGGL((k_sweep_batch<float, false>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_batch<float, kSweepHist>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
                            A, b->sweepItems.p, b->nSweepItems, active);
-        hipLaunchKernelGGL((k_sweep_fixup_batch<float, false>), dim3(b->nFixChunks), dim3(256), b->fixLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_fixup_batch<float, kSweepHist>), dim3(b->nFixChunks), dim3(256), b->fixLds, b->stream,
                            A, b->fixChunks.p, active);
     }
     NRH_HIP(hipGetLastError());
@@ -1518,14 +1559,14 @@ void batch_similarity_gradient(nrh_batch *b, const int *active) {
     hipLaunchKernelGGL(k_nmi_table_batch, dim3((b->rb * b->fb + 255) / 256, b->P), dim3(256), 0, b->stream, A, active);
     const bool half = b->pairs[0]->params.image_storage == 1;
     if (half) {
-        hipLaunchKernelGGL((k_sweep_batch<__half, true>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_batch<__half, kSweepGrad>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
                            A, b->sweepItems.p, b->nSweepItems, active);
-        hipLaunchKernelGGL((k_sweep_fixup_batch<__half, true>), dim3(b->nFixChunks), dim3(256), 0, b->stream, A,
+        hipLaunchKernelGGL((k_sweep_fixup_batch<__half, kSweepGrad>), dim3(b->nFixChunks), dim3(256), 0, b->stream, A,
                            b->fixChunks.p, active);
     } else {
-        hipLaunchKernelGGL((k_sweep_batch<float, true>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
+        hipLaunchKernelGGL((k_sweep_batch<float, kSweepGrad>), dim3(b->sweepBlocks), dim3(kThreads), b->sweepLds, b->stream,
                            A, b->sweepItems.p, b->nSweepItems, active);
-        hipLaunchKernelGGL((k_sweep_fixup_batch<float, true>), dim3(b->nFixChunks), dim3(256), 0, b->stream, A,
+        hipLaunchKernelGGL((k_sweep_fixup_batch<float, kSweepGrad>), dim3(b->nFixChunks), dim3(256), 0, b->stream, A,
                            b->fixChunks.p, active);
     }
     hipLaunchKernelGGL(k_project_x_batch, dim3(b->nProjX), dim3(256), b->projXLds, b->stream,

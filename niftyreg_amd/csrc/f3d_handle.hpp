@@ -65,6 +65,7 @@ struct nrh_f3d {
 
     // LNCC: two ping-pong sets of planar numerators + density, combined mask, reductions
     nrh::DevBuf<float> lnccA, lnccB, lnccKern;
+    nrh::DevBuf<double> lnccKernD;  // the kernels as double
     nrh::DevBuf<uint8_t> lnccComb;
     nrh::DevBuf<double> lnccPart, lnccScalars;  // scalars: adjusted weight, -, value, active count
     float lnccSigma = 0.f;
@@ -87,6 +88,11 @@ struct nrh_f3d {
     // cppVersion at which the symmetric evaluation left the warped image and the joint histogram
     // of the current exponentiation (0: some other operation changed them since)
     uint64_t pairStateVersion = 0;
+    // cppVersion at which an evaluation left its field, warped image and measure state (the joint
+    // histogram's logs on the per-operation chain, the convolved LNCC sums) for a gradient at the
+    // same points (0: some other operation changed them since)
+    uint64_t evalVersion = 0;
+    void touch() { pairStateVersion = evalVersion = 0; }
     // affine components of a velocity grid: its NIfTI extensions 0 (applied before the spline,
     // removed before the squaring and restored after it) and 1 (composed after it), and the
     // content's transformation matrix (removed from the opposite direction's intermediate fields)
@@ -179,6 +185,12 @@ void wait_published(nrh_f3d *h);
 // LNCC measure (lncc.hip); value = mean |local correlation| into out_device[0] (count in [1])
 void op_lncc_value(nrh_f3d *h, double *out_device);
 void op_lncc_voxel_gradient(nrh_f3d *h, double weight);
+// The same for the evaluations, in fewer passes and with sums that differ in rounding (lncc.hip):
+// op_lncc_eval leaves the convolved sums of the warped image, from which the value and the gradient
+// are formed; the gradient is written over voxelGrad and uses the sums up.
+void op_lncc_eval(nrh_f3d *h);
+void op_lncc_eval_value(nrh_f3d *h, double *out_device);
+void op_lncc_eval_voxel_gradient(nrh_f3d *h, double weight);
 
 float node_weight_ratio(const nrh_f3d *h, float weight);
 void op_normalise_device(nrh_f3d *h);
@@ -197,6 +209,8 @@ void op_symmetrise_velocity(nrh_f3d *fw, nrh_f3d *bw);
 // fused evaluation (f3d_fused.hip)
 bool fused_supported(nrh_f3d *h);
 void fused_release(const nrh_f3d *h);
+bool fused_warp_supported(nrh_f3d *h);
+void fused_warp(nrh_f3d *h);
 // beValue: also the bending energy (into scalars[0]), in the exact pass's launch
 // pubN1 >= 0: the finalisation also publishes the entropies and NMI followed by pubS1[0..pubN1)
 // (op_publish's layout, the sequence number advanced)

@@ -936,7 +936,7 @@ void op_vel_def_field(nrh_f3d *h, bool update) {
     }
     h->velFieldVersion = 0;
     h->velChainVersion = 0;
-    h->pairStateVersion = 0;
+    h->touch();
     ensure_field(h);
     const FieldGeom f = field_geom(h->ref);
     const VelGrid g = vel_grid(h);
@@ -1081,7 +1081,7 @@ void op_resample_gradient(nrh_f3d *h, float pad, float *out) {
 void op_compose_field(nrh_f3d *h, const nrh_geom& g, const float *def) {
     NRH_REQUIRE(!h->field.empty(), NRH_ERR_STATE, "deformation field not computed");
     h->velFieldVersion = 0;
-    h->pairStateVersion = 0;
+    h->touch();
     launch_compose(def, field_geom(g), h->field.p, h->N, h->field.p, h->stream);
     NRH_HIP(hipGetLastError());
 }

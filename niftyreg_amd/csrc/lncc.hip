@@ -7,7 +7,9 @@
 // density together: planar [K + 1][N] arrays, one launch per axis, ping-ponging between two
 // buffers.  Each output sample is the reference's line sum in the reference's order (float
 // products added in double, reg-lib/cpu/_reg_tools.cpp:1047-1053), so the results equal the
-// reference's scalar build bit for bit.
+// reference's scalar build bit for bit.  That is the per-operation measure (op_lncc_value,
+// op_lncc_voxel_gradient).  The evaluations take the passes at the end of the kernels below, which
+// form the same sums without rounding the products and in fewer trips to memory.
 
 #include "f3d_handle.hpp"
 #include "device.hpp"
@@ -163,8 +165,57 @@ k_conv_lines_x(const float *__restrict__ in, float *__restrict__ out, int K, siz
     }
 }
 
-// Local statistics (UpdateLocalStatImages, reg-lib/cpu/_reg_lncc.cpp:236-244) and the per-voxel
-// |local correlation| of reg_getLnccValue (:282-297), reduced per block in a fixed order.
+// The local means and deviations of UpdateLocalStatImages (reg-lib/cpu/_reg_lncc.cpp:236-244) from a
+// voxel's six convolved sums (ref, ref^2, warped, warped^2, ref * warped, density).
+struct LocalStats {
+    float mean, wmean, corr, sdev, wsdev;
+};
+
+__device__ __forceinline__ LocalStats local_stats(float r, float rr, float w, float ww, float rw, float d) {
+#pragma clang fp contract(off)
+    LocalStats s;
+    s.mean = r / d;
+    s.wmean = w / d;
+    s.corr = rw / d;
+    const float sq = rr / d, wsq = ww / d;
+    s.sdev = sqrtf(sq - s.mean * s.mean);
+    s.wsdev = sqrtf(wsq - s.wmean * s.wmean);
+    if (s.sdev < 1.e-06) s.sdev = 0.f;
+    if (s.wsdev < 1.e-06) s.wsdev = 0.f;
+    return s;
+}
+
+// |local correlation| of reg_getLnccValue (:282-297); false where it is no number.
+__device__ __forceinline__ bool lncc_value_term(const LocalStats& s, double& v) {
+#pragma clang fp contract(off)
+    const double l = (double)((s.corr - (s.mean * s.wmean)) / (s.sdev * s.wsdev));
+    v = fabs(l);
+    return l == l && !isinf(l);
+}
+
+// The three derivative terms of reg_getVoxelBasedLnccGradient (:441-470); false (and zero) where one
+// is no number.
+__device__ __forceinline__ bool lncc_gradient_terms(const LocalStats& s, float t[3]) {
+#pragma clang fp contract(off)
+    const double rm = s.mean, wm = s.wmean, rs = s.sdev, ws = s.wsdev;
+    const double c = (double)s.corr - (rm * wm);
+    double t1 = 1.0 / (rs * ws);
+    double t2 = c / (rs * ws * ws * ws);
+    double t3 = (c * wm) / (rs * ws * ws * ws) - rm / (rs * ws);
+    t[0] = t[1] = t[2] = 0.f;
+    if (!(t1 == t1 && !isinf(t1) && t2 == t2 && !isinf(t2) && t3 == t3 && !isinf(t3))) return false;
+    if (c < 0) {
+        t1 = -t1;
+        t2 = -t2;
+        t3 = -t3;
+    }
+    t[0] = (float)t1;
+    t[1] = (float)t2;
+    t[2] = (float)t3;
+    return true;
+}
+
+// The value's terms from the six convolved arrays, reduced per block in a fixed order.
 __global__ void __launch_bounds__(kB)
 k_lncc_value(const float *__restrict__ C, const uint8_t *__restrict__ comb, size_t N, double *__restrict__ partSum,
              unsigned long long *__restrict__ partCnt) {
@@ -175,15 +226,9 @@ k_lncc_value(const float *__restrict__ C, const uint8_t *__restrict__ comb, size
     unsigned long long cnt = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (size_t)gridDim.x * blockDim.x) {
         if (!comb[i]) continue;
-        const float d = C[5 * N + i];
-        const float mean = C[i] / d, sq = C[N + i] / d, wmean = C[2 * N + i] / d, wsq = C[3 * N + i] / d;
-        const float corr = C[4 * N + i] / d;
-        float sdev = sqrtf(sq - mean * mean), wsdev = sqrtf(wsq - wmean * wmean);
-        if (sdev < 1.e-06) sdev = 0.f;
-        if (wsdev < 1.e-06) wsdev = 0.f;
-        const double l = (double)((corr - (mean * wmean)) / (sdev * wsdev));
-        if (l == l && !isinf(l)) {
-            sum += fabs(l);
+        double l;
+        if (lncc_value_term(local_stats(C[i], C[N + i], C[2 * N + i], C[3 * N + i], C[4 * N + i], C[5 * N + i]), l)) {
+            sum += l;
             ++cnt;
         }
     }
@@ -233,7 +278,7 @@ __global__ void k_lncc_finish(const double *__restrict__ partSum, const unsigned
     }
 }
 
-// The three per-voxel derivative terms of reg_getVoxelBasedLnccGradient (:441-470), written as
+// The three per-voxel derivative terms, written as
 // the numerators of the second convolution set (density last), and the active-voxel count.
 __global__ void __launch_bounds__(kB)
 k_lncc_terms(const float *__restrict__ C, const uint8_t *__restrict__ comb, size_t N, float *__restrict__ T,
@@ -242,34 +287,13 @@ k_lncc_terms(const float *__restrict__ C, const uint8_t *__restrict__ comb, size
     __shared__ unsigned long long sC[kB / 64];
     unsigned long long cnt = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (size_t)gridDim.x * blockDim.x) {
-        float t1f = 0.f, t2f = 0.f, t3f = 0.f;
-        if (comb[i]) {
-            const float d = C[5 * N + i];
-            const float mean = C[i] / d, sq = C[N + i] / d, wmean = C[2 * N + i] / d, wsq = C[3 * N + i] / d;
-            const float corr = C[4 * N + i] / d;
-            float sdev = sqrtf(sq - mean * mean), wsdev = sqrtf(wsq - wmean * wmean);
-            if (sdev < 1.e-06) sdev = 0.f;
-            if (wsdev < 1.e-06) wsdev = 0.f;
-            const double rm = mean, wm = wmean, rs = sdev, ws = wsdev;
-            const double c = (double)corr - (rm * wm);
-            double t1 = 1.0 / (rs * ws);
-            double t2 = c / (rs * ws * ws * ws);
-            double t3 = (c * wm) / (rs * ws * ws * ws) - rm / (rs * ws);
-            if (t1 == t1 && !isinf(t1) && t2 == t2 && !isinf(t2) && t3 == t3 && !isinf(t3)) {
-                if (c < 0) {
-                    t1 = -t1;
-                    t2 = -t2;
-                    t3 = -t3;
-                }
-                t1f = (float)t1;
-                t2f = (float)t2;
-                t3f = (float)t3;
-                ++cnt;
-            }
-        }
-        T[i] = t1f;
-        T[N + i] = t2f;
-        T[2 * N + i] = t3f;
+        float t[3] = { 0.f, 0.f, 0.f };
+        if (comb[i] &&
+            lncc_gradient_terms(local_stats(C[i], C[N + i], C[2 * N + i], C[3 * N + i], C[4 * N + i], C[5 * N + i]), t))
+            ++cnt;
+        T[i] = t[0];
+        T[N + i] = t[1];
+        T[2 * N + i] = t[2];
         T[3 * N + i] = comb[i] ? 1.f : 0.f;
     }
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_down(cnt, off, 64);
@@ -313,6 +337,347 @@ k_lncc_apply(const float *__restrict__ T, const uint8_t *__restrict__ comb, cons
     }
 }
 
+// ------------------------------------------------------------------ evaluation passes
+// The evaluations' convolutions.  Per tap a fused multiply-add in double of the exact product, where
+// the per-operation passes round the product to float, widen it and add (three instructions, the
+// widening at a quarter of the rate): the sums are closer to exact, and each axis still ends in one
+// rounding to float.  The lines lie in LDS as doubles, widened once per sample; a lane holds a sliding
+// window of 16 samples in registers for 8 outputs, so a sample is read from LDS about 5 times, not 31.
+// The x pass forms the six numerators from the two images as it stages them, and the z pass ends in
+// the value or the derivative terms, so that the six arrays cross memory four times instead of ten.
+// At 256 x 256 x 160, sigma 5 voxels (31 taps): the x, y and z passes of the six sums take 137, 175
+// and 205 us, about 300 each before, with a preparing and a reducing pass of 52 and 70 us; the
+// derivative's three arrays 78, 87 and 139 us.  The sums themselves are 50 us of each six-array pass
+// (double multiply-adds at the vector rate), its bytes 64, 97 and 48; the z pass also takes five
+// divisions and two square roots a voxel.
+constexpr int kEvalRadius = 30;  // radii above take the per-operation passes (LDS rows of 64 KB)
+constexpr int kColOut = 32;      // outputs along y / z per workgroup: four waves of 8
+constexpr int kEvalRows = 32;    // rows per workgroup of the x pass
+
+// chunks of 8 samples that 8 outputs over `taps` taps touch
+__host__ __device__ constexpr int eval_chunks(int taps) { return taps / 8 + 2; }
+size_t eval_lds_cols(int radius) {
+    return (size_t)8 * (kColOut / 8 - 1 + eval_chunks(2 * radius + 1)) * 64 * sizeof(double);
+}
+// x rows: chunk k of a row starts at 9 k doubles (the ninth unused), rows at a stride of 1 modulo 32:
+// the 8 segments of neighbouring rows then read distinct bank pairs but for one
+__host__ __device__ constexpr int eval_row_stride(int taps) { return (9 * (7 + eval_chunks(taps)) + 30) / 32 * 32 + 1; }
+size_t eval_lds_rows(int radius) { return (size_t)kEvalRows * eval_row_stride(2 * radius + 1) * sizeof(double); }
+
+// acc[o] = sum_k kern[k] s[o + k], o < 8, in ascending k, where sample 8 c + e lies at
+// base[c * CHUNK + e * STEP].  Samples past o + k = 7 + taps - 1 are loaded, not used.
+template<int CHUNK, int STEP>
+__device__ __forceinline__ void conv8(const double *base, const double *__restrict__ kern, int taps, double (&acc)[8]) {
+    double w[16];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        w[e] = base[e * STEP];
+        acc[e] = 0.0;
+    }
+    int c = 0;
+    for (; 8 * c + 8 <= taps; ++c) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * CHUNK + e * STEP];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const double kv = kern[8 * c + k];
+#pragma unroll
+            for (int o = 0; o < 8; ++o) acc[o] = fma(kv, w[o + k], acc[o]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = w[8 + e];
+    }
+    const int rest = taps - 8 * c;
+    if (rest > 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * CHUNK + e * STEP];
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+            if (k < rest) {  // uniform
+                const double kv = kern[8 * c + k];
+#pragma unroll
+                for (int o = 0; o < 8; ++o) acc[o] = fma(kv, w[o + k], acc[o]);
+            }
+    }
+}
+
+// x pass.  A lane takes 8 neighbouring outputs of one row (8 segments by 32 rows a workgroup).
+// FIRST: the six numerators of k_lncc_prepare, formed from the images, and the combined mask; else
+// array blockIdx.z of `in`.
+template<bool FIRST>
+__global__ void __launch_bounds__(kB)
+k_eval_x(const float *__restrict__ ref, const float *__restrict__ war, const int *__restrict__ mask,
+         const float *__restrict__ in, float *__restrict__ out, uint8_t *__restrict__ comb, size_t N, int nx, int nrows,
+         const double *__restrict__ kern, int radius) {
+#pragma clang fp contract(off)
+    extern __shared__ double rowsD[];
+    const int taps = 2 * radius + 1, W = 64 + 2 * radius, S = eval_row_stride(taps);
+    const int x0 = blockIdx.y * 64, row0 = blockIdx.x * kEvalRows;
+    // a wave stages every fourth row, a lane its samples `lane` and 64 + lane: every load in flight
+    // before one is used, addresses clamped to the image
+    constexpr int kEl = kEvalRows / (kB / 64);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float a[kEl][2], b[kEl][2];
+    bool ok[kEl][2];
+#pragma unroll
+    for (int e = 0; e < kEl; ++e)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int p = lane + 64 * h, x = x0 - radius + p, row = row0 + w + e * (kB / 64);
+            ok[e][h] = p < W && x >= 0 && x < nx && row < nrows;
+            const size_t i = (size_t)min(row, nrows - 1) * nx + min(max(x, 0), nx - 1);
+            if (FIRST) {
+                a[e][h] = ref[i];
+                b[e][h] = war[i];
+                if (mask) ok[e][h] = ok[e][h] && mask[i] > -1;
+            } else {
+                a[e][h] = in[blockIdx.z * N + i];
+            }
+        }
+    if (FIRST) {
+#pragma unroll
+        for (int e = 0; e < kEl; ++e)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int p = lane + 64 * h, x = x0 - radius + p, row = row0 + w + e * (kB / 64);
+                ok[e][h] = ok[e][h] && a[e][h] == a[e][h] && b[e][h] == b[e][h];
+                if (p >= radius && p < radius + 64 && x < nx && row < nrows)
+                    comb[(size_t)row * nx + x] = ok[e][h] ? 1 : 0;
+            }
+    }
+    const int seg = threadIdx.x & 7, r = threadIdx.x >> 3, row = row0 + r, x = x0 + 8 * seg;
+    const int at0 = (lane >> 3) * 9 + (lane & 7);
+#pragma unroll
+    for (int q = 0; q < (FIRST ? 6 : 1); ++q) {
+#pragma unroll
+        for (int e = 0; e < kEl; ++e)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float u = a[e][h], t = b[e][h];
+                const float v = !FIRST ? u : q == 0 ? u : q == 1 ? u * u : q == 2 ? t : q == 3 ? t * t : q == 4 ? u * t : 1.f;
+                if (lane + 64 * h < W)
+                    rowsD[(w + e * (kB / 64)) * S + at0 + 72 * h] = ok[e][h] ? (double)v : 0.0;
+            }
+        __syncthreads();
+        double acc[8];
+        conv8<9, 1>(rowsD + r * S + 9 * seg, kern, taps, acc);
+        float *dst = out + (size_t)(FIRST ? q : blockIdx.z) * N + (size_t)row * nx + x;
+        if (row < nrows && x + 8 <= nx) {
+            // two 16-byte stores (4-byte aligned)
+            typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
+            *reinterpret_cast<Float4 *>(dst) = Float4{ (float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3] };
+            *reinterpret_cast<Float4 *>(dst + 4) = Float4{ (float)acc[4], (float)acc[5], (float)acc[6], (float)acc[7] };
+        } else {
+#pragma unroll
+            for (int o = 0; o < 8; ++o)
+                if (row < nrows && x + o < nx) dst[o] = (float)acc[o];
+        }
+        __syncthreads();
+    }
+}
+
+// Columns of a y or z pass: column c of the flattened (x, outer) pairs starts at
+// c % nx + (c / nx) * outerStride, so a workgroup's 64 lanes are full whatever nx is.
+struct Columns {
+    size_t count, outerStride, lineStride;
+    int nx, L;
+};
+
+__device__ __forceinline__ size_t column_base(const Columns& c, size_t col) {
+    // (the column number fits 32 bits: an image of 2^32 columns has no room for its six arrays)
+    const uint32_t outer = (uint32_t)col / (uint32_t)c.nx;
+    return ((uint32_t)col - outer * (uint32_t)c.nx) + (size_t)outer * c.outerStride;
+}
+
+// One array's tile of 64 columns, positions t0 - radius ..: loaded (every load in flight before one is
+// used, addresses clamped to the line), then widened into LDS with zeros outside the line.  A pass
+// over several arrays loads the next while it sums the last.
+constexpr int kStage = (kColOut + 2 * kEvalRadius + kB / 64 - 1) / (kB / 64);
+
+__device__ __forceinline__ void load_columns(const float *__restrict__ src, const Columns& c, int t0, int radius,
+                                             float (&v)[kStage]) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rows = kColOut + 2 * radius;
+#pragma unroll
+    for (int u = 0; u < kStage; ++u) {
+        const int p = w + u * (kB / 64);
+        if (p < rows) v[u] = src[(size_t)min(max(t0 - radius + p, 0), c.L - 1) * c.lineStride];
+    }
+}
+
+__device__ __forceinline__ void store_columns(const float (&v)[kStage], const Columns& c, bool col, int t0, int radius,
+                                              double *tile) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rows = kColOut + 2 * radius;
+#pragma unroll
+    for (int u = 0; u < kStage; ++u) {
+        const int p = w + u * (kB / 64), pos = t0 - radius + p;
+        if (p < rows) tile[p * 64 + lane] = col && pos >= 0 && pos < c.L ? (double)v[u] : 0.0;
+    }
+}
+
+// y pass of array blockIdx.z.
+__global__ void __launch_bounds__(kB)
+k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Columns c, const double *__restrict__ kern,
+            int radius) {
+    extern __shared__ double tileD[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
+    const bool col = colIdx < c.count;
+    const size_t base = blockIdx.z * N + column_base(c, col ? colIdx : 0);
+    const int t0 = blockIdx.y * kColOut;
+    float v[kStage];
+    load_columns(in + base, c, t0, radius, v);
+    store_columns(v, c, col, t0, radius, tileD);
+    __syncthreads();
+    double acc[8];
+    conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        const int pos = t0 + w * 8 + o;
+        if (col && pos < c.L) out[base + (size_t)pos * c.lineStride] = (float)acc[o];
+    }
+}
+
+// z pass of the six sums, ending in the value's terms (GRAD = false: their sum and number per block)
+// or the derivative's (GRAD = true: three arrays and the convolved density into T, and their number).
+template<bool GRAD>
+__global__ void __launch_bounds__(kB)
+k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, size_t N, Columns c,
+             const double *__restrict__ kern, int radius, float *__restrict__ T, double *__restrict__ partSum,
+             unsigned long long *__restrict__ partCnt) {
+    extern __shared__ double tileD[];
+    __shared__ double sS[kB / 64];
+    __shared__ unsigned long long sC[kB / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
+    const bool col = colIdx < c.count;
+    const size_t base = column_base(c, col ? colIdx : 0);
+    const int t0 = blockIdx.y * kColOut;
+    float sum[6][8], v[kStage];
+    load_columns(in + base, c, t0, radius, v);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        store_columns(v, c, col, t0, radius, tileD);
+        __syncthreads();
+        if (q < 5) load_columns(in + (q + 1) * N + base, c, t0, radius, v);
+        double acc[8];
+        conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
+#pragma unroll
+        for (int o = 0; o < 8; ++o) sum[q][o] = (float)acc[o];
+        __syncthreads();
+    }
+    double s = 0.0;
+    unsigned long long cnt = 0;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        const int pos = t0 + w * 8 + o;
+        if (!(col && pos < c.L)) continue;
+        const size_t i = base + (size_t)pos * c.lineStride;
+        const bool used = comb[i] != 0;
+        const LocalStats st = local_stats(sum[0][o], sum[1][o], sum[2][o], sum[3][o], sum[4][o], sum[5][o]);
+        if (GRAD) {
+            float t[3] = { 0.f, 0.f, 0.f };
+            if (used && lncc_gradient_terms(st, t)) ++cnt;
+            T[i] = t[0];
+            T[N + i] = t[1];
+            T[2 * N + i] = t[2];
+            T[3 * N + i] = sum[5][o];
+        } else {
+            double l;
+            if (used && lncc_value_term(st, l)) {
+                s += l;
+                ++cnt;
+            }
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_down(s, off, 64);
+        cnt += __shfl_down(cnt, off, 64);
+    }
+    if (lane == 0) {
+        sS[w] = s;
+        sC[w] = cnt;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const size_t b = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+        for (int k = 1; k < kB / 64; ++k) {
+            s += sS[k];
+            cnt += sC[k];
+        }
+        partSum[b] = s;
+        partCnt[b] = cnt;
+    }
+}
+
+// z pass of the three derivative arrays, ending in k_lncc_apply's voxel gradient, which is written
+// (not added to); the density is the one of the six sums, convolved already.
+__global__ void __launch_bounds__(kB)
+k_eval_apply(const float *__restrict__ in, const uint8_t *__restrict__ comb, const float *__restrict__ dens, size_t N,
+             Columns c, const double *__restrict__ kern, int radius, const float *__restrict__ ref,
+             const float *__restrict__ war, const float *__restrict__ wgrad, const double *__restrict__ adjusted,
+             float *__restrict__ grad) {
+#pragma clang fp contract(off)
+    extern __shared__ double tileD[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
+    const bool col = colIdx < c.count;
+    const size_t base = column_base(c, col ? colIdx : 0);
+    const int t0 = blockIdx.y * kColOut;
+    float sum[3][8], v[kStage];
+    load_columns(in + base, c, t0, radius, v);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        store_columns(v, c, col, t0, radius, tileD);
+        __syncthreads();
+        if (q < 2) load_columns(in + (q + 1) * N + base, c, t0, radius, v);
+        double acc[8];
+        conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
+#pragma unroll
+        for (int o = 0; o < 8; ++o) sum[q][o] = (float)acc[o];
+        __syncthreads();
+    }
+    const double aw = adjusted[0];
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+        const int pos = t0 + w * 8 + o;
+        if (!(col && pos < c.L)) continue;
+        const size_t i = base + (size_t)pos * c.lineStride;
+        float g[3] = { 0.f, 0.f, 0.f };
+        if (comb[i]) {
+            const float d = dens[i];
+            const float t1 = sum[0][o] / d, t2 = sum[1][o] / d, t3 = sum[2][o] / d;
+            const double common = (double)(t1 * ref[i] - t2 * war[i] + t3) * aw;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float v = 0.f - (float)((double)wgrad[k * N + i] * common);
+                g[k] = v != v || isinf(v) ? 0.f : v;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) grad[k * N + i] = g[k];
+    }
+}
+
+// Sums of the block partials, one workgroup of 1024 in a fixed order; the value (out[0] = sum /
+// count, out[1] = count) or the gradient's weight (out[0] = weight / count).
+__global__ void __launch_bounds__(1024)
+k_eval_finish(const double *__restrict__ partSum, const unsigned long long *__restrict__ partCnt, int nb, int grad,
+              double weight, double *__restrict__ out) {
+    __shared__ double red[16];
+    double s = 0.0, n = 0.0;  // counts below 2^53 add exactly
+    for (int b = threadIdx.x; b < nb; b += 1024) {
+        if (!grad) s += partSum[b];
+        n += (double)partCnt[b];
+    }
+    s = block_sum_double(s, red);
+    n = block_sum_double(n, red);
+    if (threadIdx.x == 0) {
+        out[0] = grad ? weight / n : s / n;
+        if (!grad) out[1] = n;
+    }
+}
+
 // Gaussian kernel of reg_tools_kernelConvolution (:866-901); returns the radius.
 int gaussian_kernel(float sigma, float pixdim, std::vector<float>& k) {
     const double temp = sigma > 0 ? (double)(sigma / pixdim) : std::fabs((double)sigma);
@@ -323,12 +688,26 @@ int gaussian_kernel(float sigma, float pixdim, std::vector<float>& k) {
     return radius;
 }
 
+// columns and lines of the evaluation's z pass
+Columns z_columns(const nrh_f3d *h) {
+    const size_t plane = (size_t)h->ref.nx * h->ref.ny;
+    return { plane, (size_t)h->ref.nx, plane, h->ref.nx, h->ref.nz };
+}
+dim3 column_grid(const Columns& c, unsigned arrays) {
+    return dim3((unsigned)((c.count + 63) / 64), (unsigned)((c.L + kColOut - 1) / kColOut), arrays);
+}
+size_t eval_blocks(const nrh_f3d *h) {
+    const dim3 g = column_grid(z_columns(h), 1);
+    return (size_t)g.x * g.y;
+}
+
 void ensure_lncc(nrh_f3d *h) {
     const size_t N = h->N;
     h->lnccA.alloc(6 * N);
     h->lnccB.alloc(6 * N);
     h->lnccComb.alloc(N);
-    h->lnccPart.alloc(2 * kRedBlocks);
+    // partial sums and counts: the per-operation measure's blocks, or the evaluation's z-pass blocks
+    h->lnccPart.alloc(2 * std::max<size_t>(kRedBlocks, eval_blocks(h)));
     h->lnccScalars.alloc(4);
     if (h->lnccKern.empty() || h->lnccSigma != h->params.lncc_sigma) {
         std::vector<float> all;
@@ -339,6 +718,11 @@ void ensure_lncc(nrh_f3d *h) {
             h->lnccKernOff[a] = (int)all.size();
             all.insert(all.end(), k.begin(), k.end());
         }
+        std::vector<double> wide(all.begin(), all.end());
+        wide.push_back(1.0);  // the kernel of an axis that is not smoothed
+        h->lnccKernD.alloc(wide.size());
+        NRH_HIP(hipMemcpyAsync(h->lnccKernD.p, wide.data(), wide.size() * sizeof(double), hipMemcpyHostToDevice,
+                               h->stream));
         h->lnccKern.alloc(all.size());
         NRH_HIP(hipMemcpyAsync(h->lnccKern.p, all.data(), all.size() * sizeof(float), hipMemcpyHostToDevice,
                                h->stream));
@@ -381,13 +765,110 @@ float *convolve_set(nrh_f3d *h, float *a, float *b, int K1) {
 float *lncc_statistics(nrh_f3d *h) {
     NRH_REQUIRE(!h->warped.empty(), NRH_ERR_STATE, "LNCC needs the warped image");
     ensure_lncc(h);
+    h->evalVersion = 0;  // the evaluation's sums are overwritten
     hipLaunchKernelGGL(k_lncc_prepare, dim3(blocks_of(h->N)), dim3(kB), 0, h->stream, ref_ptr(h), h->warped.p,
                        h->mask.p, h->N, h->lnccComb.p, h->lnccA.p);
     NRH_HIP(hipGetLastError());
     return convolve_set(h, h->lnccA.p, h->lnccB.p, 6);
 }
 
+// Radius and kernel of one axis of the evaluation's passes: an axis that is not smoothed has the
+// single tap 1.
+int eval_axis(const nrh_f3d *h, int axis, const double **kern) {
+    const int dims[3] = { h->ref.nx, h->ref.ny, h->ref.nz };
+    const int r = h->lnccRadius[axis];
+    if (dims[axis] <= 1 || r <= 0) {
+        *kern = h->lnccKernD.p + (h->lnccKernD.n - 1);
+        return 0;
+    }
+    *kern = h->lnccKernD.p + h->lnccKernOff[axis];
+    return r;
+}
+
+// The tiled passes hold lines with up to kEvalRadius voxels on each side.
+bool eval_tiled(const nrh_f3d *h) {
+    return h->lnccRadius[0] <= kEvalRadius && h->lnccRadius[1] <= kEvalRadius && h->lnccRadius[2] <= kEvalRadius;
+}
+
+// x then y pass of `arrays` planar arrays: in (null: the six numerators of the images) -> mid -> out.
+void eval_xy(nrh_f3d *h, const float *in, float *mid, float *out, int arrays) {
+    const int nx = h->ref.nx, ny = h->ref.ny, nz = h->ref.nz, nrows = ny * nz;
+    const double *kern;
+    int r = eval_axis(h, 0, &kern);
+    const dim3 rows((nrows + kEvalRows - 1) / kEvalRows, (nx + 63) / 64, in ? arrays : 1);
+    if (in)
+        hipLaunchKernelGGL(k_eval_x<false>, rows, dim3(kB), eval_lds_rows(r), h->stream, nullptr, nullptr, nullptr, in, mid,
+                           nullptr, h->N, nx, nrows, kern, r);
+    else
+        hipLaunchKernelGGL(k_eval_x<true>, rows, dim3(kB), eval_lds_rows(r), h->stream, ref_ptr(h), h->warped.p, h->mask.p,
+                           nullptr, mid, h->lnccComb.p, h->N, nx, nrows, kern, r);
+    NRH_HIP(hipGetLastError());
+    r = eval_axis(h, 1, &kern);
+    const Columns c{ (size_t)nx * nz, (size_t)nx * ny, (size_t)nx, nx, ny };
+    hipLaunchKernelGGL(k_eval_cols, column_grid(c, arrays), dim3(kB), eval_lds_cols(r), h->stream, mid, out, h->N, c, kern,
+                       r);
+    NRH_HIP(hipGetLastError());
+}
+
 }  // namespace
+
+void op_lncc_eval(nrh_f3d *h) {
+    NRH_REQUIRE(!h->warped.empty(), NRH_ERR_STATE, "LNCC needs the warped image");
+    ensure_lncc(h);
+    if (eval_tiled(h)) eval_xy(h, nullptr, h->lnccA.p, h->lnccB.p, 6);  // in lnccB for the z pass
+}
+
+void op_lncc_eval_value(nrh_f3d *h, double *out_device) {
+    if (!eval_tiled(h)) {
+        const uint64_t keep = h->evalVersion;  // the warped image stays
+        op_lncc_value(h, out_device);
+        h->evalVersion = keep;
+        return;
+    }
+    const double *kern;
+    const int r = eval_axis(h, 2, &kern);
+    const Columns c = z_columns(h);
+    const dim3 grid = column_grid(c, 1);
+    const int nb = (int)eval_blocks(h);
+    double *ps = h->lnccPart.p;
+    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p + nb);
+    hipLaunchKernelGGL(k_eval_stats<false>, grid, dim3(kB), eval_lds_cols(r), h->stream, h->lnccB.p, h->lnccComb.p, h->N, c,
+                       kern, r, nullptr, ps, pc);
+    NRH_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_eval_finish, dim3(1), dim3(1024), 0, h->stream, ps, pc, nb, 0, 0.0, out_device);
+    NRH_HIP(hipGetLastError());
+}
+
+void op_lncc_eval_voxel_gradient(nrh_f3d *h, double weight) {
+    h->evalVersion = 0;  // the sums are used up
+    if (!eval_tiled(h)) {
+        zero_voxel_gradient(h);
+        op_lncc_voxel_gradient(h, weight);
+        return;
+    }
+    ensure_voxel_grad(h);
+    h->voxelGradPending = false;
+    NRH_REQUIRE(!h->warpedGrad.empty(), NRH_ERR_STATE, "LNCC gradient needs the warped image gradient");
+    const double *kern;
+    const int r = eval_axis(h, 2, &kern);
+    const Columns c = z_columns(h);
+    const dim3 grid = column_grid(c, 1);
+    const int nb = (int)eval_blocks(h);
+    double *ps = h->lnccPart.p;
+    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p + nb);
+    float *T = h->lnccA.p, *dens = h->lnccA.p + 3 * h->N;
+    hipLaunchKernelGGL(k_eval_stats<true>, grid, dim3(kB), eval_lds_cols(r), h->stream, h->lnccB.p, h->lnccComb.p, h->N, c,
+                       kern, r, T, ps, pc);
+    NRH_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_eval_finish, dim3(1), dim3(1024), 0, h->stream, ps, pc, nb, 1, weight, h->lnccScalars.p);
+    NRH_HIP(hipGetLastError());
+    // the six sums are done with: their buffer takes the terms' x and y passes
+    eval_xy(h, T, h->lnccB.p, h->lnccB.p + 3 * h->N, 3);
+    hipLaunchKernelGGL(k_eval_apply, grid, dim3(kB), eval_lds_cols(r), h->stream, h->lnccB.p + 3 * h->N, h->lnccComb.p,
+                       dens, h->N, c, kern, r, ref_ptr(h), h->warped.p, h->warpedGrad.p, h->lnccScalars.p,
+                       h->voxelGrad.p);
+    NRH_HIP(hipGetLastError());
+}
 
 void op_lncc_value(nrh_f3d *h, double *out_device) {
     const float *C = lncc_statistics(h);

@@ -1,0 +1,74 @@
+"""The LNCC evaluation's passes against the per-operation measure.
+
+objective / gradient convolve with fused multiply-adds and warp with the fused sweep where the grid
+allows it; the per-operation calls round every product to float as the reference does.  Bounds: a
+product rounded to float is off by 2^-24, so a convolved sum of positive terms by at most 6e-8 an
+axis, and a local variance by that times mean^2 / variance, up to about 2.5e3 on these images
+(noise 0.01 on intensities in [0, 1]): 5e-4 at single voxels.  The mean value is far closer (1e-5
+allowed), the gradient's L2 error is bounded by 1e-3.  Kernels too long for the tiled passes take
+the per-operation ones: on a grid off the voxels the results are then equal.
+"""
+import numpy as np
+import pytest
+
+from niftyreg_amd import _lib, phantoms
+from niftyreg_amd.f3d import F3dContent, default_params
+from niftyreg_amd.geometry import Geom, create_control_point_grid
+
+pytestmark = pytest.mark.gpu
+
+
+def _chain(h, cpp, weight):
+    h.set_control_points(cpp)
+    h.GetDeformationField()
+    h.ResampleImage()
+    value = h.GetLnccValue()
+    h.GetImageGradient()
+    h.ZeroVoxelBasedMeasureGradient()
+    h.GetVoxelBasedLnccGradient(1.0)
+    voxel = h.voxel_gradient()
+    h.ConvolveImage()
+    h.VoxelCentricToNodeCentric(weight)
+    h.ApproxBendingEnergyGradient(1.0 - weight)
+    return value, voxel, h.node_gradient()
+
+
+@pytest.mark.parametrize("dims,spacing,sigma,masked,nans,voxel", [
+    ((64, 32, 32), 5.0, -5.0, False, False, (1, 1, 1)),       # whole tiles
+    ((65, 33, 41), 5.0, -5.0, True, False, (1, 1, 1)),        # one past them, masked
+    ((23, 70, 12), 4.0, -5.0, False, True, (1, 1, 1)),        # lines shorter than the kernel, NaN voxels
+    ((40, 36, 34), 5.0, 4.5, False, False, (1.0, 1.2, 20.0)), # no smoothing along z (radius 0)
+    ((41, 37, 35), 5.0, -10.0, False, False, (1, 1, 1)),      # the longest tiled kernel (radius 30)
+    ((41, 37, 35), 5.0, -1.0, False, False, (1, 1, 1)),       # fewer taps than a chunk
+    ((36, 34, 30), 4.6, -3.0, True, True, (1, 1, 1)),         # nodes off the voxels
+    ((36, 34, 30), 4.6, -11.0, False, False, (1, 1, 1)),      # and too long a kernel
+])
+def test_evaluation_matches_per_operation_measure(gpu, dims, spacing, sigma, masked, nans, voxel):
+    g = Geom.identity(dims, spacing=voxel)
+    rng = np.random.default_rng(sum(dims))
+    ref = phantoms.blob_phantom(dims, 1).ravel()
+    flo = phantoms.blob_phantom(dims, 2).ravel()
+    if nans:
+        ref[rng.integers(0, ref.size, 20)] = np.nan
+        flo[rng.integers(0, flo.size, 20)] = np.nan
+    cg, cpp = create_control_point_grid(g, [spacing * p for p in g.pixdim])
+    cpp = (cpp + rng.uniform(-1, 1, cpp.size)).astype(np.float32)
+    mask = (rng.uniform(size=g.nvox) > 0.2).astype(np.int32) - 1 if masked else None
+    p = default_params(similarity_weight=0.99, be_weight=0.01, measure=_lib.MEASURE_LNCC, lncc_sigma=sigma)
+    h = F3dContent(g, ref, g, flo, cg, cpp, mask=mask, params=p)
+    h.rescale_intensities((0, 1), (0, 1))
+    value, terms = h.objective()
+    h.gradient()
+    got, vox = h.node_gradient(), h.voxel_gradient()
+    h.set_control_points(cpp)
+    h.gradient()  # without the objective: the same gradient
+    assert np.array_equal(got, h.node_gradient())
+    want_value, want_voxel, want = _chain(h, cpp, 0.99)
+    h.close()
+    exact = sigma == -11.0
+    assert abs(terms[0] / np.float32(0.99) - want_value) <= (1e-12 if exact else 1e-5) * abs(want_value)
+    assert np.isfinite(got).all() and np.isfinite(vox).all() and np.abs(want).max() > 0
+    if exact:
+        assert np.array_equal(got, want)
+    else:
+        assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
