@@ -41,10 +41,11 @@ namespace nrh {
 
 namespace {
 
-constexpr int TX = 64, TY = 8, TZ = 8;
+constexpr int TX = 64, TY = 8;  // a tile is 64 x 8 x depth voxels (tile_depth)
+constexpr int kMaxDepth = 8;
 constexpr int WXM = 20, WYM = 6, WZM = 6;  // node-window bounds for spacing >= 4 voxels
 constexpr int kThreads = 256;
-constexpr int kTileVoxels = TX * TY * TZ;
+constexpr int kSliceVoxels = TX * TY;
 
 struct FusedArgs {
     const void *ref;
@@ -61,6 +62,7 @@ struct FusedArgs {
     const int *preX, *preY, *preZ;
     const float4 *bX, *bY, *bZ;
     int tilesX, tilesY, tilesZ, numTiles;
+    int tileVoxels;  // slots of a tile's list: 64 x 8 x depth
     Affine cppXyz;  // grid voxel -> mm
     uint32_t *hist;
     const double *ent;
@@ -70,7 +72,7 @@ struct FusedArgs {
                       // histogram sweep, for checking
     float *warpOut;   // warp sweep: the warped image
     // voxels left to the exact pass: positions within ambTol (floating voxels) of a voxel plane;
-    // tile t lists its voxels in ambList[t * kTileVoxels ..] and their number in ambCounts[t]
+    // tile t lists its voxels in ambList[t * tileVoxels ..] and their number in ambCounts[t]
     uint32_t *ambList;
     uint32_t *ambCounts;
     float ambTol;
@@ -429,7 +431,7 @@ __device__ __forceinline__ void fixup_tiles(const FusedArgs& a, const int t0, co
     for (uint32_t i = tid; i < total; i += blockDim.x) {
         int k = 0;
         while (i >= sOff[k + 1]) ++k;
-        const uint32_t idx = a.ambList[(size_t)(t0 + k) * kTileVoxels + (i - sOff[k])];
+        const uint32_t idx = a.ambList[(size_t)(t0 + k) * a.tileVoxels + (i - sOff[k])];
         fixup_voxel<TImg, MODE>(a, idx, h);
     }
     if (MODE == kSweepHist) {
@@ -483,10 +485,11 @@ k_sweep_fixup_batch(const FusedArgs *__restrict__ A, const int4 *__restrict__ ch
     fixup_tiles<TImg, MODE>(A[c.x], c.y, c.z, fixLds);
 }
 
-// A 64 x 8 x 8 tile per workgroup.  The control-point window is staged in LDS and contracted
+// A 64 x 8 x TZ tile per workgroup.  The control-point window is staged in LDS and contracted
 // along z and y for every (z, y) row of the tile in one pass; the voxels then run without
 // barriers (one wave per x row), which keeps many floating-image gathers in flight.  The window
 // shares LDS with the histogram / NMI table, which are filled after the contraction.
+template<int TZ>
 struct SweepShared {
     float sAyz[TZ][TY][WXM][3];
     double sIdYZ[TZ][TY][3];  // identity terms of each row: m[c][1] uy + m[c][2] uz + m[c][3]
@@ -497,8 +500,8 @@ struct SweepShared {
 
 // One tile t of the pair described by a; dyn: the dynamic LDS (window [3][WZM][WYM][WXM], then
 // the histogram or the table K).  Called by every thread of the workgroup.
-template<class TImg, int MODE>
-__device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, SweepShared& S, float *dyn) {
+template<class TImg, int MODE, int TZ>
+__device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, SweepShared<TZ>& S, float *dyn) {
     auto& sAyz = S.sAyz;
     auto& sIdYZ = S.sIdYZ;
     auto& sBx = S.sBx;
@@ -509,7 +512,7 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
     auto& sPz = S.sPz;
     const int tid = threadIdx.x;
     if (tid == 0) S.ambCount = 0u;  // read after the tile's barriers
-    uint32_t *ambList = a.ambList + (size_t)t * kTileVoxels;
+    uint32_t *ambList = a.ambList + (size_t)t * (kSliceVoxels * TZ);
     const int tx = t % a.tilesX, ty = (t / a.tilesX) % a.tilesY, tz = t / (a.tilesX * a.tilesY);
     const int x0 = tx * TX, y0 = ty * TY, z0 = tz * TZ;
     const int nX = min(TX, a.nx - x0), nY = min(TY, a.ny - y0), nZ = min(TZ, a.nz - z0);
@@ -681,13 +684,13 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
     }
 }
 
-template<class TImg, int MODE>
+template<class TImg, int MODE, int TZ>
 __global__ void __launch_bounds__(kThreads) k_sweep(FusedArgs a) {
-    __shared__ SweepShared S;
+    __shared__ SweepShared<TZ> S;
     extern __shared__ __align__(16) float dyn[];
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     if (t >= a.numTiles) return;
-    sweep_tile<TImg, MODE>(a, t, S, dyn);
+    sweep_tile<TImg, MODE, TZ>(a, t, S, dyn);
 }
 
 // Persistent sweep over the (pair, tile) work list of a batch of pairs: item = pair << 20 | tile,
@@ -699,7 +702,7 @@ template<class TImg, int MODE>
 __global__ void __launch_bounds__(kThreads)
 k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ items, int nItems,
               const int *__restrict__ active) {
-    __shared__ SweepShared S;
+    __shared__ SweepShared<kMaxDepth> S;
     extern __shared__ __align__(16) float dyn[];
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, perXcd = gridDim.x / 8;
     const int per = (nItems + 7) / 8;
@@ -708,7 +711,7 @@ k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ i
         const uint32_t it = __builtin_amdgcn_readfirstlane(items[i]);  // uniform: scalar loads of the arguments
         const int pair = (int)(it >> 20);
         if (active && !active[pair]) continue;  // uniform over the workgroup
-        sweep_tile<TImg, MODE>(args[pair], (int)(it & 0xfffffu), S, dyn);
+        sweep_tile<TImg, MODE, kMaxDepth>(args[pair], (int)(it & 0xfffffu), S, dyn);
         __syncthreads();  // the next tile reuses the LDS
     }
 }
@@ -1015,7 +1018,8 @@ __global__ void k_to_half(const float *in, __half *out, size_t n) {
 // Device tables of the fused path, built once per handle.
 struct FusedPlan {
     bool ok = false;
-    int tilesX = 0, tilesY = 0, tilesZ = 0, numTiles = 0;
+    int tilesX = 0, tilesY = 0, nz = 0;
+    int depth = kMaxDepth;  // of the pair's own sweeps; a batch's tiles are kMaxDepth deep
     DevBuf<int> preX, preY, preZ;
     DevBuf<float4> bX, bY, bZ;
     DevBuf<int2> rX, rY, rZ;     // voxels [first, last] in the support of each node, per axis
@@ -1024,11 +1028,24 @@ struct FusedPlan {
     DevBuf<float> invNx, invNy, invNz;
     DevBuf<float> gvox, projX, projY;  // voxel gradient [3][N]; after the x pass; after the y pass
     DevBuf<float> kTab;                // NMI derivative table, rb * fb rounded up to 4 floats
-    DevBuf<uint32_t> ambList;          // voxels left to the exact pass, kTileVoxels slots per tile
+    DevBuf<uint32_t> ambList;          // voxels left to the exact pass, a slot per voxel of a tile
     DevBuf<uint32_t> ambCounts;        // listed voxels per tile
     float ambTol = 0.f;                // floating voxels
     bool lut = false;
+    int tiles(int d) const { return tilesX * tilesY * ((nz + d - 1) / d); }
 };
+
+// Depth of a pair's own tiles, from the number of tiles across a slice and of slices.  A tile stages
+// and contracts its window before its voxels run one wave a row, so deep tiles cost least per voxel,
+// but an image of fewer 8-deep tiles than compute units leaves most of the chip idle through a long
+// tile, and one of a few tiles per unit ends in a nearly empty last round.  Histogram / gradient sweep
+// in us at depth 8, 4, 2: 64^3 (64 tiles) 31 / 34, 22 / 23, 18 / 17; 96^3 (288) 35 / 40, 31 / 35,
+// 30 / 31; 128 x 144 x 112 (504) 40 / 44, 36 / 40, 44 / 43; 160^3 (1200) 66 / 75, 59 / 73, 71 / 78;
+// 192^3 (1728) 82 / 97, 82 / 99, 96 / 109; 256 x 256 x 160 (2560) 108 / 131, 110 / 136, 133 / 154.
+static int tile_depth(int across, int nz) {
+    const long deep = (long)across * ((nz + kMaxDepth - 1) / kMaxDepth);
+    return deep <= 256 ? 2 : deep <= 1536 ? 4 : kMaxDepth;
+}
 
 // The plan is kept beside the handle in a side table keyed by handle address.
 static std::map<const nrh_f3d *, FusedPlan *> g_planMap;
@@ -1075,7 +1092,7 @@ static FusedPlan *plan_of(nrh_f3d *h) {
         const bool lut = gv[0] == 5.f && gv[1] == 5.f && gv[2] == 5.f;
         const int dims[3] = { h->ref.nx, h->ref.ny, h->ref.nz };
         const int gdims[3] = { h->cpp.nx, h->cpp.ny, h->cpp.nz };
-        const int tsz[3] = { TX, TY, TZ };
+        const int tsz[3] = { TX, TY, kMaxDepth };
         const int wmax[3] = { WXM, WYM, WZM };
         DevBuf<int> *pre[3] = { &p->preX, &p->preY, &p->preZ };
         DevBuf<float4> *bb[3] = { &p->bX, &p->bY, &p->bZ };
@@ -1149,8 +1166,8 @@ static FusedPlan *plan_of(nrh_f3d *h) {
         }
         p->tilesX = tiles[0];
         p->tilesY = tiles[1];
-        p->tilesZ = tiles[2];
-        p->numTiles = tiles[0] * tiles[1] * tiles[2];
+        p->nz = h->ref.nz;
+        p->depth = tile_depth(tiles[0] * tiles[1], h->ref.nz);
         p->ok = ok;
         p->lut = lut;
         // Tolerance of the exact pass: the reference's float field is within a few float ulps of
@@ -1172,8 +1189,9 @@ static FusedPlan *plan_of(nrh_f3d *h) {
             rowMax = std::max(rowMax, (double)std::fabs(h->flo.ijk[r * 4]) + std::fabs(h->flo.ijk[r * 4 + 1]) +
                                           std::fabs(h->flo.ijk[r * 4 + 2]));
         p->ambTol = (float)(48.0 * std::ldexp(1.0, -24) * (1.25 * M + 8.0) * rowMax);
-        p->ambList.alloc((size_t)p->numTiles * kTileVoxels);
-        p->ambCounts.alloc(p->numTiles);
+        // shallower tiles round less up: the deepest ones have the most slots
+        p->ambList.alloc((size_t)p->tiles(kMaxDepth) * kSliceVoxels * kMaxDepth);
+        p->ambCounts.alloc(p->tiles(p->depth));
         NRH_HIP(hipStreamSynchronize(h->stream));
     }
     std::lock_guard<std::mutex> lk(g_planMutex);
@@ -1201,6 +1219,12 @@ void collect_sweep_times(nrh_f3d *h) {
         h->nSweep[k] += 1;
         h->evPending[k] = false;
     }
+}
+
+static void set_depth(FusedArgs& a, const FusedPlan *p, int depth) {
+    a.tilesZ = (p->nz + depth - 1) / depth;
+    a.numTiles = p->tiles(depth);
+    a.tileVoxels = kSliceVoxels * depth;
 }
 
 static FusedArgs make_args(nrh_f3d *h, FusedPlan *p) {
@@ -1233,8 +1257,8 @@ static FusedArgs make_args(nrh_f3d *h, FusedPlan *p) {
     a.G = h->G;
     a.preX = p->preX.p; a.preY = p->preY.p; a.preZ = p->preZ.p;
     a.bX = p->bX.p; a.bY = p->bY.p; a.bZ = p->bZ.p;
-    a.tilesX = p->tilesX; a.tilesY = p->tilesY; a.tilesZ = p->tilesZ;
-    a.numTiles = p->numTiles;
+    a.tilesX = p->tilesX; a.tilesY = p->tilesY;
+    set_depth(a, p, p->depth);
     a.ambList = p->ambList.p;
     a.ambCounts = p->ambCounts.p;
     a.ambTol = p->ambTol;
@@ -1249,11 +1273,22 @@ static FusedArgs make_args(nrh_f3d *h, FusedPlan *p) {
 
 static unsigned grid_for(int numTiles) { return (unsigned)((numTiles + 7) / 8 * 8); }
 
+// One sweep of a pair in tiles of its plan's depth.
+template<class TImg, int MODE>
+static void launch_sweep(const FusedArgs& a, int depth, size_t lds, hipStream_t s) {
+    const dim3 grid(grid_for(a.numTiles)), block(kThreads);
+    if (depth == 2) hipLaunchKernelGGL((k_sweep<TImg, MODE, 2>), grid, block, lds, s, a);
+    else if (depth == 4) hipLaunchKernelGGL((k_sweep<TImg, MODE, 4>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((k_sweep<TImg, MODE, kMaxDepth>), grid, block, lds, s, a);
+    NRH_HIP(hipGetLastError());
+}
+
 // Dynamic LDS of a sweep: the control-point window and its z contraction, then the histogram / NMI
 // table in their place.
-static size_t sweep_lds(const FusedArgs& a) {
-    // window [3][WZM][WYM][WXM] + its z contraction [3][TZ][WYM][WXM]; then histogram / table K
-    return std::max<size_t>(((size_t)a.rb * a.fb + 3) / 4 * 4, (size_t)3 * (WZM + TZ) * WYM * WXM) * sizeof(float);
+static size_t window_lds(int depth) { return (size_t)3 * (WZM + depth) * WYM * WXM * sizeof(float); }
+static size_t sweep_lds(const FusedArgs& a, int depth) {
+    // window [3][WZM][WYM][WXM] + its z contraction [3][depth][WYM][WXM]; then histogram / table K
+    return std::max<size_t>(((size_t)a.rb * a.fb + 3) / 4 * 4 * sizeof(float), window_lds(depth));
 }
 
 void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pubS1, int pubN1) {
@@ -1263,19 +1298,16 @@ void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pu
     a.hist = h->histCount.p;
     a.fieldOut = fieldOut;
     // histCount is zero here: allocation zeroes it and every finalisation consumes it
-    const size_t lds = sweep_lds(a);
+    const size_t lds = sweep_lds(a, p->depth);
     const bool timed = h->profile && h->profileSeen[0]++ % h->profilePeriod == 0;
     if (timed) NRH_HIP(hipEventRecord(h->ev[0], h->stream));
-    if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep<__half, kSweepHist>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
-    else
-        hipLaunchKernelGGL((k_sweep<float, kSweepHist>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
-    NRH_HIP(hipGetLastError());
+    if (h->params.image_storage == 1) launch_sweep<__half, kSweepHist>(a, p->depth, lds, h->stream);
+    else launch_sweep<float, kSweepHist>(a, p->depth, lds, h->stream);
     if (timed) {
         NRH_HIP(hipEventRecord(h->ev[1], h->stream));
         h->evPending[0] = true;
     }
-    const unsigned fixBlocks = (unsigned)((p->numTiles + kFixChunk - 1) / kFixChunk);
+    const unsigned fixBlocks = (unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk);
     const size_t fixLds = (size_t)a.rb * a.fb * sizeof(uint32_t);
     if (beValue) {
         BeValueArgs be;
@@ -1326,10 +1358,8 @@ void fused_warp(nrh_f3d *h) {
     a.flo = h->floImg.p;
     a.fieldOut = h->field.p;
     a.warpOut = h->warped.p;
-    const size_t lds = (size_t)3 * (WZM + TZ) * WYM * WXM * sizeof(float);
-    hipLaunchKernelGGL((k_sweep<float, kSweepWarp>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
-    NRH_HIP(hipGetLastError());
-    hipLaunchKernelGGL((k_sweep_fixup<float, kSweepWarp>), dim3((unsigned)((p->numTiles + kFixChunk - 1) / kFixChunk)),
+    launch_sweep<float, kSweepWarp>(a, p->depth, window_lds(p->depth), h->stream);
+    hipLaunchKernelGGL((k_sweep_fixup<float, kSweepWarp>), dim3((unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk)),
                        dim3(256), 0, h->stream, a);
     NRH_HIP(hipGetLastError());
 }
@@ -1426,19 +1456,16 @@ void fused_gradient(nrh_f3d *h, float weight, float beWeight, uint32_t *maxBits)
         hipLaunchKernelGGL(k_nmi_table, dim3((nbins + 255) / 256), dim3(256), 0, h->stream, h->histLog.p, a.ent, a.rb,
                            a.fb, p->kTab.p);
     a.kTab = p->kTab.p;
-    const size_t lds = sweep_lds(a);
+    const size_t lds = sweep_lds(a, p->depth);
     const bool timed = h->profile && h->profileSeen[1]++ % h->profilePeriod == 0;
     if (timed) NRH_HIP(hipEventRecord(h->ev[2], h->stream));
-    if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep<__half, kSweepGrad>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
-    else
-        hipLaunchKernelGGL((k_sweep<float, kSweepGrad>), dim3(grid_for(p->numTiles)), dim3(kThreads), lds, h->stream, a);
-    NRH_HIP(hipGetLastError());
+    if (h->params.image_storage == 1) launch_sweep<__half, kSweepGrad>(a, p->depth, lds, h->stream);
+    else launch_sweep<float, kSweepGrad>(a, p->depth, lds, h->stream);
     if (timed) {
         NRH_HIP(hipEventRecord(h->ev[3], h->stream));
         h->evPending[1] = true;
     }
-    const dim3 fixGrid((unsigned)((p->numTiles + kFixChunk - 1) / kFixChunk));
+    const dim3 fixGrid((unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk));
     if (h->params.image_storage == 1)
         hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepGrad>), fixGrid, dim3(256), 0, h->stream, a);
     else
@@ -1475,8 +1502,10 @@ void batch_fused_setup(nrh_batch *b) {
                     "batched pairs need the fused path (integer grid spacing >= 4 voxels, nodes on voxels)");
         NRH_REQUIRE(h->params.image_storage == storage, NRH_ERR_ARG, "batched pairs share one image storage type");
         FusedPlan *p = plan_of(h);
-        NRH_REQUIRE(p->numTiles < (1 << 20) && b->P < 4096, NRH_ERR_UNSUPPORTED, "batch too large for the work list");
+        const int numTiles = p->tiles(kMaxDepth);
+        NRH_REQUIRE(numTiles < (1 << 20) && b->P < 4096, NRH_ERR_UNSUPPORTED, "batch too large for the work list");
         FusedArgs a = make_args(h, p);
+        set_depth(a, p, kMaxDepth);
         a.hist = h->histCount.p;
         p->gvox.alloc(3 * h->N);
         a.gvox = p->gvox.p;
@@ -1484,10 +1513,10 @@ void batch_fused_setup(nrh_batch *b) {
         p->kTab.alloc((size_t)(nbins + 3) / 4 * 4);
         a.kTab = p->kTab.p;
         args[q] = a;
-        b->sweepLds = std::max(b->sweepLds, sweep_lds(a));
-        for (int t = 0; t < p->numTiles; ++t) items.push_back(((uint32_t)q << 20) | (uint32_t)t);
-        for (int t = 0; t < p->numTiles; t += kFixChunk)
-            fixChunks.push_back(make_int4(q, t, std::min(kFixChunk, p->numTiles - t), 0));
+        b->sweepLds = std::max(b->sweepLds, sweep_lds(a, kMaxDepth));
+        for (int t = 0; t < numTiles; ++t) items.push_back(((uint32_t)q << 20) | (uint32_t)t);
+        for (int t = 0; t < numTiles; t += kFixChunk)
+            fixChunks.push_back(make_int4(q, t, std::min(kFixChunk, numTiles - t), 0));
         b->fixLds = std::max(b->fixLds, (size_t)nbins * sizeof(uint32_t));
         size_t ldsX = 0;
         projection_args(h, p, p->gvox.p, h->params.similarity_weight, pxs[q], pys[q], nds[q], &ldsX);
