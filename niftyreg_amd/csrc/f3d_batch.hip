@@ -121,11 +121,11 @@ void batch_objective(nrh_batch *b, const int *active) {
     batch_values(b, active);
 }
 
-// nrh_f3d_gradient(h, &max_length) for every active pair: the histogram at the current points,
-// the similarity gradient, the bending-energy gradient (with the displacement round trip of the
-// points) and the normalisation by the max length.
-void batch_gradient(nrh_batch *b, const int *active, bool normalise) {
-    batch_histogram(b, active);
+// nrh_f3d_gradient(h, &max_length) for every active pair: the histogram at the current points
+// (unless they are those of the last objective), the similarity gradient, the bending-energy
+// gradient (with the displacement round trip of the points) and the normalisation by the max length.
+void batch_gradient(nrh_batch *b, const int *active, bool normalise, bool histogram) {
+    if (histogram) batch_histogram(b, active);
     batch_similarity_gradient(b, active);
     batch_be_gradient(b, active);
     if (normalise) batch_normalise(b, active);
@@ -162,7 +162,7 @@ void batch_ls_iteration(nrh_batch *b) {
     int *active = b->lsFlags.p, *first = active + b->P, *searching = first + b->P, *store = searching + b->P;
     hipLaunchKernelGGL(k_ls_begin, dim3(g), dim3(64), 0, b->stream, b->lsState.p, b->P, active, first, searching,
                        b->lsScales.p);
-    batch_gradient(b, active, true);
+    batch_gradient(b, active, true, true);
     batch_cg(b, active, first);
     for (int step = 0; step < 12; ++step) {
         batch_update(b, searching, b->lsScales.p);
@@ -189,6 +189,7 @@ void batch_touch(nrh_batch *b, bool pointsChanged) {
         }
         h->kTabCurrent = false;  // the batch's finalisation leaves the pair's own table as it was
         h->touch();
+        if (!pointsChanged) h->batchVersion = h->cppVersion;
         h->velFieldVersion = 0;
     }
 }
@@ -301,7 +302,10 @@ int nrh_batch_objective(nrh_batch *b, double *values, double *nmi) {
 int nrh_batch_gradient(nrh_batch *b, double *max_lengths) {
     return guard([&] {
         NRH_REQUIRE(b, NRH_ERR_ARG, "null batch");
-        batch_gradient(b, nullptr, max_lengths != nullptr);
+        // every pair's histogram is that of its points after an objective there, as for one pair
+        const bool stale = std::any_of(b->pairs.begin(), b->pairs.end(),
+                                       [](const nrh_f3d *h) { return h->batchVersion != h->cppVersion; });
+        batch_gradient(b, nullptr, max_lengths != nullptr, stale);
         NRH_HIP(hipStreamSynchronize(b->stream));
         batch_touch(b, true);
         if (max_lengths)

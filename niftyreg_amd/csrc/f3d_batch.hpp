@@ -79,7 +79,7 @@ void batch_values(nrh_batch *b, const int *active);             // results[] of 
 nrh_batch *batch_new(nrh_f3d *const *pairs, int n);
 void batch_free(nrh_batch *b);
 void batch_objective(nrh_batch *b, const int *active);
-void batch_gradient(nrh_batch *b, const int *active, bool normalise);
+void batch_gradient(nrh_batch *b, const int *active, bool normalise, bool histogram);
 void batch_touch(nrh_batch *b, bool pointsChanged);
 void batch_autotune(nrh_batch *b);
 void batch_ls_alloc(nrh_batch *b);

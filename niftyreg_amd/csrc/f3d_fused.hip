@@ -501,7 +501,7 @@ struct SweepShared {
 // One tile t of the pair described by a; dyn: the dynamic LDS (window [3][WZM][WYM][WXM], then
 // the histogram or the table K).  Called by every thread of the workgroup.
 template<class TImg, int MODE, int TZ>
-__device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, SweepShared<TZ>& S, float *dyn) {
+__device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, const int tid, SweepShared<TZ>& S, float *dyn) {
     auto& sAyz = S.sAyz;
     auto& sIdYZ = S.sIdYZ;
     auto& sBx = S.sBx;
@@ -510,7 +510,6 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
     auto& sPx = S.sPx;
     auto& sPy = S.sPy;
     auto& sPz = S.sPz;
-    const int tid = threadIdx.x;
     if (tid == 0) S.ambCount = 0u;  // read after the tile's barriers
     uint32_t *ambList = a.ambList + (size_t)t * (kSliceVoxels * TZ);
     const int tx = t % a.tilesX, ty = (t / a.tilesX) % a.tilesY, tz = t / (a.tilesX * a.tilesY);
@@ -603,14 +602,13 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, Swee
         float4 *dst4 = (float4 *)dyn;
         for (int base = 0; base < n4; base += 4 * kThreads) {
             // unconditional loads (clamped index) keep v in registers with all four in flight
-            float4 v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = src[min(base + u * kThreads + tid, n4 - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = base + u * kThreads + tid;
-                if (i < n4) dst4[i] = v[u];
-            }
+            const int i0 = base + tid, i1 = i0 + kThreads, i2 = i1 + kThreads, i3 = i2 + kThreads;
+            const float4 v0 = src[min(i0, n4 - 1)], v1 = src[min(i1, n4 - 1)], v2 = src[min(i2, n4 - 1)],
+                         v3 = src[min(i3, n4 - 1)];
+            if (i0 < n4) dst4[i0] = v0;
+            if (i1 < n4) dst4[i1] = v1;
+            if (i2 < n4) dst4[i2] = v2;
+            if (i3 < n4) dst4[i3] = v3;
         }
         coef = 1.0 / (a.ent[2] * a.ent[3]);
     } else if (MODE == kSweepHist) {
@@ -690,7 +688,7 @@ __global__ void __launch_bounds__(kThreads) k_sweep(FusedArgs a) {
     extern __shared__ __align__(16) float dyn[];
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     if (t >= a.numTiles) return;
-    sweep_tile<TImg, MODE, TZ>(a, t, S, dyn);
+    sweep_tile<TImg, MODE, TZ>(a, t, (int)threadIdx.x, S, dyn);
 }
 
 // Persistent sweep over the (pair, tile) work list of a batch of pairs: item = pair << 20 | tile,
@@ -699,7 +697,7 @@ __global__ void __launch_bounds__(kThreads) k_sweep(FusedArgs a) {
 // workgroups of an XCD take the items of its range in turn.  Items of pairs whose flag in
 // `active` is 0 are skipped (a line search that has ended for that pair).
 template<class TImg, int MODE>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 4)
 k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ items, int nItems,
               const int *__restrict__ active) {
     __shared__ SweepShared<kMaxDepth> S;
@@ -711,7 +709,9 @@ k_sweep_batch(const FusedArgs *__restrict__ args, const uint32_t *__restrict__ i
         const uint32_t it = __builtin_amdgcn_readfirstlane(items[i]);  // uniform: scalar loads of the arguments
         const int pair = (int)(it >> 20);
         if (active && !active[pair]) continue;  // uniform over the workgroup
-        sweep_tile<TImg, MODE, kMaxDepth>(args[pair], (int)(it & 0xfffffu), S, dyn);
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // opaque: nothing of a tile is hoisted out of the loop
+        sweep_tile<TImg, MODE, kMaxDepth>(args[pair], (int)(it & 0xfffffu), tid, S, dyn);
         __syncthreads();  // the next tile reuses the LDS
     }
 }

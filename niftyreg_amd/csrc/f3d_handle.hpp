@@ -92,7 +92,9 @@ struct nrh_f3d {
     // histogram's logs on the per-operation chain, the convolved LNCC sums) for a gradient at the
     // same points (0: some other operation changed them since)
     uint64_t evalVersion = 0;
-    void touch() { pairStateVersion = evalVersion = 0; }
+    // cppVersion at which a batch's objective left the histogram's logs and entropies (0: as above)
+    uint64_t batchVersion = 0;
+    void touch() { pairStateVersion = evalVersion = batchVersion = 0; }
     // affine components of a velocity grid: its NIfTI extensions 0 (applied before the spline,
     // removed before the squaring and restored after it) and 1 (composed after it), and the
     // content's transformation matrix (removed from the opposite direction's intermediate fields)
