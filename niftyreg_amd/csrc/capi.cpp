@@ -160,7 +160,7 @@ static nrh_f3d *f3d_finish(std::unique_ptr<nrh_f3d> h, const int *mask) {
     h->ent.alloc(8);
     h->scalars.alloc(16);
     h->maxBits.alloc(8);
-    NRH_HIP(hipMemsetAsync(h->maxBits.p, 0, h->maxBits.bytes(), h->stream));  // [6]: BE reduction ticket
+    NRH_HIP(hipMemsetAsync(h->maxBits.p, 0, h->maxBits.bytes(), h->stream));  // [7]: LE reduction ticket
     h->partials.alloc(4096);
     NRH_HIP(hipStreamSynchronize(h->stream));
     return h.release();
@@ -253,10 +253,6 @@ int nrh_f3d_destroy(nrh_f3d *h) {
         for (int i = 0; i < 4; ++i)
             if (h->ev[i]) (void)hipEventDestroy(h->ev[i]);
         if (h->evPair) (void)hipEventDestroy(h->evPair);
-        if (h->side) (void)hipStreamSynchronize(h->side);
-        if (h->evFork) (void)hipEventDestroy(h->evFork);
-        if (h->evJoin) (void)hipEventDestroy(h->evJoin);
-        if (h->side) (void)hipStreamDestroy(h->side);
         hipStream_t s = h->stream;
         delete h;
         if (s) (void)hipStreamDestroy(s);

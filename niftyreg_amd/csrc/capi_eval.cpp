@@ -159,10 +159,9 @@ static void gradient_body(nrh_f3d *h, double *max_length) {
             lncc_gradient(h, p.similarity_weight);
         } else if (p.similarity_weight > 0) {
             if (fused_supported(h)) {
-                // the bending-energy gradient sums run on the side stream beside the projection
-                // passes; the node projection adds them
+                // the bending-energy gradient sums run in the exact pass's launch, which also clears
+                // maxBits; the node projection adds them
                 const bool trackMax = be && max_length != nullptr && !le;
-                if (trackMax) op_fill_u32(h->maxBits.p, 1, 0u, h->stream);
                 if (h->histVersion != h->cppVersion) fused_histogram(h);
                 fused_gradient(h, p.similarity_weight, be ? p.be_weight : 0.f, trackMax ? h->maxBits.p : nullptr);
                 beDone = be;

@@ -118,7 +118,7 @@ __global__ void k_ls_end(LsState *__restrict__ st, int n, const int *__restrict_
 void batch_objective(nrh_batch *b, const int *active) {
     batch_histogram(b, active);
     batch_be_value(b, active);
-    batch_values(b, active);
+    batch_values(b, active, true);
 }
 
 // nrh_f3d_gradient(h, &max_length) for every active pair: the histogram at the current points
@@ -126,10 +126,10 @@ void batch_objective(nrh_batch *b, const int *active) {
 // gradient (with the displacement round trip of the points) and the normalisation by the max length.
 void batch_gradient(nrh_batch *b, const int *active, bool normalise, bool histogram) {
     if (histogram) batch_histogram(b, active);
-    batch_similarity_gradient(b, active);
     batch_be_gradient(b, active);
+    batch_similarity_gradient(b, active);  // its node projection adds the bending-energy gradient
     if (normalise) batch_normalise(b, active);
-    batch_values(b, active);
+    batch_values(b, active, false);
 }
 
 void batch_ls_alloc(nrh_batch *b) {

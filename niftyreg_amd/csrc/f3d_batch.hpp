@@ -63,18 +63,20 @@ constexpr int kBatchResults = 8;
 // f3d_fused.hip
 void batch_fused_setup(nrh_batch *b);
 void batch_histogram(nrh_batch *b, const int *active);          // sweep + exact pass + finalize
-void batch_similarity_gradient(nrh_batch *b, const int *active);  // K table, sweep, exact pass, projections
+// K table, sweep, exact pass, projections; then the node gradient with the bending-energy one added,
+// the points' round trip and the max length
+void batch_similarity_gradient(nrh_batch *b, const int *active);
 void batch_set_sweep_blocks(nrh_batch *b, int blocksPerXcd);
 // f3d_ops.hip
 void batch_ops_setup(nrh_batch *b);
 void batch_finalize(nrh_batch *b, const int *active);
 void batch_be_value(nrh_batch *b, const int *active);
-void batch_be_gradient(nrh_batch *b, const int *active);       // with the max length of the result
+void batch_be_gradient(nrh_batch *b, const int *active);       // the sums, and cleared max lengths
 void batch_normalise(nrh_batch *b, const int *active);
 void batch_cg(nrh_batch *b, const int *active, const int *first);
 void batch_update(nrh_batch *b, const int *active, const float *scales);
 void batch_copy_dof(nrh_batch *b, const int *active, bool toBest);
-void batch_values(nrh_batch *b, const int *active);             // results[] of the objective
+void batch_values(nrh_batch *b, const int *active, bool sumBe);             // results[] of the objective
 // f3d_batch.hip
 nrh_batch *batch_new(nrh_f3d *const *pairs, int n);
 void batch_free(nrh_batch *b);

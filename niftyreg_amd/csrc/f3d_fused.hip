@@ -413,13 +413,16 @@ template<class TImg, int MODE>
 __device__ __forceinline__ void fixup_tiles(const FusedArgs& a, const int t0, const int nt, uint32_t *h) {
     __shared__ uint32_t sOff[kFixChunk + 1];
     const int tid = threadIdx.x;
-    if (tid == 0) {
-        uint32_t o = 0;
-        for (int k = 0; k < nt; ++k) {
-            sOff[k] = o;
-            o += a.ambCounts[t0 + k];
+    if (tid < 64) {
+        // the counts loaded together, then their running sums
+        uint32_t o = tid < nt ? a.ambCounts[t0 + tid] : 0u;
+#pragma unroll
+        for (int d = 1; d < kFixChunk; d *= 2) {
+            const uint32_t p = __shfl_up(o, d, 64);
+            if (tid >= d) o += p;
         }
-        for (int k = nt; k <= kFixChunk; ++k) sOff[k] = o;
+        if (tid < kFixChunk) sOff[tid + 1] = o;
+        if (tid == 0) sOff[0] = 0u;
     }
     __syncthreads();
     const uint32_t total = sOff[kFixChunk];
@@ -448,31 +451,38 @@ __global__ void __launch_bounds__(256) k_sweep_fixup(FusedArgs a) {
     fixup_tiles<TImg, MODE>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
 }
 
-// The histogram pass's exact pass with the bending energy in the same launch: workgroups
-// [0, be.nb) evaluate the bending-energy bricks (be_value_block, its result into be.out), the
-// others the exact-pass chunks.  The two are independent (the bricks read only the control
-// points), and both are latency-bound, so one launch overlaps them without a second stream.
-struct BeValueArgs {
+// An exact pass with the bending energy of the same points in the same launch: the last 3 be.nb
+// workgroups take the bricks' components (the histogram pass their energies' partials, the gradient
+// pass the gradient's sums), those before the exact-pass chunks, which take longer each.  The two are
+// independent (the bricks read only the control points), and both are latency-bound, so one launch
+// overlaps them without a second stream.  The gradient pass also clears maxBits for the kernels that follow.
+struct BeArgs {
     const float *cpp;
     int gnx, gny, gnz;
     BrickGrid bg;
-    double *partials;
-    uint32_t *ticket;
-    double scale;
-    double *out;
-    int nb;  // bricks
+    Affine xyz;
+    double *partials;   // histogram pass: [3 nb]
+    float *beGrad;      // gradient pass: [3][G]
+    uint32_t *maxBits;  // gradient pass, optional
+    int nb;             // bricks
 };
 
-template<class TImg>
-__global__ void __launch_bounds__(256) k_sweep_fixup_be(FusedArgs a, BeValueArgs be, BeBasis B) {
+template<class TImg, int MODE>
+__global__ void __launch_bounds__(256) k_sweep_fixup_be(FusedArgs a, BeArgs be) {
     extern __shared__ __align__(16) uint32_t fixLds[];
-    if ((int)blockIdx.x < be.nb) {  // uniform over the workgroup
-        be_value_block(be.cpp, be.gnx, be.gny, be.gnz, be.bg, B, be.partials, be.ticket, be.scale, be.out,
-                       (int)blockIdx.x, be.nb);
+    const int fix = (a.numTiles + kFixChunk - 1) / kFixChunk;
+    if ((int)blockIdx.x < fix) {  // uniform over the workgroup
+        const int t0 = (int)blockIdx.x * kFixChunk;
+        fixup_tiles<TImg, MODE>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
         return;
     }
-    const int t0 = ((int)blockIdx.x - be.nb) * kFixChunk;
-    fixup_tiles<TImg, kSweepHist>(a, t0, min(kFixChunk, a.numTiles - t0), fixLds);
+    const int b = (int)blockIdx.x - fix;
+    if (MODE == kSweepHist) {
+        be_value_block(be.cpp, be.gnx, be.gny, be.gnz, be.bg, be.partials, b % be.nb, b / be.nb);
+    } else {
+        if (b == 0 && threadIdx.x == 0 && be.maxBits) *be.maxBits = 0u;
+        be_gradient_block(be.cpp, be.gnx, be.gny, be.gnz, be.bg, be.xyz, be.beGrad, b % be.nb, b / be.nb);
+    }
 }
 
 // Batched: one workgroup per chunk (pair, first tile, tiles) of the exact-pass chunk list.
@@ -850,7 +860,7 @@ struct NodeArgs {
     float weight;
     float *nodeGrad;
     // optional bending-energy term (reg_spline_approxBendingEnergyGradient3D's gathered sums,
-    // computed beside the sweep): grad += beRatio * beGrad, then the points' in-place
+    // computed beside the exact pass): grad += beRatio * beGrad, then the points' in-place
     // (p - node) + node round trip (reg-lib/cpu/_reg_localTrans_regul.cpp:312, 450)
     const float *beGrad;
     float beRatio;
@@ -937,15 +947,8 @@ __global__ void __launch_bounds__(256) k_project_y(ProjYArgs p) {
 }
 
 __global__ void __launch_bounds__(256) k_project_nodes(NodeArgs r) {
-    uint32_t bm = project_nodes_at(r, (size_t)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
-    if (r.maxBits) {
-        // reg_getMaximalLength of the final gradient (lengths >= 0 order like their bit patterns)
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t o = __shfl_down(bm, off, 64);
-            bm = o > bm ? o : bm;
-        }
-        if ((threadIdx.x & 63) == 0) atomicMax(r.maxBits, bm);
-    }
+    const uint32_t bits = project_nodes_at(r, (size_t)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
+    if (r.maxBits) block_track_max(r.maxBits, bits);  // reg_getMaximalLength of the final gradient
 }
 
 // Batched projections: item (pair, block of that pair); each output element is computed by the
@@ -969,7 +972,8 @@ __global__ void __launch_bounds__(256)
 k_project_nodes_batch(const NodeArgs *__restrict__ A, const int2 *__restrict__ items, const int *active) {
     const int2 it = items[blockIdx.x];
     if (active && !active[it.x]) return;
-    project_nodes_at(A[it.x], (size_t)it.y * blockDim.x + threadIdx.x);
+    const uint32_t bits = project_nodes_at(A[it.x], (size_t)it.y * blockDim.x + threadIdx.x);
+    block_track_max(A[it.x].maxBits, bits);
 }
 
 // K[r + w rb] = log p_r + log p_w - NMI log p_rw, evaluated in FP64 from the reference's log
@@ -1291,6 +1295,20 @@ static size_t sweep_lds(const FusedArgs& a, int depth) {
     return std::max<size_t>(((size_t)a.rb * a.fb + 3) / 4 * 4 * sizeof(float), window_lds(depth));
 }
 
+static BeArgs be_args(nrh_f3d *h) {
+    BeArgs be{};
+    be.cpp = h->cppPos.p;
+    be.gnx = h->cpp.nx;
+    be.gny = h->cpp.ny;
+    be.gnz = h->cpp.nz;
+    be.bg = be_brick_grid(h->cpp.nx, h->cpp.ny, h->cpp.nz);
+    be.nb = be.bg.bx * be.bg.by * be.bg.bz;
+    be.xyz = to_affine(h->cpp.xyz);
+    h->partials.alloc(std::max<size_t>(h->partials.n, 3 * (size_t)be.nb));
+    be.partials = h->partials.p;
+    return be;
+}
+
 void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pubS1, int pubN1) {
     FusedPlan *p = plan_of(h);
     NRH_REQUIRE(fused_supported(h), NRH_ERR_UNSUPPORTED, "fused path unavailable for this geometry or bin count");
@@ -1309,33 +1327,24 @@ void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pu
     }
     const unsigned fixBlocks = (unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk);
     const size_t fixLds = (size_t)a.rb * a.fb * sizeof(uint32_t);
+    int bePartials = 0;
     if (beValue) {
-        BeValueArgs be;
-        be.cpp = h->cppPos.p;
-        be.gnx = h->cpp.nx;
-        be.gny = h->cpp.ny;
-        be.gnz = h->cpp.nz;
-        be.bg = be_brick_grid(h->cpp.nx, h->cpp.ny, h->cpp.nz);
-        be.nb = be.bg.bx * be.bg.by * be.bg.bz;
-        h->partials.alloc(std::max<size_t>(h->partials.n, 2 * (size_t)be.nb + 64));
-        be.partials = h->partials.p;
-        be.ticket = h->maxBits.p + 6;
-        be.scale = 1.0 / (double)(3 * h->G);
-        be.out = h->scalars.p + 0;
-        const dim3 grid(fixBlocks + (unsigned)be.nb);
+        const BeArgs be = be_args(h);
+        bePartials = 3 * be.nb;
+        const dim3 grid(fixBlocks + (unsigned)bePartials);
         if (h->params.image_storage == 1)
-            hipLaunchKernelGGL(k_sweep_fixup_be<__half>, grid, dim3(256), fixLds, h->stream, a, be, be_basis());
+            hipLaunchKernelGGL((k_sweep_fixup_be<__half, kSweepHist>), grid, dim3(256), fixLds, h->stream, a, be);
         else
-            hipLaunchKernelGGL(k_sweep_fixup_be<float>, grid, dim3(256), fixLds, h->stream, a, be, be_basis());
+            hipLaunchKernelGGL((k_sweep_fixup_be<float, kSweepHist>), grid, dim3(256), fixLds, h->stream, a, be);
     } else if (h->params.image_storage == 1) {
         hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepHist>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
     } else {
         hipLaunchKernelGGL((k_sweep_fixup<float, kSweepHist>), dim3(fixBlocks), dim3(256), fixLds, h->stream, a);
     }
     NRH_HIP(hipGetLastError());
-    // the finalisation also writes the gradient sweep's NMI table
+    // the finalisation also writes the gradient sweep's NMI table and sums the bending energy
     p->kTab.alloc((size_t)(a.rb * a.fb + 3) / 4 * 4);
-    op_nmi_finalize(h, p->kTab.p, pubS1, pubN1);
+    op_nmi_finalize(h, p->kTab.p, pubS1, pubN1, bePartials);
     h->histVersion = h->cppVersion;
 }
 
@@ -1411,11 +1420,18 @@ static void projection_args(nrh_f3d *h, FusedPlan *p, const float *g, float weig
     r.maxBits = nullptr;
 }
 
+static void add_bending_energy(nrh_f3d *h, float weight, NodeArgs& r) {
+    h->beGrad.alloc(3 * h->G);
+    r.beGrad = h->beGrad.p;
+    r.beRatio = weight / (float)h->G;
+    r.cpp = h->cppPos.p;
+    r.cppXyz = to_affine(h->cpp.xyz);
+}
+
 // The voxel gradient g (planar [3][N]) projected onto the nodes: x pass (rows staged in LDS,
 // cell sums), y pass, z pass with normalisation, reorientation and weight, into h->nodeGrad.
-// beWeight > 0: the bending-energy sums the side stream computes (op_bending_energy_gradient_raw)
-// are joined in and added by the z pass, which also round-trips the points and, with maxBits,
-// tracks the final gradient's max length.
+// beWeight > 0: the bending-energy sums in h->beGrad are added by the z pass, which also round-trips
+// the points and, with maxBits, tracks the final gradient's max length.
 static void project_to_nodes(nrh_f3d *h, FusedPlan *p, const float *g, float weight, float beWeight = 0.f,
                              uint32_t *maxBits = nullptr) {
     ProjXArgs px;
@@ -1424,13 +1440,7 @@ static void project_to_nodes(nrh_f3d *h, FusedPlan *p, const float *g, float wei
     size_t ldsX = 0;
     projection_args(h, p, g, weight, px, py, r, &ldsX);
     if (beWeight > 0.f) {
-        // the bending-energy gradient sums on the side stream beside the x and y passes
-        fork_side(h);
-        op_bending_energy_gradient_raw(h, h->side);
-        r.beGrad = h->beGrad.p;
-        r.beRatio = beWeight / (float)h->G;
-        r.cpp = h->cppPos.p;
-        r.cppXyz = to_affine(h->cpp.xyz);
+        add_bending_energy(h, beWeight, r);
         r.maxBits = maxBits;
     }
     hipLaunchKernelGGL(k_project_x, dim3((unsigned)((px.rows + px.rowsPerBlock - 1) / px.rowsPerBlock)), dim3(256),
@@ -1438,7 +1448,6 @@ static void project_to_nodes(nrh_f3d *h, FusedPlan *p, const float *g, float wei
     // xcd_tile needs a grid that is a multiple of 8 (extra blocks find no work)
     auto blocks8 = [](size_t n) { return dim3((unsigned)(((n + 255) / 256 + 7) / 8 * 8)); };
     hipLaunchKernelGGL(k_project_y, blocks8((size_t)py.nz * py.gny * py.gnx), dim3(256), 0, h->stream, py);
-    if (beWeight > 0.f) join_side(h);
     hipLaunchKernelGGL(k_project_nodes, blocks8(h->G), dim3(256), 0, h->stream, r);
     NRH_HIP(hipGetLastError());
 }
@@ -1465,11 +1474,22 @@ void fused_gradient(nrh_f3d *h, float weight, float beWeight, uint32_t *maxBits)
         NRH_HIP(hipEventRecord(h->ev[3], h->stream));
         h->evPending[1] = true;
     }
-    const dim3 fixGrid((unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk));
-    if (h->params.image_storage == 1)
-        hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepGrad>), fixGrid, dim3(256), 0, h->stream, a);
-    else
-        hipLaunchKernelGGL((k_sweep_fixup<float, kSweepGrad>), fixGrid, dim3(256), 0, h->stream, a);
+    const unsigned fixBlocks = (unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk);
+    if (beWeight > 0.f) {
+        BeArgs be = be_args(h);
+        h->beGrad.alloc(3 * h->G);
+        be.beGrad = h->beGrad.p;
+        be.maxBits = maxBits;
+        const dim3 grid(fixBlocks + 3 * (unsigned)be.nb);
+        if (h->params.image_storage == 1)
+            hipLaunchKernelGGL((k_sweep_fixup_be<__half, kSweepGrad>), grid, dim3(256), 0, h->stream, a, be);
+        else
+            hipLaunchKernelGGL((k_sweep_fixup_be<float, kSweepGrad>), grid, dim3(256), 0, h->stream, a, be);
+    } else if (h->params.image_storage == 1) {
+        hipLaunchKernelGGL((k_sweep_fixup<__half, kSweepGrad>), dim3(fixBlocks), dim3(256), 0, h->stream, a);
+    } else {
+        hipLaunchKernelGGL((k_sweep_fixup<float, kSweepGrad>), dim3(fixBlocks), dim3(256), 0, h->stream, a);
+    }
     NRH_HIP(hipGetLastError());
     project_to_nodes(h, p, p->gvox.p, weight, beWeight, maxBits);
     if (beWeight > 0.f) h->cppVersion++;  // the round trip may have changed the last bit of some points
@@ -1520,6 +1540,8 @@ void batch_fused_setup(nrh_batch *b) {
         b->fixLds = std::max(b->fixLds, (size_t)nbins * sizeof(uint32_t));
         size_t ldsX = 0;
         projection_args(h, p, p->gvox.p, h->params.similarity_weight, pxs[q], pys[q], nds[q], &ldsX);
+        add_bending_energy(h, h->params.be_weight, nds[q]);
+        nds[q].maxBits = h->maxBits.p;
         b->projXLds = std::max(b->projXLds, ldsX);
         const int nbx = (int)((pxs[q].rows + pxs[q].rowsPerBlock - 1) / pxs[q].rowsPerBlock);
         for (int k = 0; k < nbx; ++k) itX.push_back(make_int2(q, k));

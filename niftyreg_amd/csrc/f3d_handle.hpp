@@ -32,12 +32,7 @@ struct nrh_f3d {
 
     // control points (planar [3][G]) and optimiser arrays
     nrh::DevBuf<float> cppPos, best, nodeGrad, cgG, cgH;
-    nrh::DevBuf<float> beGrad;  // bending-energy gradient sums computed beside the gradient sweep [3][G]
-
-    // a second stream for work that overlaps the sweeps (the bending energy), forked from and
-    // joined back to `stream` with the two events
-    hipStream_t side = nullptr;
-    hipEvent_t evFork = nullptr, evJoin = nullptr;
+    nrh::DevBuf<float> beGrad;  // bending-energy gradient sums [3][G]
 
     // per-operation buffers, allocated on first use
     nrh::DevBuf<float> field, warped, warpedGrad, voxelGrad;
@@ -141,8 +136,10 @@ void op_resample(nrh_f3d *h);
 void op_image_gradient(nrh_f3d *h);
 void op_joint_histogram(nrh_f3d *h, const float *warped);
 // kTab (optional): also the fused gradient sweep's NMI table, when the histogram fits the LDS
-// finalisation (h->kTabCurrent says whether it was written)
-void op_nmi_finalize(nrh_f3d *h, float *kTab = nullptr, const double *pubS1 = nullptr, int pubN1 = -1);
+// finalisation (h->kTabCurrent says whether it was written); bePartials > 0: the bending energy too,
+// into scalars[0], from that many partials
+void op_nmi_finalize(nrh_f3d *h, float *kTab = nullptr, const double *pubS1 = nullptr, int pubN1 = -1,
+                     int bePartials = 0);
 void op_nmi_voxel_gradient(nrh_f3d *h, double weight);
 void op_convolve_voxel_gradient(nrh_f3d *h);
 void op_voxel_to_node(nrh_f3d *h, float weight);
@@ -157,11 +154,9 @@ void zero_voxel_gradient(nrh_f3d *h);
 // voxel transform and the reorientation of op_voxel_to_node
 int convolution_kernel(float spacing, float pixdim, std::vector<float>& kern);
 void node_transforms(const nrh_f3d *h, Affine& T, Affine& R);
-// stream: where the launch goes (null: the handle's stream)
-void op_bending_energy(nrh_f3d *h, double *out_device, hipStream_t stream = nullptr);
-// the bending-energy gradient's gathered sums alone into h->beGrad (no weight, no round trip),
-// for a projection that adds them (fused_gradient's BE overlap)
-void op_bending_energy_gradient_raw(nrh_f3d *h, hipStream_t stream);
+void op_bending_energy(nrh_f3d *h, double *out_device);
+// the bending energy from n partials of be_value_block in h->partials
+void op_bending_energy_sum(nrh_f3d *h, int n, double *out_device);
 // trackMax: also leave the max length of the final gradient in maxBits[0] (float bits)
 void op_bending_energy_gradient(nrh_f3d *h, float weight, bool trackMax = false);
 void op_max_length(nrh_f3d *h);
@@ -218,13 +213,9 @@ void fused_warp(nrh_f3d *h);
 // (op_publish's layout, the sequence number advanced)
 void fused_histogram(nrh_f3d *h, float *fieldOut = nullptr, bool beValue = false, const double *pubS1 = nullptr,
                      int pubN1 = -1);
-// beWeight > 0: the bending-energy gradient sums run on the side stream beside the x and y
-// projection passes (op_bending_energy_gradient_raw); the node projection joins and adds them,
-// round-trips the points and, with maxBits, tracks the final gradient's max length
+// beWeight > 0: the bending-energy gradient sums run in the exact pass's launch; the node projection
+// adds them, round-trips the points and, with maxBits, tracks the final gradient's max length
 void fused_gradient(nrh_f3d *h, float weight, float beWeight = 0.f, uint32_t *maxBits = nullptr);
-// work on h->side after everything enqueued on h->stream so far / h->stream after h->side's work
-void fork_side(nrh_f3d *h);
-void join_side(nrh_f3d *h);
 void collect_sweep_times(nrh_f3d *h);  // after a stream synchronisation
 // The separable node projection of a voxel gradient (integer spacing, nodes on voxels): the
 // convolution + VoxelCentricToNodeCentric of the reference as three passes, into nodeGrad.

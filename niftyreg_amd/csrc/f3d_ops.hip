@@ -189,11 +189,10 @@ k_nmi_finalize(uint32_t *__restrict__ counts, int rb, int fb, double *__restrict
     }
 }
 
-// K[i] = log p_r + log p_w - NMI log p_rw for joint bin i = r + w rb, from the logs L (joint
-// [0, nb), reference marginal [nb, nb + rb), floating marginal after), rounded once to float.
-__device__ __forceinline__ float nmi_table_entry(const double *L, int nb, int rb, double nmi, int i) {
+// K[i] = log p_r + log p_w - NMI log p_rw for joint bin i = r + w rb, rounded once to float.
+__device__ __forceinline__ float nmi_table_value(double lr, double lw, double nmi, double l) {
 #pragma clang fp contract(off)
-    return (float)((L[nb + i % rb] + L[nb + rb + i / rb]) - nmi * L[i]);
+    return (float)((lr + lw) - nmi * l);
 }
 
 // The same finalisation with the working array in LDS (histograms of up to kFinLds entries):
@@ -201,107 +200,141 @@ __device__ __forceinline__ float nmi_table_entry(const double *L, int nb, int rb
 constexpr int kFinLds = 7936;
 constexpr int kFinPer = (kFinLds + 1023) / 1024;
 
-// Phase 1: P (LDS) = the smoothed joint histogram normalised by its total, then its marginals;
-// consume: the counts are zeroed as they are read, ready for the next histogram.
-__device__ __forceinline__ void fin_probabilities(uint32_t *__restrict__ counts, bool consume, int rb, int fb,
-                                                  double *P, double *red, double& totalS) {
-    const int nb = rb * fb, total = nb + rb + fb;
+// Phase 1: v[q] = the smoothed joint histogram, normalised by its total, at entries
+// tid + 1024 q (also in P, LDS), r[q] and f[q] their bins; then its marginals in P.  The counts are
+// zeroed as they are read, ready for the next histogram.
+__device__ __forceinline__ void fin_probabilities(uint32_t *__restrict__ counts, int rb, int fb, double *P, double *red,
+                                                  double& totalS, double (&v)[kFinPer], int (&r)[kFinPer],
+                                                  int (&f)[kFinPer]) {
+    const int nb = rb * fb, tid = threadIdx.x;
     const double k0 = 1.0 / 6.0, k1 = (double)(2.f / 3.f);
-    // the counts are consumed: zeroed as they are read, ready for the next histogram
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
-        P[i] = i < nb ? (double)counts[i] : 0.0;
-        if (consume && i < nb) counts[i] = 0u;
+    {
+        // one division per thread: the bins of the next entry are 1024 entries further
+        const int dr = 1024 % rb, df = 1024 / rb;
+        r[0] = tid % rb;
+        f[0] = tid / rb;
+#pragma unroll
+        for (int q = 1; q < kFinPer; ++q) {
+            const bool wrap = r[q - 1] + dr >= rb;
+            r[q] = r[q - 1] + dr - (wrap ? rb : 0);
+            f[q] = f[q - 1] + df + (wrap ? 1 : 0);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kFinPer; ++q) {
+        const int i = tid + q * 1024;
+        if (i < nb) {
+            P[i] = (double)counts[i];
+            counts[i] = 0u;
+        }
     }
     __syncthreads();
-    double v[kFinPer];
     // along the reference axis
 #pragma unroll
     for (int q = 0; q < kFinPer; ++q) {
-        const int i = threadIdx.x + q * 1024;
+        const int i = tid + q * 1024;
         v[q] = 0;
         if (i < nb) {
-            const int r = i % rb;
             double t = 0;
-            if (r - 1 > -1) t += P[i - 1] * k0;
+            if (r[q] - 1 > -1) t += P[i - 1] * k0;
             t += P[i] * k1;
-            if (r + 1 < rb) t += P[i + 1] * k0;
+            if (r[q] + 1 < rb) t += P[i + 1] * k0;
             v[q] = t;
         }
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kFinPer; ++q) {
-        const int i = threadIdx.x + q * 1024;
+        const int i = tid + q * 1024;
         if (i < nb) P[i] = v[q];
     }
     __syncthreads();
-    // along the floating axis
-#pragma unroll
-    for (int q = 0; q < kFinPer; ++q) {
-        const int i = threadIdx.x + q * 1024;
-        v[q] = 0;
-        if (i < nb) {
-            const int f = i / rb;
-            double t = 0;
-            if (f - 1 > -1) t += P[i - rb] * k0;
-            t += P[i] * k1;
-            if (f + 1 < fb) t += P[i + rb] * k0;
-            v[q] = t;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kFinPer; ++q) {
-        const int i = threadIdx.x + q * 1024;
-        if (i < nb) P[i] = v[q];
-    }
-    __syncthreads();
+    // along the floating axis, and the total
     double s = 0;
-    for (int i = threadIdx.x; i < total; i += blockDim.x) s += P[i];
-    s = block_sum_double(s, red);
-    if (threadIdx.x == 0) totalS = s;
+#pragma unroll
+    for (int q = 0; q < kFinPer; ++q) {
+        const int i = tid + q * 1024;
+        v[q] = 0;
+        if (i < nb) {
+            double t = 0;
+            if (f[q] - 1 > -1) t += P[i - rb] * k0;
+            t += P[i] * k1;
+            if (f[q] + 1 < fb) t += P[i + rb] * k0;
+            v[q] = t;
+            s += t;
+        }
+    }
+    s = block_sum_double(s, red);  // its barriers also end the reads of P
+    if (tid == 0) totalS = s;
     __syncthreads();
     const double act = totalS;
-    for (int i = threadIdx.x; i < total; i += blockDim.x) P[i] /= act;
-    __syncthreads();
-    for (int i = threadIdx.x; i < rb + fb; i += blockDim.x) {
-        double m = 0;
-        if (i < rb) {
-            for (int f = 0; f < fb; ++f) m += P[i + rb * f];
-        } else {
-            const int f = i - rb;
-            for (int r = 0; r < rb; ++r) m += P[rb * f + r];
+#pragma unroll
+    for (int q = 0; q < kFinPer; ++q) {
+        const int i = tid + q * 1024;
+        if (i < nb) {
+            v[q] /= act;
+            P[i] = v[q];
         }
-        P[nb + i] = m;
     }
     __syncthreads();
+    for (int i = tid; i < rb + fb; i += 1024) {
+        double m = 0;
+        const double *p = i < rb ? P + i : P + rb * (i - rb);
+        const int n = i < rb ? fb : rb, stride = i < rb ? rb : 1;
+        int k = 0;
+        for (; k + 8 <= n; k += 8) {
+            double w[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) w[u] = p[(k + u) * stride];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) m += w[u];
+        }
+        for (; k < n; ++k) m += p[k * stride];
+        P[nb + i] = m;
+    }
 }
 
 // Phase 2: the logarithms (written with the probabilities), the entropies (each thread's strided
-// terms, then block sums: H_r, H_f, H_rf), ent[] and the table K.  P holds the logs after.
+// terms, then block sums: H_r, H_f, H_rf), ent[] and the table K.
 __device__ __forceinline__ void fin_entropies(int rb, int fb, double *P, double *red /* 48 */, double& totalS,
-                                              double *__restrict__ pro, double *__restrict__ logh,
-                                              float *__restrict__ logf, double *__restrict__ ent,
-                                              float *__restrict__ kTab) {
-    const int nb = rb * fb, total = nb + rb + fb;
+                                              const double (&v)[kFinPer], const int (&r)[kFinPer],
+                                              const int (&f)[kFinPer], double *__restrict__ pro,
+                                              double *__restrict__ logh, float *__restrict__ logf,
+                                              double *__restrict__ ent, float *__restrict__ kTab) {
+    const int nb = rb * fb, total = nb + rb + fb, tid = threadIdx.x;
     const double act = totalS;
-    double hr = 0, hf = 0, hj = 0;
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
+    double hr = 0, hf = 0, hj = 0, l[kFinPer];
+    // the joint entries need no marginal: no barrier keeps them waiting for the threads that sum those
+#pragma unroll
+    for (int q = 0; q < kFinPer; ++q) {
+        const int i = tid + q * 1024;
+        l[q] = 0;
+        if (i < nb) {
+            if (v[q] > 0) {
+                l[q] = log(v[q]);
+                hj -= v[q] * l[q];
+            }
+            pro[i] = v[q];
+            logh[i] = l[q];
+            logf[i] = (float)l[q];
+        }
+    }
+    __syncthreads();
+    for (int i = nb + (tid - nb % 1024 + 1024) % 1024; i < total; i += 1024) {
         const double p = P[i];
-        double l = 0;
+        double lm = 0;
         if (p > 0) {
-            l = log(p);
-            if (i < nb) hj -= p * l;
-            else if (i < nb + rb) hr -= p * l;
-            else hf -= p * l;
+            lm = log(p);
+            if (i < nb + rb) hr -= p * lm;
+            else hf -= p * lm;
         }
         pro[i] = p;
-        logh[i] = l;
-        logf[i] = (float)l;
-        P[i] = l;  // the logs stay in LDS for the table K
+        logh[i] = lm;
+        logf[i] = (float)lm;
+        P[i] = lm;  // for the table K
     }
     block_sum_double3(hr, hf, hj, red);
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         ent[0] = hr;
         ent[1] = hf;
         ent[2] = hj;
@@ -314,11 +347,18 @@ __device__ __forceinline__ void fin_entropies(int rb, int fb, double *P, double 
         // k_nmi_table computes it, from the same FP64 logs)
         __syncthreads();
         const double nmi = totalS;
-        for (int i = threadIdx.x; i < nb; i += blockDim.x) kTab[i] = nmi_table_entry(P, nb, rb, nmi, i);
+#pragma unroll
+        for (int q = 0; q < kFinPer; ++q) {
+            const int i = tid + q * 1024;
+            if (i < nb) kTab[i] = nmi_table_value(P[nb + r[q]], P[nb + rb + f[q]], nmi, l[q]);
+        }
     }
 }
 
-// The whole finalisation in one workgroup.
+// The whole finalisation in one workgroup of 1024 threads.  One workgroup does it all because every
+// step needs the one before it whole; what it takes is the instructions of its 16 waves, so each
+// entry is loaded, smoothed and logged by one thread that keeps it in registers.  64 x 64 bins:
+// 20 us with every entry's bins found by division in each of five passes over LDS, 15 us so.
 __device__ __forceinline__ void
 nmi_finalize_lds_block(uint32_t *__restrict__ counts, int rb, int fb, double *__restrict__ pro,
                    double *__restrict__ logh, float *__restrict__ logf, double *__restrict__ ent,
@@ -326,8 +366,10 @@ nmi_finalize_lds_block(uint32_t *__restrict__ counts, int rb, int fb, double *__
     __shared__ double P[kFinLds];
     __shared__ double red[48];
     __shared__ double totalS;
-    fin_probabilities(counts, true, rb, fb, P, red, totalS);
-    fin_entropies(rb, fb, P, red, totalS, pro, logh, logf, ent, kTab);
+    double v[kFinPer];
+    int r[kFinPer], f[kFinPer];
+    fin_probabilities(counts, rb, fb, P, red, totalS, v, r, f);
+    fin_entropies(rb, fb, P, red, totalS, v, r, f, pro, logh, logf, ent, kTab);
 }
 
 // reg_getVoxelBasedNmiGradient3d<float> (reg-lib/cpu/_reg_nmi.cpp:501-593); grad +=
@@ -483,143 +525,28 @@ k_voxel_to_node(const float *__restrict__ vg, int nx, int ny, int nz, int gnx, i
 }
 
 // ------------------------------------------------------------------ bending energy
-// (the basis, brick grid and value block body are in be_blocks.hpp)
+// (the basis, the brick grid and the bodies over bricks are in be_blocks.hpp)
 
-// reg_spline_approxBendingEnergyGradient3D (regul.cpp:287-451) on a brick: the displacement
-// (cpp - node) of the brick with a two-node halo in LDS, the 18 second derivatives of every node
-// of the brick with a one-node halo (regul.cpp:317-379, the cross terms doubled in double), then
-// the adjoint 27-point gather grad += weight / G * value (regul.cpp:381-448) for the brick's
-// nodes.  Optionally tracks the max length of the final gradient.  The reference's in-place
-// (p - node) + node round trip of the points is k_round_trip, run after this kernel.  RAW: the
-// gathered sums alone are written to grad (planar [3][G]) for a later grad += weight / G * value.
-template<bool RAW = false>
-__device__ __forceinline__ void
-be_gradient_block(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, Affine xyz, BeBasis B,
-              float ratio, float *__restrict__ grad, uint32_t *__restrict__ maxBits, int bid) {
-#pragma clang fp contract(off)
-    constexpr int CX = BBX + 4, CY = BBY + 4, CZ = BBZ + 4, CN = CX * CY * CZ;  // points: two-node halo
-    constexpr int DX = BBX + 2, DY = BBY + 2, DZ = BBZ + 2, DN = DX * DY * DZ;  // derivatives: one-node halo
-    __shared__ float sC[3][CN];
-    __shared__ float sD[18][DN];
-    __shared__ float sB[27][8];  // basis values per neighbour (xx, yy, zz, xy, yz, xz), read as broadcasts
-    const size_t G = (size_t)gnx * gny * gnz;
-    int x0, y0, z0;
-    brick_origin(bg, bid, x0, y0, z0);
-    if (threadIdx.x < 27 * 6) sB[threadIdx.x / 6][threadIdx.x % 6] = B.b[threadIdx.x % 6][threadIdx.x / 6];
-    {
-        constexpr int kIter = (3 * CN + 255) / 256;
-        float v[kIter];
-#pragma unroll
-        for (int u = 0; u < kIter; ++u) {
-            // clamped, unconditional loads keep v in registers (out-of-grid entries are never read)
-            const int i = min((int)threadIdx.x + u * 256, 3 * CN - 1);
-            const int c = i / CN, r = i % CN, hx = r % CX, hy = (r / CX) % CY, hz = r / (CX * CY);
-            const int X = min(max(x0 - 2 + hx, 0), gnx - 1), Y = min(max(y0 - 2 + hy, 0), gny - 1),
-                      Z = min(max(z0 - 2 + hz, 0), gnz - 1);
-            v[u] = cpp[c * G + ((size_t)Z * gny + Y) * gnx + X] - node_pos(xyz, c, X, Y, Z);
-        }
-#pragma unroll
-        for (int u = 0; u < kIter; ++u) {
-            const int i = threadIdx.x + u * 256;
-            if (i < 3 * CN) sC[i / CN][i % CN] = v[u];
-        }
-    }
-    __syncthreads();
-    for (int r = threadIdx.x; r < DN; r += 256) {
-        const int hx = r % DX, hy = (r / DX) % DY, hz = r / (DX * DY);
-        const int x = x0 - 1 + hx, y = y0 - 1 + hy, z = z0 - 1 + hz;
-        float d[3][6] = {};
-        if (x >= 0 && y >= 0 && z >= 0 && x < gnx && y < gny && z < gnz) {
-            int i = 0;
-#pragma unroll
-            for (int c = -1; c < 2; ++c)
-#pragma unroll
-                for (int b = -1; b < 2; ++b)
-#pragma unroll
-                    for (int a = -1; a < 2; ++a, ++i) {
-                        const int X = x + a, Y = y + b, Z = z + c;
-                        if (X < 0 || Y < 0 || Z < 0 || X >= gnx || Y >= gny || Z >= gnz) continue;
-                        const int h = ((hz + 1 + c) * CY + hy + 1 + b) * CX + hx + 1 + a;
-                        float bt[6];
-#pragma unroll
-                        for (int t = 0; t < 6; ++t) bt[t] = sB[i][t];
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) {
-                            const float cv = sC[k][h];
-#pragma unroll
-                            for (int t = 0; t < 6; ++t) d[k][t] += bt[t] * cv;
-                        }
-                    }
-        }
-        for (int t = 0; t < 3; ++t)
-            for (int k = 0; k < 3; ++k) sD[t * 3 + k][r] = d[k][t];
-        for (int t = 3; t < 6; ++t)
-            for (int k = 0; k < 3; ++k) sD[t * 3 + k][r] = (float)(2.0 * (double)d[k][t]);
-    }
-    __syncthreads();
-    const int tx = threadIdx.x % BBX, ty = (threadIdx.x / BBX) % BBY, tz = threadIdx.x / (BBX * BBY);
-    const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
-    const bool valid = x < gnx && y < gny && z < gnz;
-    float g0 = 0.f, g1 = 0.f, g2 = 0.f;
-    if (valid) {
-        const size_t n = ((size_t)z * gny + y) * gnx + x;
-        float gv[3] = { 0.f, 0.f, 0.f };
-        int a = 0;
-#pragma unroll
-        for (int c = -1; c < 2; ++c)
-#pragma unroll
-            for (int b = -1; b < 2; ++b)
-#pragma unroll
-                for (int q = -1; q < 2; ++q, ++a) {
-                    const int X = x + q, Y = y + b, Z = z + c;
-                    if (X < 0 || Y < 0 || Z < 0 || X >= gnx || Y >= gny || Z >= gnz) continue;
-                    const int r = ((tz + 1 + c) * DY + ty + 1 + b) * DX + tx + 1 + q;
-                    float bt[6];
-#pragma unroll
-                    for (int t = 0; t < 6; ++t) bt[t] = sB[a][t];
-#pragma unroll
-                    for (int t = 0; t < 6; ++t)
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) gv[k] += sD[t * 3 + k][r] * bt[t];
-                }
-        if (RAW) {
-            grad[n] = gv[0];
-            grad[n + G] = gv[1];
-            grad[n + 2 * G] = gv[2];
-        } else {
-            g0 = grad[n] + ratio * gv[0];
-            g1 = grad[n + G] + ratio * gv[1];
-            g2 = grad[n + 2 * G] + ratio * gv[2];
-            grad[n] = g0;
-            grad[n + G] = g1;
-            grad[n + 2 * G] = g2;
-        }
-    }
-    if (!RAW && maxBits) {
-        // reg_getMaximalLength of the final gradient (lengths >= 0 order like their bit patterns)
-        uint32_t bm = valid ? __float_as_uint(sqrtf(g0 * g0 + g1 * g1 + g2 * g2)) : 0u;
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t o = __shfl_down(bm, off, 64);
-            bm = o > bm ? o : bm;
-        }
-        if ((threadIdx.x & 63) == 0) atomicMax(maxBits, bm);
-    }
-}
-
-// The in-place reg_getDisplacementFromDeformation / reg_getDeformationFromDisplacement pair the
-// reference wraps around the bending-energy gradient (regul.cpp:312, 450): p <- (p - node) + node.
-__device__ __forceinline__ void
-round_trip_block(float *__restrict__ cpp, int gnx, int gny, int gnz, Affine xyz, int bid) {
+// The end of the bending-energy gradient at node n: grad += ratio * (the gathered sums), and the
+// in-place reg_getDisplacementFromDeformation / reg_getDeformationFromDisplacement pair the
+// reference wraps around it (regul.cpp:312, 450): p <- (p - node) + node.  Returns the float bits
+// of the final gradient's length (0 past the grid).
+__device__ __forceinline__ uint32_t
+be_apply_at(float *__restrict__ cpp, int gnx, int gny, int gnz, const Affine& xyz, const float *__restrict__ beGrad,
+            float ratio, float *__restrict__ grad, size_t n) {
 #pragma clang fp contract(off)
     const size_t G = (size_t)gnx * gny * gnz;
-    const size_t n = (size_t)bid * blockDim.x + threadIdx.x;
-    if (n >= G) return;
+    if (n >= G) return 0u;
     int x, y, z;
     index_xyz(n, gnx, gny, x, y, z);
+    float g[3];
     for (int k = 0; k < 3; ++k) {
+        g[k] = grad[n + k * G] + ratio * beGrad[n + k * G];
+        grad[n + k * G] = g[k];
         const float node = node_pos(xyz, k, x, y, z);
         cpp[n + k * G] = (cpp[n + k * G] - node) + node;
     }
+    return __float_as_uint(sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]));
 }
 
 // ------------------------------------------------------------------ linear energy
@@ -747,14 +674,7 @@ k_le_grad(const float *__restrict__ diag, int gnx, int gny, int gnz, LeBasis B, 
         grad[n + G] = g1;
         grad[n + 2 * G] = g2;
     }
-    if (maxBits) {
-        uint32_t bits = valid ? __float_as_uint(sqrtf(g0 * g0 + g1 * g1 + g2 * g2)) : 0u;
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t o = __shfl_down(bits, off, 64);
-            bits = o > bits ? o : bits;
-        }
-        if ((threadIdx.x & 63) == 0) atomicMax(maxBits, bits);
-    }
+    if (maxBits) block_track_max(maxBits, valid ? __float_as_uint(sqrtf(g0 * g0 + g1 * g1 + g2 * g2)) : 0u);
 }
 
 // ------------------------------------------------------------------ optimiser helpers
@@ -770,11 +690,7 @@ k_max_length(const float *__restrict__ g, size_t G, uint32_t *__restrict__ out) 
         const uint32_t b = __float_as_uint(l);
         best = b > best ? b : best;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        const uint32_t o = __shfl_down(best, off, 64);
-        best = o > best ? o : best;
-    }
-    if ((threadIdx.x & 63) == 0) atomicMax(out, best);
+    block_track_max(out, best);
 }
 
 __global__ void k_max_to_scalar(const uint32_t *__restrict__ bits, double *__restrict__ out) {
@@ -921,43 +837,58 @@ __global__ void k_fill_f32(float *p, size_t n, float v) {
 // The single-pair finalisation (one workgroup).  pub (may be null): it then publishes ent[0..4]
 // and s1[0..n1) to coherent host memory followed by the sequence number seq (k_publish's
 // layout), so the objective needs no publishing kernel of its own.
+// be (may be null): the bending-energy partials of the launch before, summed into *beOut as k_be_sum
+// does.
 __global__ void __launch_bounds__(1024)
 k_nmi_finalize_lds(uint32_t *__restrict__ counts, int rb, int fb, double *__restrict__ pro,
                    double *__restrict__ logh, float *__restrict__ logf, double *__restrict__ ent,
-                   float *__restrict__ kTab, double *__restrict__ pub, const double *__restrict__ s1, int n1,
+                   float *__restrict__ kTab, const double *__restrict__ be, int nBe, double beScale,
+                   double *__restrict__ beOut, double *__restrict__ pub, const double *__restrict__ s1, int n1,
                    uint64_t seq) {
+    __shared__ double redBe[16];
+    if (be) {
+        const double t = sum_partials_256(be, nBe, redBe);
+        if (threadIdx.x == 0) *beOut = t * beScale;
+    }
     nmi_finalize_lds_block(counts, rb, fb, pro, logh, logf, ent, kTab);
     if (pub) {
         __syncthreads();
         const int i = threadIdx.x;
-        if (i < 5) pub[i] = ent[i];
-        else if (i < 5 + n1) pub[i] = s1[i - 5];
-        __threadfence_system();
-        __syncthreads();
-        if (i == 0) __hip_atomic_store((uint64_t *)(pub + 15), seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (i < 64) {  // the first wave alone publishes
+            if (i < 5) pub[i] = ent[i];
+            else if (i < 5 + n1) pub[i] = s1[i - 5];
+            __threadfence_system();
+            if (i == 0)
+                __hip_atomic_store((uint64_t *)(pub + 15), seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
+// Bending energy: a workgroup per brick (x) and component (y).
 __global__ void __launch_bounds__(256)
-k_be_value(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, BeBasis B,
-           double *__restrict__ partials, uint32_t *__restrict__ ticket, double scale, double *__restrict__ out) {
-    be_value_block(cpp, gnx, gny, gnz, bg, B, partials, ticket, scale, out, blockIdx.x, gridDim.x);
+k_be_value(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, double *__restrict__ partials) {
+    be_value_block(cpp, gnx, gny, gnz, bg, partials, blockIdx.x, blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256)
-k_be_gradient(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, Affine xyz, BeBasis B,
-              float ratio, float *__restrict__ grad, uint32_t *__restrict__ maxBits) {
-    be_gradient_block(cpp, gnx, gny, gnz, bg, xyz, B, ratio, grad, maxBits, blockIdx.x);
+k_be_sum(const double *__restrict__ partials, int n, double scale, double *__restrict__ out) {
+    __shared__ double red[16];
+    const double t = sum_partials_256(partials, n, red);
+    if (threadIdx.x == 0) *out = t * scale;
 }
 
 __global__ void __launch_bounds__(256)
-k_be_gradient_raw(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, Affine xyz, BeBasis B,
-                  float *__restrict__ out) {
-    be_gradient_block<true>(cpp, gnx, gny, gnz, bg, xyz, B, 0.f, out, nullptr, blockIdx.x);
+k_be_gradient(const float *__restrict__ cpp, int gnx, int gny, int gnz, BrickGrid bg, Affine xyz,
+              float *__restrict__ out) {
+    be_gradient_block(cpp, gnx, gny, gnz, bg, xyz, out, blockIdx.x, blockIdx.y);
 }
 
-__global__ void __launch_bounds__(256) k_round_trip(float *__restrict__ cpp, int gnx, int gny, int gnz, Affine xyz) {
-    round_trip_block(cpp, gnx, gny, gnz, xyz, blockIdx.x);
+__global__ void __launch_bounds__(256)
+k_be_apply(float *__restrict__ cpp, int gnx, int gny, int gnz, Affine xyz, const float *__restrict__ beGrad, float ratio,
+           float *__restrict__ grad, uint32_t *__restrict__ maxBits) {
+    const uint32_t bits = be_apply_at(cpp, gnx, gny, gnz, xyz, beGrad, ratio, grad,
+                                      (size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (maxBits) block_track_max(maxBits, bits);
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -1006,7 +937,7 @@ struct PairOps {
     float beRatio;         // bending-energy weight / G
     double beScale;        // 1 / (3 G)
     double *partials;      // bending-energy value and CG dot partials
-    uint32_t *beTicket;
+    float *beGrad;
     double *beOut;         // bending energy (scalars[0])
     uint32_t *maxBits;     // max gradient length as float bits
     double *maxLen;        // scalars[1]
@@ -1027,27 +958,19 @@ __global__ void __launch_bounds__(1024) k_nmi_finalize_batch(const PairOps *__re
 }
 
 __global__ void __launch_bounds__(256)
-k_be_value_batch(const PairOps *__restrict__ P, const int2 *__restrict__ items, BeBasis B, const int *active) {
+k_be_value_batch(const PairOps *__restrict__ P, const int2 *__restrict__ items, const int *active) {
     const int2 it = items[blockIdx.x];
     if (skip_pair(active, it.x)) return;
     const PairOps& q = P[it.x];
-    be_value_block(q.cpp, q.gnx, q.gny, q.gnz, q.bg, B, q.partials, q.beTicket, q.beScale, q.beOut, it.y, q.beBlocks);
+    be_value_block(q.cpp, q.gnx, q.gny, q.gnz, q.bg, q.partials, it.y, blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256)
-k_be_gradient_batch(const PairOps *__restrict__ P, const int2 *__restrict__ items, BeBasis B, const int *active) {
+k_be_gradient_batch(const PairOps *__restrict__ P, const int2 *__restrict__ items, const int *active) {
     const int2 it = items[blockIdx.x];
     if (skip_pair(active, it.x)) return;
     const PairOps& q = P[it.x];
-    be_gradient_block(q.cpp, q.gnx, q.gny, q.gnz, q.bg, q.xyz, B, q.beRatio, q.grad, q.maxBits, it.y);
-}
-
-__global__ void __launch_bounds__(256)
-k_round_trip_batch(const PairOps *__restrict__ P, const int2 *__restrict__ items, const int *active) {
-    const int2 it = items[blockIdx.x];
-    if (skip_pair(active, it.x)) return;
-    const PairOps& q = P[it.x];
-    round_trip_block(q.cpp, q.gnx, q.gny, q.gnz, q.xyz, it.y);
+    be_gradient_block(q.cpp, q.gnx, q.gny, q.gnz, q.bg, q.xyz, q.beGrad, it.y, blockIdx.y);
 }
 
 // items over 3 G: element-wise kernels of the control-point arrays
@@ -1120,37 +1043,7 @@ __global__ void k_zero_max_bits_batch(const PairOps *__restrict__ P, int n, cons
     if (i < n && !skip_pair(active, i)) *P[i].maxBits = 0u;
 }
 
-// Round to the 6-decimal literals the reference tabulates (reg-lib/cpu/_reg_splineBasis.cpp:292-457).
-float round6(double v) {
-    const double r = std::floor(std::fabs(v) * 1e6 + 0.5) / 1e6;
-    return (float)(v < 0 ? -r : r);
-}
-
-BeBasis make_be_basis() {
-    // Tensor products of the cubic B-spline at a node: value {1/6, 2/3, 1/6}, first
-    // derivative {-1/2, 0, 1/2}, second derivative {1, -2, 1}.
-    const double v[3] = { 1.0 / 6.0, 2.0 / 3.0, 1.0 / 6.0 }, d1[3] = { -0.5, 0.0, 0.5 }, d2[3] = { 1.0, -2.0, 1.0 };
-    BeBasis B;
-    int i = 0;
-    for (int c = 0; c < 3; ++c)
-        for (int b = 0; b < 3; ++b)
-            for (int a = 0; a < 3; ++a, ++i) {
-                B.b[0][i] = round6(d2[a] * v[b] * v[c]);
-                B.b[1][i] = round6(v[a] * d2[b] * v[c]);
-                B.b[2][i] = round6(v[a] * v[b] * d2[c]);
-                B.b[3][i] = round6(d1[a] * d1[b] * v[c]);
-                B.b[4][i] = round6(v[a] * d1[b] * d1[c]);
-                B.b[5][i] = round6(d1[a] * v[b] * d1[c]);
-            }
-    return B;
-}
-
 }  // namespace
-
-BeBasis be_basis() {
-    static const BeBasis B = make_be_basis();
-    return B;
-}
 
 // ------------------------------------------------------------------ launches
 void op_fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s) {
@@ -1221,18 +1114,20 @@ void op_joint_histogram(nrh_f3d *h, const float *warped) {
     NRH_HIP(hipGetLastError());
 }
 
-void op_nmi_finalize(nrh_f3d *h, float *kTab, const double *pubS1, int pubN1) {
+void op_nmi_finalize(nrh_f3d *h, float *kTab, const double *pubS1, int pubN1, int bePartials) {
     h->kTabCurrent = kTab != nullptr && h->totalBins() <= kFinLds;
     NRH_REQUIRE(pubN1 < 0 || (h->totalBins() <= kFinLds && pubN1 <= 10), NRH_ERR_ARG, "finalisation cannot publish");
     if (h->totalBins() <= kFinLds) {
         const bool pub = pubN1 >= 0;
         hipLaunchKernelGGL(k_nmi_finalize_lds, dim3(1), dim3(1024), 0, h->stream, h->histCount.p, h->params.ref_bins,
                            h->params.flo_bins, h->histPro.p, h->histLog.p, h->histLogF.p, h->ent.p,
-                           h->kTabCurrent ? kTab : nullptr, pub ? h->publishedDev : nullptr, pubS1, pub ? pubN1 : 0,
-                           pub ? ++h->publishSeq : (uint64_t)0);
+                           h->kTabCurrent ? kTab : nullptr, bePartials > 0 ? (const double *)h->partials.p : nullptr,
+                           bePartials, 1.0 / (double)(3 * h->G), h->scalars.p + 0, pub ? h->publishedDev : nullptr, pubS1,
+                           pub ? pubN1 : 0, pub ? ++h->publishSeq : (uint64_t)0);
     } else {
         hipLaunchKernelGGL(k_nmi_finalize, dim3(1), dim3(1024), 0, h->stream, h->histCount.p, h->params.ref_bins,
                            h->params.flo_bins, h->histPro.p, h->histLog.p, h->histLogF.p, h->ent.p);
+        if (bePartials > 0) op_bending_energy_sum(h, bePartials, h->scalars.p + 0);
     }
     NRH_HIP(hipGetLastError());
 }
@@ -1373,59 +1268,33 @@ void op_voxel_to_node(nrh_f3d *h, float weight) {
     NRH_HIP(hipGetLastError());
 }
 
-static BrickGrid brick_grid(const nrh_f3d *h) {
-    BrickGrid g;
-    g.bx = (h->cpp.nx + BBX - 1) / BBX;
-    g.by = (h->cpp.ny + BBY - 1) / BBY;
-    g.bz = (h->cpp.nz + BBZ - 1) / BBZ;
-    return g;
-}
+static BrickGrid brick_grid(const nrh_f3d *h) { return be_brick_grid(h->cpp.nx, h->cpp.ny, h->cpp.nz); }
 
-void op_bending_energy(nrh_f3d *h, double *out_device, hipStream_t stream) {
-    static const BeBasis B = make_be_basis();
+void op_bending_energy(nrh_f3d *h, double *out_device) {
     const BrickGrid bg = brick_grid(h);
     const unsigned nb = (unsigned)(bg.bx * bg.by * bg.bz);
-    h->partials.alloc(std::max<size_t>(h->partials.n, 2 * (size_t)nb + 64));
-    hipLaunchKernelGGL(k_be_value, dim3(nb), dim3(256), 0, stream ? stream : h->stream, h->cppPos.p, h->cpp.nx,
-                       h->cpp.ny, h->cpp.nz, bg, B, h->partials.p, h->maxBits.p + 6, 1.0 / (double)(3 * h->G),
-                       out_device);
+    h->partials.alloc(std::max<size_t>(h->partials.n, 3 * (size_t)nb));
+    hipLaunchKernelGGL(k_be_value, dim3(nb, 3), dim3(256), 0, h->stream, h->cppPos.p, h->cpp.nx, h->cpp.ny, h->cpp.nz, bg,
+                       h->partials.p);
     NRH_HIP(hipGetLastError());
+    op_bending_energy_sum(h, (int)(3 * nb), out_device);
 }
 
-void fork_side(nrh_f3d *h) {
-    if (!h->side) {
-        NRH_HIP(hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
-        NRH_HIP(hipEventCreateWithFlags(&h->evFork, hipEventDisableTiming));
-        NRH_HIP(hipEventCreateWithFlags(&h->evJoin, hipEventDisableTiming));
-    }
-    NRH_HIP(hipEventRecord(h->evFork, h->stream));
-    NRH_HIP(hipStreamWaitEvent(h->side, h->evFork, 0));
-}
-
-void join_side(nrh_f3d *h) {
-    NRH_HIP(hipEventRecord(h->evJoin, h->side));
-    NRH_HIP(hipStreamWaitEvent(h->stream, h->evJoin, 0));
-}
-
-void op_bending_energy_gradient_raw(nrh_f3d *h, hipStream_t stream) {
-    static const BeBasis B = make_be_basis();
-    const BrickGrid bg = brick_grid(h);
-    h->beGrad.alloc(3 * h->G);
-    hipLaunchKernelGGL(k_be_gradient_raw, dim3((unsigned)(bg.bx * bg.by * bg.bz)), dim3(256), 0, stream,
-                       h->cppPos.p, h->cpp.nx, h->cpp.ny, h->cpp.nz, bg, to_affine(h->cpp.xyz), B, h->beGrad.p);
+void op_bending_energy_sum(nrh_f3d *h, int n, double *out_device) {
+    hipLaunchKernelGGL(k_be_sum, dim3(1), dim3(256), 0, h->stream, (const double *)h->partials.p, n,
+                       1.0 / (double)(3 * h->G), out_device);
     NRH_HIP(hipGetLastError());
 }
 
 void op_bending_energy_gradient(nrh_f3d *h, float weight, bool trackMax) {
-    static const BeBasis B = make_be_basis();
     const BrickGrid bg = brick_grid(h);
-    uint32_t *mb = trackMax ? h->maxBits.p : nullptr;
     if (trackMax) op_fill_u32(h->maxBits.p, 1, 0u, h->stream);
-    const float ratio = weight / (float)h->G;
-    hipLaunchKernelGGL(k_be_gradient, dim3((unsigned)(bg.bx * bg.by * bg.bz)), dim3(256), 0, h->stream, h->cppPos.p,
-                       h->cpp.nx, h->cpp.ny, h->cpp.nz, bg, to_affine(h->cpp.xyz), B, ratio, h->nodeGrad.p, mb);
-    hipLaunchKernelGGL(k_round_trip, dim3(blocks_for(h->G)), dim3(256), 0, h->stream, h->cppPos.p, h->cpp.nx,
-                       h->cpp.ny, h->cpp.nz, to_affine(h->cpp.xyz));
+    h->beGrad.alloc(3 * h->G);
+    hipLaunchKernelGGL(k_be_gradient, dim3((unsigned)(bg.bx * bg.by * bg.bz), 3), dim3(256), 0, h->stream, h->cppPos.p,
+                       h->cpp.nx, h->cpp.ny, h->cpp.nz, bg, to_affine(h->cpp.xyz), h->beGrad.p);
+    hipLaunchKernelGGL(k_be_apply, dim3(blocks_for(h->G)), dim3(256), 0, h->stream, h->cppPos.p, h->cpp.nx, h->cpp.ny,
+                       h->cpp.nz, to_affine(h->cpp.xyz), (const float *)h->beGrad.p, weight / (float)h->G, h->nodeGrad.p,
+                       trackMax ? h->maxBits.p : nullptr);
     NRH_HIP(hipGetLastError());
     h->cppVersion++;  // the round trip may have changed the last bit of some points
 }
@@ -1681,20 +1550,31 @@ double read_scalar(nrh_f3d *h, const double *dev) {
 // ------------------------------------------------------------------ batches of pairs
 namespace {
 
-// The objective terms of each active pair into results[8 q ..]: NMI, H_r, H_f, H_rf, total, the
-// bending energy, the weighted value (reg_f3d::GetObjectiveFunctionValue with the linear energy
-// off), and the current max gradient length; mirrored into coherent host memory.
-__global__ void k_batch_values(const PairOps *__restrict__ P, int n, const int *active, const float *__restrict__ w,
-                               double *__restrict__ res, double *__restrict__ host) {
+// The objective terms of each active pair (a workgroup each) into results[8 q ..]: NMI, H_r, H_f,
+// H_rf, total, the bending energy, the weighted value (reg_f3d::GetObjectiveFunctionValue with the
+// linear energy off), and the current max gradient length; mirrored into coherent host memory.
+// sumBe: the bending energy is summed from the partials of the launch before.
+__global__ void __launch_bounds__(256)
+k_batch_values(const PairOps *__restrict__ P, const int *active, int sumBe, const float *__restrict__ w,
+               double *__restrict__ res, double *__restrict__ host) {
 #pragma clang fp contract(off)
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n || skip_pair(active, q)) return;
+    __shared__ double red[16];
+    const int q = blockIdx.x;
+    if (skip_pair(active, q)) return;
     const PairOps& o = P[q];
+    double be = 0;
+    if (sumBe) {
+        const double t = sum_partials_256(o.partials, 3 * o.beBlocks, red);
+        if (threadIdx.x == 0) *o.beOut = be = t * o.beScale;
+    } else if (threadIdx.x == 0) {
+        be = *o.beOut;
+    }
+    if (threadIdx.x != 0) return;
     const double simW = (double)w[2 * q], beW = (double)w[2 * q + 1];
     double r[kBatchResults];
     r[0] = o.ent[4];
     for (int k = 0; k < 4; ++k) r[1 + k] = o.ent[k];
-    r[5] = beW > 0 ? *o.beOut : 0.0;
+    r[5] = beW > 0 ? be : 0.0;
     const double wMeasure = simW > 0 ? simW * r[0] : 0.0;
     const double wBE = beW > 0 ? beW * r[5] : 0.0;
     r[6] = wMeasure - wBE;
@@ -1720,7 +1600,8 @@ void batch_ops_setup(nrh_batch *b) {
         const int nb = bg.bx * bg.by * bg.bz;
         const size_t n3 = 3 * h->G;
         const int cgBlocks = (int)std::min(blocks_for(n3), 512u);
-        h->partials.alloc(std::max<size_t>(h->partials.n, 2 * (size_t)std::max(nb, cgBlocks) + 64));
+        h->partials.alloc(std::max(h->partials.n, std::max(3 * (size_t)nb, 2 * (size_t)cgBlocks + 64)));
+        h->beGrad.alloc(3 * h->G);
         PairOps o{};
         o.cpp = h->cppPos.p;
         o.best = h->best.p;
@@ -1738,7 +1619,7 @@ void batch_ops_setup(nrh_batch *b) {
         o.beRatio = h->params.be_weight / (float)h->G;
         o.beScale = 1.0 / (double)(3 * h->G);
         o.partials = h->partials.p;
-        o.beTicket = h->maxBits.p + 6;
+        o.beGrad = h->beGrad.p;
         o.beOut = h->scalars.p + 0;
         o.maxBits = h->maxBits.p;
         o.maxLen = h->scalars.p + 1;
@@ -1783,18 +1664,15 @@ void batch_finalize(nrh_batch *b, const int *active) {
 }
 
 void batch_be_value(nrh_batch *b, const int *active) {
-    static const BeBasis B = make_be_basis();
-    hipLaunchKernelGGL(k_be_value_batch, dim3(b->nBE), dim3(256), 0, b->stream, (const PairOps *)b->pairOps.p,
-                       b->itBE.p, B, active);
+    hipLaunchKernelGGL(k_be_value_batch, dim3(b->nBE, 3), dim3(256), 0, b->stream, (const PairOps *)b->pairOps.p,
+                       b->itBE.p, active);
     NRH_HIP(hipGetLastError());
 }
 
 void batch_be_gradient(nrh_batch *b, const int *active) {
-    static const BeBasis B = make_be_basis();
     const PairOps *P = (const PairOps *)b->pairOps.p;
     hipLaunchKernelGGL(k_zero_max_bits_batch, dim3((b->P + 255) / 256), dim3(256), 0, b->stream, P, b->P, active);
-    hipLaunchKernelGGL(k_be_gradient_batch, dim3(b->nBE), dim3(256), 0, b->stream, P, b->itBE.p, B, active);
-    hipLaunchKernelGGL(k_round_trip_batch, dim3(b->nG), dim3(256), 0, b->stream, P, b->itG.p, active);
+    hipLaunchKernelGGL(k_be_gradient_batch, dim3(b->nBE, 3), dim3(256), 0, b->stream, P, b->itBE.p, active);
     NRH_HIP(hipGetLastError());
 }
 
@@ -1825,9 +1703,9 @@ void batch_copy_dof(nrh_batch *b, const int *active, bool toBest) {
     NRH_HIP(hipGetLastError());
 }
 
-void batch_values(nrh_batch *b, const int *active) {
-    hipLaunchKernelGGL(k_batch_values, dim3((b->P + 63) / 64), dim3(64), 0, b->stream, (const PairOps *)b->pairOps.p,
-                       b->P, active, b->weights.p, b->results.p, b->publishedDev);
+void batch_values(nrh_batch *b, const int *active, bool sumBe) {
+    hipLaunchKernelGGL(k_batch_values, dim3(b->P), dim3(256), 0, b->stream, (const PairOps *)b->pairOps.p, active,
+                       sumBe ? 1 : 0, b->weights.p, b->results.p, b->publishedDev);
     NRH_HIP(hipGetLastError());
 }
 
