@@ -5,7 +5,7 @@
 // (reg-lib/_reg_aladin.cpp:302-313) is three launches on the handle's stream with the current
 // matrix kept in device memory:
 //   k_affine_warp   field = (A * ref.sto_xyz) * voxel in FP64, trilinear warp of the floating image
-//   k_block_match   one workgroup per active 4x4x4 block, one lane per capture offset (343)
+//   k_block_match   five active 4x4x4 blocks a workgroup, a lane per (y, z) of their capture offsets
 //   k_lts           one 1024-lane workgroup: compaction, FP64 moment fits, radix-select trimming
 // Block variances for the active-block choice are computed on the device; their heap-sort
 // ranking runs on the host because its tie order is part of the reference's result.
@@ -39,7 +39,7 @@ struct nrh_aladin {
     int nb[3] = { 0, 0, 0 };
     int totalBlocks = 0, activeBlocks = 0;
     std::vector<int> totalBlock;      // _reg_blockMatchingParam::totalBlock
-    nrh::DevBuf<int> activeList;      // rank -> block index
+    nrh::DevBuf<int2> activeList;     // (block index, rank), in block order
     nrh::DevBuf<float> refPos, warpPos;
     nrh::DevBuf<float> matrix;        // current affine, 16 floats row-major
     nrh::DevBuf<int> counters;        // [0] defined blocks of the last matching, [1] LTS status,
@@ -53,7 +53,6 @@ namespace nrh {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kMatchThreads = 384;  // 343 capture offsets rounded up to whole waves
 constexpr int kLtsThreads = 1024;
 constexpr int kLtsUnroll = 4;  // points per thread whose loads the LTS passes issue together
 
@@ -177,114 +176,270 @@ k_affine_warp(const float *__restrict__ flo, int fnx, int fny, int fnz, Affine f
 }
 
 // ------------------------------------------------------------------ block matching
-// block_matching_method3D<float> (reg-lib/cpu/_reg_blockMatching.cpp:455-690).  Workgroup =
-// one active block (grid = active block count, in rank order); lane t < 343 = capture offset
-// (l, m, n) = (t % 7, t / 7 % 7, t / 49) - 3, the reference's loop order.  Each lane keeps its 64
-// warped values in registers and runs the reference's two float passes (means, then variances
-// and covariance) in voxel order; wave 0 then replays the sequential "cc > best -> best =
-// cc + 1e-7" rule with ballots, which gives the same winner as the reference's scan.
+// block_matching_method3D<float> (reg-lib/cpu/_reg_blockMatching.cpp:455-690).  A workgroup takes
+// kMatchBlocks active blocks (neighbours: the list is in block order, as undefined values come in clusters); a lane takes one (m, n) of a block's 7 x 7 capture
+// offsets along y and z and all 7 along x, so the 10 warped values of a row are read from LDS once for
+// the 28 products that they enter.  Each offset runs the reference's two float passes (means, then
+// variances and covariance) in voxel order; a wave per block then replays the sequential
+// "cc > best -> best = cc + 1e-7" rule with ballots, which gives the same winner as the reference's
+// scan over offsets (l, m, n) = (o % 7, o / 7 % 7, o / 49) - 3.
+//
+// Bound by vector instructions: 343 offsets x 64 voxels x 6 for a block whose values are all defined
+// (its mean and variance are the same for every offset and come from one lane), 16 with a check of
+// each value otherwise; a wave takes the short way when every block it works on allows.  One offset
+// a lane, both checks always and an atomic per block on the count of defined blocks: 254 us for the
+// 16384 blocks of 128^3; so, 93 us (in rank order, which scatters the blocks with undefined values, and
+// with the coordinates of each staged value found by division, 179 us).  5 blocks fill 245 of 256 lanes.
+constexpr int kMatchBlocks = 5;
+constexpr int kMatchThreads = 256;
+
+struct MatchShared {
+    float W[kMatchBlocks][1000];    // warped values, 3 voxels around the block
+    float R[kMatchBlocks][68];      // reference values (NaN: undefined or masked)
+    float rt[kMatchBlocks][64];     // reference values less their mean (blocks without NaN)
+    float rv[kMatchBlocks];         // and the sum of their squares
+    float cc[kMatchBlocks][343];
+    int rank[kMatchBlocks];
+    int org[kMatchBlocks][3];       // first voxel
+    int bad[kMatchBlocks];          // an undefined value among R or W
+    int defined;
+};
+
+// cc of the 7 offsets along x, every value of the block and its surroundings defined.
+__device__ __forceinline__ void match_defined(const MatchShared& S, int blk, int m, int n, float (&cc)[7]) {
+#pragma clang fp contract(off)
+    const float *w0 = S.W[blk] + n * 100 + m * 10;  // rows start on even indices: pairs are aligned
+    float wm[7] = {};
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            float w[10];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                const float2 v = *reinterpret_cast<const float2 *>(w0 + z * 100 + y * 10 + 2 * k);
+                w[2 * k] = v.x;
+                w[2 * k + 1] = v.y;
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int l = 0; l < 7; ++l) wm[l] += w[l + x];
+        }
+    float wv[7] = {}, c[7] = {};
+#pragma unroll
+    for (int l = 0; l < 7; ++l) wm[l] /= 64.f;
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            float w[10];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                const float2 v = *reinterpret_cast<const float2 *>(w0 + z * 100 + y * 10 + 2 * k);
+                w[2 * k] = v.x;
+                w[2 * k + 1] = v.y;
+            }
+            const float4 r4 = *reinterpret_cast<const float4 *>(&S.rt[blk][z * 16 + y * 4]);
+            const float rt[4] = { r4.x, r4.y, r4.z, r4.w };
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int l = 0; l < 7; ++l) {
+                    const float wt = w[l + x] - wm[l];
+                    wv[l] += wt * wt;
+                    c[l] += rt[x] * wt;
+                }
+        }
+    const float rv = S.rv[blk];
+#pragma unroll
+    for (int l = 0; l < 7; ++l) cc[l] = (rv * wv[l]) > 0.f ? fabsf(c[l] / sqrtf(rv * wv[l])) : 0.f;
+}
+
+// The same over the pairs whose two values are defined (an undefined one adds 0), more than 32 of them.
+__device__ __forceinline__ void match_checked(const MatchShared& S, int blk, int m, int n, float (&cc)[7]) {
+#pragma clang fp contract(off)
+    const float *w0 = S.W[blk] + n * 100 + m * 10;
+    // a row's values and which of them are defined: one comparison each, for all that they enter
+    float w[10], r[4];
+    bool wok[10], rok[4];
+    auto row = [&](int q) {
+        const float *p = w0 + (q >> 2) * 100 + (q & 3) * 10;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const float2 v = *reinterpret_cast<const float2 *>(p + 2 * k);
+            w[2 * k] = v.x;
+            w[2 * k + 1] = v.y;
+        }
+        const float4 v = *reinterpret_cast<const float4 *>(&S.R[blk][q * 4]);
+        r[0] = v.x;
+        r[1] = v.y;
+        r[2] = v.z;
+        r[3] = v.w;
+#pragma unroll
+        for (int k = 0; k < 10; ++k) wok[k] = w[k] == w[k];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) rok[x] = r[x] == r[x];
+    };
+    float rm[7] = {}, wm[7] = {}, cnt[7] = {};
+    for (int q = 0; q < 16; ++q) {
+        row(q);
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int l = 0; l < 7; ++l) {
+                const bool ok = rok[x] && wok[l + x];
+                rm[l] += ok ? r[x] : 0.f;
+                wm[l] += ok ? w[l + x] : 0.f;
+                cnt[l] += ok ? 1.f : 0.f;
+            }
+    }
+    float rv[7] = {}, wv[7] = {}, c[7] = {};
+#pragma unroll
+    for (int l = 0; l < 7; ++l) {
+        rm[l] /= cnt[l];
+        wm[l] /= cnt[l];
+    }
+    for (int q = 0; q < 16; ++q) {
+        row(q);
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int l = 0; l < 7; ++l) {
+                const bool ok = rok[x] && wok[l + x];
+                const float rt = ok ? r[x] - rm[l] : 0.f, wt = ok ? w[l + x] - wm[l] : 0.f;
+                rv[l] += rt * rt;
+                wv[l] += wt * wt;
+                c[l] += rt * wt;
+            }
+    }
+#pragma unroll
+    for (int l = 0; l < 7; ++l) {
+        const float v = (rv[l] * wv[l]) > 0.f ? fabsf(c[l] / sqrtf(rv[l] * wv[l])) : 0.f;
+        cc[l] = cnt[l] > 32.f ? v : -1.f;
+    }
+}
+
 __global__ void __launch_bounds__(kMatchThreads)
 k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, const int *__restrict__ mask,
-              int nx, int ny, int nz, int nbx, int nby, const int *__restrict__ activeList, Affine xyz,
+              int nx, int ny, int nz, int nbx, int nby, const int2 *__restrict__ activeList, int nActive, Affine xyz,
               float *__restrict__ refPos, float *__restrict__ warpPos, int *__restrict__ definedCount) {
 #pragma clang fp contract(off)
-    __shared__ float sR[64];
-    __shared__ float sW[1000];
-    __shared__ float sCC[kMatchThreads];
-    const int rank = blockIdx.x;
-    const int b = activeList[rank];
-    const int bi = b % nbx, bj = (b / nbx) % nby, bk = b / (nbx * nby);
-    const int x0 = 4 * bi, y0 = 4 * bj, z0 = 4 * bk;
-    const int t = threadIdx.x;
+    __shared__ __align__(16) MatchShared S;
+    const int t = threadIdx.x, first = blockIdx.x * kMatchBlocks, nb = min(kMatchBlocks, nActive - first);
     const float qnan = __builtin_nanf("");
-    if (t < 64) {
-        const int x = x0 + (t & 3), y = y0 + ((t >> 2) & 3), z = z0 + (t >> 4);
-        float v = qnan;
-        if (x < nx && y < ny && z < nz) {
-            const size_t i = ((size_t)z * ny + y) * nx + x;
-            const float r = ref[i];
-            if (r == r && (!mask || mask[i] > -1)) v = r;
-        }
-        sR[t] = v;
+    if (t < kMatchBlocks) {
+        const int2 a = activeList[first + min(t, nb - 1)];  // blocks past the last repeat it, unused
+        S.rank[t] = a.y;
+        S.org[t][0] = 4 * (a.x % nbx);
+        S.org[t][1] = 4 * ((a.x / nbx) % nby);
+        S.org[t][2] = 4 * (a.x / (nbx * nby));
+        S.bad[t] = 0;
     }
-    for (int q = t; q < 1000; q += kMatchThreads) {
-        const int x = x0 - 3 + q % 10, y = y0 - 3 + (q / 10) % 10, z = z0 - 3 + q / 100;
-        float v = qnan;
-        if (x > -1 && x < nx && y > -1 && y < ny && z > -1 && z < nz) v = warped[((size_t)z * ny + y) * nx + x];
-        sW[q] = v;
+    if (t == 0) S.defined = 0;
+    __syncthreads();
+    {
+        // the warped values first, all loads in flight before the first is stored: 50 threads a block,
+        // each two columns (x, y) and (x, y + 5) of its 10 slices
+        const int wb = min(t / 50, kMatchBlocks - 1), p = t % 50;
+        const int x = S.org[wb][0] - 3 + p % 10, y = S.org[wb][1] - 3 + p / 10, z0 = S.org[wb][2] - 3;
+        const bool in0 = x > -1 && x < nx && y > -1 && y < ny, in1 = x > -1 && x < nx && y + 5 > -1 && y + 5 < ny;
+        const float *c0 = warped + (in0 ? (size_t)y * nx + x : 0), *c1 = warped + (in1 ? (size_t)(y + 5) * nx + x : 0);
+        const size_t slice = (size_t)nx * ny;
+        float v[20];
+#pragma unroll
+        for (int u = 0; u < 10; ++u) {
+            const int z = min(max(z0 + u, 0), nz - 1);
+            v[u] = c0[z * slice];
+            v[10 + u] = c1[z * slice];
+            const bool inz = z == z0 + u;
+            if (!in0 || !inz) v[u] = qnan;
+            if (!in1 || !inz) v[10 + u] = qnan;
+        }
+        for (int i = t; i < kMatchBlocks * 64; i += kMatchThreads) {
+            const int blk = i >> 6, a = i & 63;
+            const int rx = S.org[blk][0] + (a & 3), ry = S.org[blk][1] + ((a >> 2) & 3), rz = S.org[blk][2] + (a >> 4);
+            float r = qnan;
+            if (rx < nx && ry < ny && rz < nz) {
+                const size_t k = ((size_t)rz * ny + ry) * nx + rx;
+                if (!mask || mask[k] > -1) r = ref[k];
+            }
+            S.R[blk][a] = r;
+            if (!(r == r)) S.bad[blk] = 1;
+        }
+        if (t < 50 * kMatchBlocks) {
+            bool bad = false;
+#pragma unroll
+            for (int u = 0; u < 10; ++u) {
+                S.W[wb][u * 100 + p] = v[u];
+                S.W[wb][u * 100 + 50 + p] = v[10 + u];
+                bad = bad || !(v[u] == v[u]) || !(v[10 + u] == v[10 + u]);
+            }
+            if (bad) S.bad[wb] = 1;
+        }
     }
     __syncthreads();
-    float cc = -1.f;
-    if (t < 343) {
-        const int l = t % 7, m = (t / 7) % 7, n = t / 49;
-        // the lane's 64 warped values are read from LDS in each pass (constant offsets from one
-        // base) rather than held in registers: the kernel then fits several workgroups per CU
-        const float *wb = sW + n * 100 + m * 10 + l;
-        auto W = [&](int a) { return wb[(a >> 4) * 100 + ((a >> 2) & 3) * 10 + (a & 3)]; };
-        float rm = 0.f, wm = 0.f, cnt = 0.f;
-#pragma unroll
+    if (t < kMatchBlocks && !S.bad[t]) {
+        const float *R = S.R[t];
+        float rm = 0.f, rv = 0.f;
+#pragma unroll 16
+        for (int a = 0; a < 64; ++a) rm += R[a];
+        rm /= 64.f;
+#pragma unroll 16
         for (int a = 0; a < 64; ++a) {
-            const float r = sR[a];
-            if (r == r && W(a) == W(a)) {
-                rm += r;
-                wm += W(a);
-                cnt += 1.f;
-            }
+            const float rt = R[a] - rm;
+            S.rt[t][a] = rt;
+            rv += rt * rt;
         }
-        if (cnt > 32.f) {
-            asm volatile("" ::: "memory");  // the second pass reads LDS again
-            rm /= cnt;
-            wm /= cnt;
-            float rv = 0.f, wv = 0.f, c = 0.f;
-#pragma unroll
-            for (int a = 0; a < 64; ++a) {
-                const float r = sR[a];
-                if (r == r && W(a) == W(a)) {
-                    const float rt = r - rm, wt = W(a) - wm;
-                    rv += rt * rt;
-                    wv += wt * wt;
-                    c += rt * wt;
-                }
-            }
-            cc = (rv * wv) > 0.f ? fabsf(c / sqrtf(rv * wv)) : 0.f;
-        }
+        S.rv[t] = rv;
     }
-    sCC[t] = cc;
     __syncthreads();
-    if (t >= 64) return;
-    float best = 0.f;
-    int win = -1;
-    for (int c = 0; c < kMatchThreads / 64; ++c) {
-        const int o = c * 64 + t;
-        const float v = o < 343 ? sCC[o] : -1.f;
-        unsigned long long mk = __ballot(v > best);
-        while (mk) {
-            const int first = __ffsll((long long)mk) - 1;
-            best = __shfl(v, first, 64) + 1.0e-7f;
-            win = c * 64 + first;
-            mk = __ballot(v > best && t > first);
+    {
+        const int blk = min(t / 49, kMatchBlocks - 1), o = t % 49, m = o % 7, n = o / 7;
+        float cc[7];
+        if (__any(S.bad[blk])) match_checked(S, blk, m, n, cc);
+        else match_defined(S, blk, m, n, cc);
+        if (t < kMatchBlocks * 49)
+            for (int l = 0; l < 7; ++l) S.cc[blk][n * 49 + m * 7 + l] = cc[l];
+    }
+    __syncthreads();
+    for (int blk = t >> 6; blk < nb; blk += kMatchThreads / 64) {
+        const int lane = t & 63;
+        float best = 0.f;
+        int win = -1;
+        for (int c = 0; c < (343 + 63) / 64; ++c) {
+            const int o = c * 64 + lane;
+            const float v = o < 343 ? S.cc[blk][o] : -1.f;
+            unsigned long long mk = __ballot(v > best);
+            while (mk) {
+                const int f = __ffsll((long long)mk) - 1;
+                best = __shfl(v, f, 64) + 1.0e-7f;
+                win = c * 64 + f;
+                mk = __ballot(v > best && lane > f);
+            }
         }
+        if (lane != 0) continue;
+        const int rank = S.rank[blk];
+        const float cx = (float)S.org[blk][0], cy = (float)S.org[blk][1], cz = (float)S.org[blk][2];
+        float dx = qnan, dy = 0.f, dz = 0.f;
+        if (win >= 0) {
+            dx = (float)(win % 7 - 3);
+            dy = (float)((win / 7) % 7 - 3);
+            dz = (float)(win / 49 - 3);
+            atomicAdd(&S.defined, 1);
+        }
+        dx += cx;
+        dy += cy;
+        dz += cz;
+        const float3 rp = affine_apply_d(xyz, cx, cy, cz);
+        const float3 wp = affine_apply_d(xyz, dx, dy, dz);
+        refPos[3 * rank + 0] = rp.x;
+        refPos[3 * rank + 1] = rp.y;
+        refPos[3 * rank + 2] = rp.z;
+        warpPos[3 * rank + 0] = wp.x;
+        warpPos[3 * rank + 1] = wp.y;
+        warpPos[3 * rank + 2] = wp.z;
     }
-    if (t != 0) return;
-    const float cx = (float)x0, cy = (float)y0, cz = (float)z0;
-    float dx = qnan, dy = 0.f, dz = 0.f;
-    if (win >= 0) {
-        dx = (float)(win % 7 - 3);
-        dy = (float)((win / 7) % 7 - 3);
-        dz = (float)(win / 49 - 3);
-    }
-    dx += cx;
-    dy += cy;
-    dz += cz;
-    const float3 rp = affine_apply_d(xyz, cx, cy, cz);
-    const float3 wp = affine_apply_d(xyz, dx, dy, dz);
-    refPos[3 * rank + 0] = rp.x;
-    refPos[3 * rank + 1] = rp.y;
-    refPos[3 * rank + 2] = rp.z;
-    warpPos[3 * rank + 0] = wp.x;
-    warpPos[3 * rank + 1] = wp.y;
-    warpPos[3 * rank + 2] = wp.z;
-    if (win >= 0) atomicAdd(definedCount, 1);
+    __syncthreads();
+    if (t == 0 && S.defined > 0) atomicAdd(definedCount, S.defined);
 }
 
 // ------------------------------------------------------------------ LTS
@@ -1028,16 +1183,15 @@ void select_blocks(nrh_aladin *h) {
     for (int b = 0; b < total; ++b) ix[b] = b;
     heap_sort_indexed(v, ix);
     h->totalBlock.assign(total, -1);
-    std::vector<int> list(std::max(active, 0));
-    for (int r = 0; r < active; ++r) {
-        const int b = ix[total - 1 - r];
-        h->totalBlock[b] = r;
-        list[r] = b;
-    }
+    for (int r = 0; r < active; ++r) h->totalBlock[ix[total - 1 - r]] = r;
+    std::vector<int2> list;  // (block, rank) in block order
+    list.reserve(std::max(active, 0));
+    for (int b = 0; b < total; ++b)
+        if (h->totalBlock[b] >= 0) list.push_back(make_int2(b, h->totalBlock[b]));
     NRH_REQUIRE(active >= 2, NRH_ERR_NUMERIC, "There are less than 2 active blocks");
     h->activeBlocks = active;
     h->activeList.alloc(active);
-    NRH_HIP(hipMemcpyAsync(h->activeList.p, list.data(), active * sizeof(int), hipMemcpyHostToDevice, h->stream));
+    NRH_HIP(hipMemcpyAsync(h->activeList.p, list.data(), active * sizeof(int2), hipMemcpyHostToDevice, h->stream));
     h->refPos.alloc(3 * (size_t)active);
     h->warpPos.alloc(3 * (size_t)active);
     h->ltsP.alloc(3 * (size_t)active);
@@ -1061,9 +1215,9 @@ void launch_warp(nrh_aladin *h) {
 
 void launch_block_matching(nrh_aladin *h) {
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, h->stream, h->counters.p);
-    hipLaunchKernelGGL(k_block_match, dim3(h->activeBlocks), dim3(kMatchThreads), 0, h->stream, h->refImg.p,
-                       h->warped.p, h->mask.p, h->ref.nx, h->ref.ny, h->ref.nz, h->nb[0], h->nb[1], h->activeList.p,
-                       to_affine(h->ref.xyz), h->refPos.p, h->warpPos.p, h->counters.p);
+    hipLaunchKernelGGL(k_block_match, dim3((h->activeBlocks + kMatchBlocks - 1) / kMatchBlocks), dim3(kMatchThreads), 0,
+                       h->stream, h->refImg.p, h->warped.p, h->mask.p, h->ref.nx, h->ref.ny, h->ref.nz, h->nb[0], h->nb[1],
+                       h->activeList.p, h->activeBlocks, to_affine(h->ref.xyz), h->refPos.p, h->warpPos.p, h->counters.p);
     NRH_HIP(hipGetLastError());
 }
 
