@@ -6,7 +6,7 @@
 // matrix kept in device memory:
 //   k_affine_warp   field = (A * ref.sto_xyz) * voxel in FP64, trilinear warp of the floating image
 //   k_block_match   five active 4x4x4 blocks a workgroup, a lane per (y, z) of their capture offsets
-//   k_lts           one 1024-lane workgroup: compaction, FP64 moment fits, radix-select trimming
+//   k_lts           one workgroup: compaction, FP64 moment fits, radix-select trimming
 // Block variances for the active-block choice are computed on the device; their heap-sort
 // ranking runs on the host because its tie order is part of the reference's result.
 
@@ -53,19 +53,23 @@ namespace nrh {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kLtsThreads = 1024;
-constexpr int kLtsUnroll = 4;  // points per thread whose loads the LTS passes issue together
+constexpr int kLtsThreads = 512;
+constexpr int kLtsUnroll = 8;  // points per thread whose loads the LTS passes issue together
 
 struct Mat4 {
     float m[16];
 };
 
-__device__ __forceinline__ float3 mat44_mul_f(const float *m, float x, float y, float z) {
+// The reference's products and sums in double; a product of two floats is exact there, so the fused
+// multiply-adds round as its separate operations do.
+template<class T>
+__device__ __forceinline__ float3 mat44_mul_f(const T *m, float x, float y, float z) {
 #pragma clang fp contract(off)
+    const double X = (double)x, Y = (double)y, Z = (double)z;
     float3 r;
-    r.x = (float)((double)m[0] * (double)x + (double)m[1] * (double)y + (double)m[2] * (double)z + (double)m[3]);
-    r.y = (float)((double)m[4] * (double)x + (double)m[5] * (double)y + (double)m[6] * (double)z + (double)m[7]);
-    r.z = (float)((double)m[8] * (double)x + (double)m[9] * (double)y + (double)m[10] * (double)z + (double)m[11]);
+    r.x = (float)(fma((double)m[2], Z, fma((double)m[1], Y, (double)m[0] * X)) + (double)m[3]);
+    r.y = (float)(fma((double)m[6], Z, fma((double)m[5], Y, (double)m[4] * X)) + (double)m[7]);
+    r.z = (float)(fma((double)m[10], Z, fma((double)m[9], Y, (double)m[8] * X)) + (double)m[11]);
     return r;
 }
 
@@ -443,25 +447,62 @@ k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, c
 }
 
 // ------------------------------------------------------------------ LTS
+// Four words of padding after every 32: the lanes of the wave that selects each read 32 of the
+// histogram's, which without it lie in the same banks for all.
+__device__ __forceinline__ uint32_t lts_bin(uint32_t b) { return b + ((b >> 5) << 2); }
+
+template<int NT>
 struct alignas(16) LtsShared {
-    double red[kLtsThreads / 64][24];
+    double red[NT / 64][24];
     double out[24];
-    double fit[21];  // the fit's centred moments and means
-    uint32_t hist[2048];
-    int wave[kLtsThreads / 64];
+    double kept[24];  // the kept points' sums: p, q, count, p_a p_b (00 01 02 11 12 22), p_a q_b
+    double fit[21];   // the fit's centred moments and means
+    uint32_t hist[2048 + 256];                  // bin b at lts_bin(b)
+    uint32_t list[NT / 64][128];                // per wave: points that enter or leave the kept set
+    int wave[kLtsUnroll][NT / 64];
     float M[16], last[16];
     int scal[4];
-    double dist;
 };
+
+template<int CTRL>
+__device__ __forceinline__ double dpp_double(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+__device__ __forceinline__ double uniform_double(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// a + b over the pairs of lanes that differ in bit 5 (ROWS: bit 4): the lanes with the bit clear get
+// a's sum, the others b's.
+template<bool ROWS>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const unsigned long long ua = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long ub = (unsigned long long)__double_as_longlong(b);
+    auto swap = [](uint32_t x, uint32_t y) {
+        if constexpr (ROWS) return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        else return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    };
+    const auto lo = swap((uint32_t)ua, (uint32_t)ub), hi = swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi[0] << 32 | lo[0])) +
+           __longlong_as_double((long long)((unsigned long long)hi[1] << 32 | lo[1]));
+}
 
 // Sum of K doubles over the workgroup in a fixed order; the result lands in s.out[0..K).
 // Inside a wave the values are halved at each exchange: the lanes whose exchange bit is clear keep
 // the lower half of the (zero-padded, power-of-two) set and send the upper half, the others the
 // reverse, so the wave makes W/2 + W/4 + ... + 1 exchanges instead of K per lane bit; after log2 W
 // of them lane l holds value (l >> (6 - log2 W)) summed over its group, and the remaining lane bits
-// are summed by plain exchanges.
-template<int K>
-__device__ void wg_sum(double (&v)[K], LtsShared& s) {
+// are summed by plain exchanges.  The exchanges are lane swaps and data-parallel moves (lane l with
+// l ^ 32, l ^ 16, l ^ 8, 7 - l of its eight, l ^ 2, l ^ 1): through LDS, 16 waves took 4800 cycles
+// for 23 values.
+template<int K, int NT>
+__device__ void wg_sum(double (&v)[K], LtsShared<NT>& s) {
     static_assert(K <= 32, "at most 32 values");
     constexpr int W = K <= 8 ? 8 : K <= 16 ? 16 : 32;
     constexpr int LW = W == 8 ? 3 : W == 16 ? 4 : 5;
@@ -470,24 +511,35 @@ __device__ void wg_sum(double (&v)[K], LtsShared& s) {
 #pragma unroll
     for (int k = 0; k < W; ++k) a[k] = k < K ? v[k] : 0.0;
 #pragma unroll
-    for (int st = 0; st < LW; ++st) {
-        const int off = 32 >> st, half = W >> (st + 1);
-        const bool upper = (lane & off) != 0;
+    for (int j = 0; j < W / 2; ++j) a[j] = swap_add<false>(a[j], a[j + W / 2]);
 #pragma unroll
-        for (int j = 0; j < half; ++j) {
+    for (int j = 0; j < W / 4; ++j) a[j] = swap_add<true>(a[j], a[j + W / 4]);
+    auto halve = [&](auto move, int half, bool upper) {
+#pragma unroll
+        for (int j = 0; j < W / 8; ++j) {
+            if (j >= half) break;
             const double send = upper ? a[j] : a[j + half];
             const double keep = upper ? a[j + half] : a[j];
-            a[j] = keep + __shfl_xor(send, off, 64);
+            a[j] = keep + move(send);
         }
-    }
-#pragma unroll
-    for (int off = 32 >> LW; off > 0; off >>= 1) a[0] += __shfl_xor(a[0], off, 64);
-    const int idx = (lane >> (6 - LW)) & (W - 1);
+    };
+    auto ror8 = [](double x) { return dpp_double<0x128>(x); };
+    auto mirror8 = [](double x) { return dpp_double<0x141>(x); };
+    auto xor2 = [](double x) { return dpp_double<0x4e>(x); };
+    auto xor1 = [](double x) { return dpp_double<0xb1>(x); };
+    halve(ror8, W / 8, (lane & 8) != 0);
+    if constexpr (LW > 3) halve(mirror8, W / 16, (lane & 4) != 0);
+    else a[0] += mirror8(a[0]);
+    if constexpr (LW > 4) halve(xor2, W / 32, (lane & 2) != 0);
+    else a[0] += xor2(a[0]);
+    a[0] += xor1(a[0]);
+    const int idx = lane >> (6 - LW);
     if ((lane & ((1 << (6 - LW)) - 1)) == 0 && idx < K) s.red[wv][idx] = a[0];
     __syncthreads();
     if (threadIdx.x < K) {
         double r = 0;
-        for (int w = 0; w < kLtsThreads / 64; ++w) r += s.red[w][threadIdx.x];
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) r += s.red[w][threadIdx.x];
         s.out[threadIdx.x] = r;
     }
     __syncthreads();
@@ -518,22 +570,28 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v) {
     return (uint32_t)incl - v;
 }
 
-// Exclusive prefix of a 0/1 flag over the workgroup (lane order = index order); returns the
-// position of this lane and writes the chunk total to *total (uniform).
-__device__ int wg_scan(bool flag, LtsShared& s, int *total) {
+// Positions of U chunks' flags over the workgroup (chunk after chunk, lane order = index order) into
+// pos; returns their number (uniform).
+template<int U, int NT>
+__device__ __forceinline__ int wg_scan(const bool (&flag)[U], int (&pos)[U], LtsShared<NT>& s) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const unsigned long long bal = __ballot(flag);
-    const int inWave = __popcll(bal & ((1ull << lane) - 1ull));
-    if (lane == 0) s.wave[wv] = __popcll(bal);
-    __syncthreads();
-    int before = 0, all = 0;
-    for (int w = 0; w < kLtsThreads / 64; ++w) {
-        if (w < wv) before += s.wave[w];
-        all += s.wave[w];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const unsigned long long bal = __ballot(flag[u]);
+        pos[u] = __popcll(bal & ((1ull << lane) - 1ull));
+        if (lane == 0) s.wave[u][wv] = __popcll(bal);
     }
     __syncthreads();
-    *total = all;
-    return before + inWave;
+    int all = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) {
+            if (w == wv) pos[u] += all;
+            all += s.wave[u][w];
+        }
+    __syncthreads();
+    return all;
 }
 
 // H = U S V^T of a 3x3 matrix by one-sided Jacobi rotations; singular values descending.
@@ -545,7 +603,7 @@ __device__ void svd3(const double H[3][3], double U[3][3], double V[3][3]) {
             V[i][j] = i == j ? 1.0 : 0.0;
         }
     for (int sweep = 0; sweep < 60; ++sweep) {
-        double off = 0;
+        bool rotated = false;
         // unrolled: every index is a compile-time constant, so A and V stay in registers
 #pragma unroll
         for (int p = 0; p < 2; ++p)
@@ -555,9 +613,10 @@ __device__ void svd3(const double H[3][3], double U[3][3], double V[3][3]) {
                 const double b = A[0][q] * A[0][q] + A[1][q] * A[1][q] + A[2][q] * A[2][q];
                 const double c = A[0][p] * A[0][q] + A[1][p] * A[1][q] + A[2][p] * A[2][q];
                 if (fabs(c) <= 1e-300 || fabs(c) <= 1e-15 * sqrt(a * b)) continue;
-                off = fmax(off, fabs(c) / sqrt(a * b));
-                const double zeta = (b - a) / (2 * c);
-                const double tn = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
+                rotated = true;
+                // tan of the rotation, the smaller root of t^2 + t (b - a) / c - 1 = 0
+                const double d = b - a, h = sqrt(d * d + 4 * c * c);
+                const double tn = 2 * c / (d >= 0 ? d + h : d - h);
                 const double cs = 1 / sqrt(1 + tn * tn), sn = cs * tn;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -569,33 +628,39 @@ __device__ void svd3(const double H[3][3], double U[3][3], double V[3][3]) {
                     V[i][q] = sn * vx + cs * vy;
                 }
             }
-        if (off < 1e-15) break;
+        if (!rotated) break;
     }
     double sv[3];
-    int o[3] = { 0, 1, 2 };
+#pragma unroll
     for (int j = 0; j < 3; ++j) sv[j] = sqrt(A[0][j] * A[0][j] + A[1][j] * A[1][j] + A[2][j] * A[2][j]);
-    for (int i = 0; i < 3; ++i)  // sort column order by descending singular value
-        for (int j = i + 1; j < 3; ++j)
-            if (sv[o[j]] > sv[o[i]]) {
-                const int tmp = o[i];
-                o[i] = o[j];
-                o[j] = tmp;
-            }
-    double V2[3][3];
-    for (int j = 0; j < 3; ++j)
+    // columns by descending singular value: exchanges of columns known at compile time
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        const int p = e == 1 ? 1 : 0, q = p + 1;
+        const bool swap = sv[q] > sv[p];
+        auto exchange = [&](double& x, double& y) {
+            const double t = swap ? y : x;
+            y = swap ? x : y;
+            x = t;
+        };
+        exchange(sv[p], sv[q]);
+#pragma unroll
         for (int i = 0; i < 3; ++i) {
-            U[i][j] = sv[o[j]] > 0 ? A[i][o[j]] / sv[o[j]] : 0.0;
-            V2[i][j] = V[i][o[j]];
+            exchange(A[i][p], A[i][q]);
+            exchange(V[i][p], V[i][q]);
         }
-    for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) V[i][j] = V2[i][j];
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) U[i][j] = sv[j] > 0 ? A[i][j] / sv[j] : 0.0;
 }
 
 // Thread 0's half of the fit: the 3x3 solve from s.fit (the centred moments Spp 00 01 02 11 12 22,
-// Spq row-major, then the means of p and q) into s.M and s.scal[0].  Out of line, so that its
+// Spq row-major, then the means of p and q) into M.  Out of line, so that its
 // registers do not add to those of the passes over the points.
-__device__ __noinline__ void lts_solve(LtsShared& s, bool affine) {
-    const double *o = s.fit, *mp = s.fit + 15, *mq = s.fit + 18;
+__device__ __noinline__ void lts_solve(const double *fit, float *M, int *solved, bool affine) {
+    const double *o = fit, *mp = fit + 15, *mq = fit + 18;
     // Spq[a][b] = sum (p_a - mp_a)(q_b - mq_b)
     const double Spq[3][3] = { { o[6], o[7], o[8] }, { o[9], o[10], o[11] }, { o[12], o[13], o[14] } };
     double L[3][3];
@@ -656,111 +721,185 @@ __device__ __noinline__ void lts_solve(LtsShared& s, bool affine) {
     }
     if (ok) {
         for (int r = 0; r < 3; ++r) {
-            for (int k = 0; k < 3; ++k) s.M[r * 4 + k] = (float)L[r][k];
-            s.M[r * 4 + 3] = (float)(mq[r] - (L[r][0] * mp[0] + L[r][1] * mp[1] + L[r][2] * mp[2]));
+            for (int k = 0; k < 3; ++k) M[r * 4 + k] = (float)L[r][k];
+            M[r * 4 + 3] = (float)(mq[r] - (L[r][0] * mp[0] + L[r][1] * mp[1] + L[r][2] * mp[2]));
         }
-        s.M[12] = s.M[13] = s.M[14] = 0.f;
-        s.M[15] = 1.f;
+        M[12] = M[13] = M[14] = 0.f;
+        M[15] = 1.f;
     }
-    s.scal[0] = ok;
+    *solved = ok;
 }
 
-// Least-squares fit of the kept correspondences (keep == nullptr: all n; fromSums:
-// from the sums the caller's keep pass left in s.out) into s.M.
-// Affine: the FP64 solution of [p 1] P = q through centred normal equations (the same minimiser
-// as EstimateAffineLeastSquares' QR, reg-lib/cpu/Maths.cpp:325-349).  Rigid: Kabsch on the centred
-// cross-covariance with the reflection guard (reg-lib/cpu/Maths.cpp:351-390).  Returns false
-// (uniformly) when the normal matrix is singular.
-__device__ bool lts_fit(const float *__restrict__ P, const float *__restrict__ Q, const uint8_t *keep, int n,
-                        bool affine, LtsShared& s, bool fromSums = false) {
-    if (fromSums) {
-        // the kept points' sums from the caller's pass, in s.out[1..22]: p, q, count, then the
-        // products p_a p_b (00 01 02 11 12 22) and p_a q_b; centred moments S = sum - count m m^T
-        // in FP64
-        if (threadIdx.x == 0) {
-            const double *sums = s.out + 1;
-            double *oc = s.fit, *mp = s.fit + 15, *mq = s.fit + 18;
-            const double cnt = sums[6];
-            for (int k = 0; k < 3; ++k) {
-                mp[k] = sums[k] / cnt;
-                mq[k] = sums[3 + k] / cnt;
-            }
-            const int pa[6] = { 0, 0, 0, 1, 1, 2 }, pb[6] = { 0, 1, 2, 1, 2, 2 };
-            for (int k = 0; k < 6; ++k) oc[k] = sums[7 + k] - cnt * mp[pa[k]] * mp[pb[k]];
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) oc[6 + a * 3 + b] = sums[13 + a * 3 + b] - cnt * mp[a] * mq[b];
-        }
-    } else {
-        double mp[3], mq[3];
-        double m[7] = { 0, 0, 0, 0, 0, 0, 0 };
-        for (int i = threadIdx.x; i < n; i += kLtsThreads) {
-            if (keep && !keep[i]) continue;
-            for (int k = 0; k < 3; ++k) {
-                m[k] += (double)P[3 * i + k];
-                m[3 + k] += (double)Q[3 * i + k];
-            }
-            m[6] += 1.0;
-        }
-        wg_sum<7>(m, s);
-        const double cnt = s.out[6];
-        for (int k = 0; k < 3; ++k) {
-            mp[k] = s.out[k] / cnt;
-            mq[k] = s.out[3 + k] / cnt;
-        }
-        __syncthreads();
-        double c[15] = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
-        for (int i = threadIdx.x; i < n; i += kLtsThreads) {
-            if (keep && !keep[i]) continue;
-            const double p0 = (double)P[3 * i] - mp[0], p1 = (double)P[3 * i + 1] - mp[1], p2 = (double)P[3 * i + 2] - mp[2];
-            const double q0 = (double)Q[3 * i] - mq[0], q1 = (double)Q[3 * i + 1] - mq[1], q2 = (double)Q[3 * i + 2] - mq[2];
-            c[0] += p0 * p0; c[1] += p0 * p1; c[2] += p0 * p2; c[3] += p1 * p1; c[4] += p1 * p2; c[5] += p2 * p2;
-            c[6] += p0 * q0; c[7] += p0 * q1; c[8] += p0 * q2;
-            c[9] += p1 * q0; c[10] += p1 * q1; c[11] += p1 * q2;
-            c[12] += p2 * q0; c[13] += p2 * q1; c[14] += p2 * q2;
-        }
-        wg_sum<15>(c, s);
-        if (threadIdx.x == 0) {
-            for (int k = 0; k < 15; ++k) s.fit[k] = s.out[k];
-            for (int k = 0; k < 3; ++k) {
-                s.fit[15 + k] = mp[k];
-                s.fit[18 + k] = mq[k];
-            }
-        }
-    }
-    if (threadIdx.x == 0) lts_solve(s, affine);
+// Least-squares fit into s.M of the points whose centred moments and means lts_moments or
+// lts_kept_moments left in s.fit.  Affine: the FP64 solution of [p 1] P = q through centred normal
+// equations (the same minimiser as EstimateAffineLeastSquares' QR, reg-lib/cpu/Maths.cpp:325-349).
+// Rigid: Kabsch on the centred cross-covariance with the reflection guard
+// (reg-lib/cpu/Maths.cpp:351-390).  Returns false (uniformly) when the normal matrix is singular.
+template<int NT>
+__device__ __forceinline__ bool lts_fit(bool affine, LtsShared<NT>& s) {
+    if (threadIdx.x == 0) lts_solve(s.fit, s.M, &s.scal[0], affine);
     __syncthreads();
     return s.scal[0] != 0;
+}
+
+// Loads kLtsUnroll points of P and Q (planes of stride floats), NT apart from i0, clamped to n - 1: all
+// loads issued together, each from a uniform base.
+template<int NT>
+__device__ __forceinline__ void lts_load(const float *__restrict__ P, const float *__restrict__ Q, int stride, int i0,
+                                         int n, float (&pq)[kLtsUnroll][6]) {
+#pragma unroll
+    for (int u = 0; u < kLtsUnroll; ++u) {
+        const uint32_t i = (uint32_t)min(i0 + u * NT, n - 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float *p = P + (size_t)c * stride, *q = Q + (size_t)c * stride;
+            pq[u][c] = p[i];
+            pq[u][3 + c] = q[i];
+        }
+    }
+    batch_loaded(pq);
+}
+
+// The centred moments of all n points, from their sums m (this thread's): a pass over the points
+// about the means.
+template<int NT>
+__device__ __forceinline__ void lts_moments(const float *__restrict__ P, const float *__restrict__ Q, int stride, int n,
+                                            double (&m)[7], LtsShared<NT>& s) {
+    wg_sum(m, s);
+    double mean[6];
+    for (int k = 0; k < 6; ++k) mean[k] = s.out[k] / s.out[6];
+    __syncthreads();
+    double c[15] = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+    for (int i0 = threadIdx.x; i0 < n; i0 += kLtsUnroll * NT) {
+        float pq[kLtsUnroll][6];
+        lts_load<NT>(P, Q, stride, i0, n, pq);
+#pragma unroll
+        for (int u = 0; u < kLtsUnroll; ++u) {
+            if (i0 + u * NT >= n) break;
+            double p[3], q[3];
+            for (int k = 0; k < 3; ++k) {
+                p[k] = (double)pq[u][k] - mean[k];
+                q[k] = (double)pq[u][3 + k] - mean[3 + k];
+            }
+            c[0] += p[0] * p[0]; c[1] += p[0] * p[1]; c[2] += p[0] * p[2];
+            c[3] += p[1] * p[1]; c[4] += p[1] * p[2]; c[5] += p[2] * p[2];
+            for (int a = 0; a < 3; ++a)
+                for (int b = 0; b < 3; ++b) c[6 + a * 3 + b] += p[a] * q[b];
+        }
+    }
+    wg_sum(c, s);
+    if (threadIdx.x == 0) {
+        for (int k = 0; k < 15; ++k) s.fit[k] = s.out[k];
+        for (int k = 0; k < 6; ++k) s.fit[15 + k] = mean[k];
+    }
+}
+
+// The same of the kept points, from their sums in s.kept: S = sum - count m m^T in FP64.
+template<int NT>
+__device__ __forceinline__ void lts_kept_moments(LtsShared<NT>& s) {
+    if (threadIdx.x != 0) return;
+    const double *sums = s.kept;
+    double *oc = s.fit, *mp = s.fit + 15, *mq = s.fit + 18;
+    const double cnt = sums[6];
+    for (int k = 0; k < 3; ++k) {
+        mp[k] = sums[k] / cnt;
+        mq[k] = sums[3 + k] / cnt;
+    }
+    const int pa[6] = { 0, 0, 0, 1, 1, 2 }, pb[6] = { 0, 1, 2, 1, 2, 2 };
+    for (int k = 0; k < 6; ++k) oc[k] = sums[7 + k] - cnt * mp[pa[k]] * mp[pb[k]];
+    for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) oc[6 + a * 3 + b] = sums[13 + a * 3 + b] - cnt * mp[a] * mq[b];
+}
+
+// dv += (or -=) the sums of the first c points of the wave's list: p, q, count and the products, each
+// exact in FP64 before it is added (a product of two floats has 48 bits).
+__device__ __forceinline__ void lts_add_listed(const float *__restrict__ P, const float *__restrict__ Q, int stride,
+                                               const volatile uint32_t *list, int c, double *dv) {
+    if ((int)(threadIdx.x & 63) >= c) return;
+    const uint32_t e = list[threadIdx.x & 63], i = e & 0x7fffffffu;
+    const double sign = e >> 31 ? -1.0 : 1.0;
+    double p[3], q[3], sp[3];
+    for (int k = 0; k < 3; ++k) {
+        const float *pk = P + (size_t)k * stride, *qk = Q + (size_t)k * stride;
+        p[k] = (double)pk[i];
+        q[k] = (double)qk[i];
+    }
+    for (int k = 0; k < 3; ++k) sp[k] = sign * p[k];
+    for (int k = 0; k < 3; ++k) {
+        dv[k] += sp[k];
+        dv[3 + k] = fma(sign, q[k], dv[3 + k]);
+    }
+    dv[6] += sign;
+    dv[7] = fma(sp[0], p[0], dv[7]);
+    dv[8] = fma(sp[0], p[1], dv[8]);
+    dv[9] = fma(sp[0], p[2], dv[9]);
+    dv[10] = fma(sp[1], p[1], dv[10]);
+    dv[11] = fma(sp[1], p[2], dv[11]);
+    dv[12] = fma(sp[2], p[2], dv[12]);
+    for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) dv[13 + a * 3 + b] = fma(sp[a], q[b], dv[13 + a * 3 + b]);
 }
 
 // optimize + optimize_3D (reg-lib/cpu/_reg_blockMatching.cpp:722-821,
 // reg-lib/cpu/_reg_globalTrans.cpp:328-394).  status: 0 ok, 1 too few correspondences,
 // 2 singular fit (the matrix is then left unchanged).  The trimmed subset is the keep smallest
 // residuals (float bit patterns, found by a three-digit radix select); ties at the threshold
-// keep the lowest indices.
+// keep the lowest indices.  P and Q: the defined correspondences, planar with nActive floats a plane
+// (the 12-byte rows of the inputs cost every load three times the cache lines).  LDS: res is in LDS and
+// holds at most 32 points a thread, whose kept flags are then a word's bits; otherwise the flags are
+// bytes after the residuals.
+//
+// One workgroup, as the 20 or so iterations are a serial chain of a residual pass, three digits and a
+// fit each, so its cost is the instructions and barriers of one compute unit.  The kept points' sums
+// are carried from one iteration to the next: only points that enter or leave the set are added or
+// subtracted, gathered in a list per wave so that 64 at a time fill the lanes (all kept points summed
+// anew took as long as the residuals).  19 iterations over 16384 points 470 -> 426 us, of which the
+// residuals are 40 % (their conversions to and from double run at a quarter of the rate) and the digits
+// 25 %; the 1000 points of a coarse level, 4 iterations, 57 -> 42 us.
+template<int NT, bool LDS>
 __device__ __forceinline__ void
 lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, int nActive, float *__restrict__ matrix,
          float *__restrict__ P, float *__restrict__ Q, uint32_t *__restrict__ res, int percent, int affine,
-         int *__restrict__ status, LtsShared& s, uint8_t *keepIn = nullptr) {
+         int *__restrict__ status, LtsShared<NT>& s) {
 #pragma clang fp contract(off)
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, stride = nActive;
     if (tid < 16) s.M[tid] = matrix[tid];
     __syncthreads();
+    double M0[12];
+    for (int k = 0; k < 12; ++k) M0[k] = uniform_double((double)s.M[k]);
     // defined correspondences in rank order, warped side mapped through the current matrix
     int n = 0;
-    for (int base = 0; base < nActive; base += kLtsThreads) {
-        const int i = base + tid;
-        const bool flag = i < nActive && warpPos[3 * i] == warpPos[3 * i];
-        int total;
-        const int pos = n + wg_scan(flag, s, &total);
-        if (flag) {
-            const float3 q = mat44_mul_f(s.M, warpPos[3 * i], warpPos[3 * i + 1], warpPos[3 * i + 2]);
-            P[3 * pos] = refPos[3 * i];
-            P[3 * pos + 1] = refPos[3 * i + 1];
-            P[3 * pos + 2] = refPos[3 * i + 2];
-            Q[3 * pos] = q.x;
-            Q[3 * pos + 1] = q.y;
-            Q[3 * pos + 2] = q.z;
+    double m[7] = { 0, 0, 0, 0, 0, 0, 0 };
+    for (int base = 0; base < nActive; base += kLtsUnroll * NT) {
+        float rw[kLtsUnroll][6];
+        bool flag[kLtsUnroll];
+        int pos[kLtsUnroll];
+#pragma unroll
+        for (int u = 0; u < kLtsUnroll; ++u) {
+            const uint32_t i = 3u * (uint32_t)min(base + u * NT + tid, nActive - 1);
+            for (int c = 0; c < 3; ++c) {
+                rw[u][c] = refPos[i + c];
+                rw[u][3 + c] = warpPos[i + c];
+            }
         }
+        batch_loaded(rw);
+#pragma unroll
+        for (int u = 0; u < kLtsUnroll; ++u)
+            flag[u] = base + u * NT + tid < nActive && rw[u][3] == rw[u][3];
+        const int total = wg_scan(flag, pos, s);
+#pragma unroll
+        for (int u = 0; u < kLtsUnroll; ++u)
+            if (flag[u]) {
+                const float3 q = mat44_mul_f(M0, rw[u][3], rw[u][4], rw[u][5]);
+                const float v[6] = { rw[u][0], rw[u][1], rw[u][2], q.x, q.y, q.z };
+                for (int c = 0; c < 3; ++c) {
+                    float *p = P + (size_t)c * stride, *q = Q + (size_t)c * stride;
+                    p[(uint32_t)(n + pos[u])] = v[c];
+                    q[(uint32_t)(n + pos[u])] = v[3 + c];
+                }
+                for (int c = 0; c < 6; ++c) m[c] += (double)v[c];
+                m[6] += 1.0;
+            }
         n += total;
     }
     const unsigned keep = (unsigned)((float)n * ((float)percent / 100.0f));
@@ -770,41 +909,35 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
     }
     __threadfence_block();
     __syncthreads();
-    if (!lts_fit(P, Q, nullptr, n, affine != 0, s)) {
+    lts_moments(P, Q, stride, n, m, s);
+    if (!lts_fit(affine != 0, s)) {
         if (tid == 0) *status = 2;
         return;
     }
-    // keep flags: after the residuals in global memory, or a separate array (LDS)
-    uint8_t *keepFlag = keepIn ? keepIn : reinterpret_cast<uint8_t *>(res + n);
+    uint8_t *keepFlag = LDS ? nullptr : reinterpret_cast<uint8_t *>(res + n);
+    uint32_t keptBits = 0;
     double lastDistance = DBL_MAX;
     if (tid < 16) s.last[tid] = 0.f;
+    if (tid < 24) s.kept[tid] = 0.0;
     __syncthreads();
     for (int it = 0; it < 30; ++it) {
         // residuals, counted into the first digit's histogram as they are formed
-        for (int b = tid; b < 2048; b += kLtsThreads) s.hist[b] = 0;
+        for (int b = tid; b < 2048 + 256; b += NT) s.hist[b] = 0;
         __syncthreads();
-        // kLtsUnroll points per thread per step: their loads are issued together (indexes
-        // clamped to n - 1, so every load stays in bounds), then the residuals formed
-        for (int i0 = tid; i0 < n; i0 += kLtsUnroll * kLtsThreads) {
+        double M[12];  // uniform: scalar registers
+        for (int k = 0; k < 12; ++k) M[k] = uniform_double((double)s.M[k]);
+        for (int i0 = tid; i0 < n; i0 += kLtsUnroll * NT) {
             float pq[kLtsUnroll][6];
+            lts_load<NT>(P, Q, stride, i0, n, pq);
 #pragma unroll
             for (int u = 0; u < kLtsUnroll; ++u) {
-                const int i = min(i0 + u * kLtsThreads, n - 1);
-                for (int c = 0; c < 3; ++c) {
-                    pq[u][c] = P[3 * i + c];
-                    pq[u][3 + c] = Q[3 * i + c];
-                }
-            }
-            batch_loaded(pq);
-#pragma unroll
-            for (int u = 0; u < kLtsUnroll; ++u) {
-                const int i = i0 + u * kLtsThreads;
+                const int i = i0 + u * NT;
                 if (i >= n) break;
-                const float3 t = mat44_mul_f(s.M, pq[u][0], pq[u][1], pq[u][2]);
+                const float3 t = mat44_mul_f(M, pq[u][0], pq[u][1], pq[u][2]);
                 const float dx = t.x - pq[u][3], dy = t.y - pq[u][4], dz = t.z - pq[u][5];
                 const uint32_t key = __float_as_uint(sqrtf(dx * dx + dy * dy + dz * dz));
                 res[i] = key;
-                atomicAdd(&s.hist[key >> 21], 1u);
+                atomicAdd(&s.hist[lts_bin(key >> 21)], 1u);
             }
         }
         __syncthreads();
@@ -816,11 +949,16 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
             const int sh = shifts[d];
             const uint32_t dm = (1u << widths[d]) - 1u;
             if (d > 0) {
-                for (int b = tid; b < 2048; b += kLtsThreads) s.hist[b] = 0;
+                for (int b = tid; b < 2048 + 256; b += NT) s.hist[b] = 0;
                 __syncthreads();
-                for (int i = tid; i < n; i += kLtsThreads) {
-                    const uint32_t key = res[i];
-                    if ((key & prefMask) == prefix) atomicAdd(&s.hist[(key >> sh) & dm], 1u);
+                for (int i0 = tid; i0 < n; i0 += kLtsUnroll * NT) {
+                    uint32_t key[kLtsUnroll];
+#pragma unroll
+                    for (int u = 0; u < kLtsUnroll; ++u) key[u] = res[(uint32_t)min(i0 + u * NT, n - 1)];
+#pragma unroll
+                    for (int u = 0; u < kLtsUnroll; ++u)
+                        if (i0 + u * NT < n && (key[u] & prefMask) == prefix)
+                            atomicAdd(&s.hist[lts_bin((key[u] >> sh) & dm)], 1u);
                 }
                 __syncthreads();
             }
@@ -828,7 +966,7 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
                 // the group of 32 bins holding the k-th key (prefix sums over the 64 groups),
                 // then the bin inside it (prefix sums over the group's 32 bins), both found
                 // by a ballot: the first bin whose inclusive count reaches k
-                const uint4 *grp = reinterpret_cast<const uint4 *>(&s.hist[tid * 32]);
+                const uint4 *grp = reinterpret_cast<const uint4 *>(&s.hist[lts_bin(tid * 32)]);
                 uint32_t local = 0;
 #pragma unroll
                 for (int b = 0; b < 8; ++b) {
@@ -839,79 +977,81 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
                 const unsigned long long inGroup = __ballot(excl < (uint32_t)k && (uint32_t)k <= excl + local);
                 const int g = inGroup ? __ffsll((long long)inGroup) - 1 : 0;
                 const uint32_t base = __shfl(excl, g, 64);
-                const uint32_t h = tid < 32 ? s.hist[g * 32 + tid] : 0u;
+                const uint32_t h = tid < 32 ? s.hist[lts_bin(g * 32 + tid)] : 0u;
                 const uint32_t before = base + wave_excl_scan(h);
                 const unsigned long long inBin = __ballot(tid < 32 && before + h >= (uint32_t)k);
                 if (tid == (inBin ? __ffsll((long long)inBin) - 1 : 0)) {
                     s.scal[1] = g * 32 + tid;
                     s.scal[2] = k - (int)before;
+                    s.scal[3] = (int)h;
                 }
             }
             __syncthreads();
-            if (d == 2) eqCount = s.hist[s.scal[1]];  // keys equal to the whole threshold
+            eqCount = (uint32_t)s.scal[3];  // after the last digit: keys equal to the whole threshold
             prefix |= (uint32_t)s.scal[1] << sh;
             prefMask |= dm << sh;
             k = s.scal[2];
             __syncthreads();
         }
-        // keep: residual below the threshold, or equal to it within the first k in index order
-        // (when every key equal to the threshold is kept, the order plays no part: one pass)
-        // the distance and the kept points' sums for the next fit (p, q, count, p p^T, p q^T): the
-        // fit then needs no pass over the points of its own
+        // keep: residual below the threshold, or equal to it within the first k in index order (when
+        // every key equal to the threshold is kept, the order plays no part); the distance is summed
+        // anew, the sums for the next fit (dv[0..22)) over the points that enter or leave the set
         double dv[23];
         for (int c = 0; c < 23; ++c) dv[c] = 0.0;
-        auto add_point = [&](const float *pf, const float *qf, uint32_t key) {
-            const double p[3] = { (double)pf[0], (double)pf[1], (double)pf[2] };
-            const double q[3] = { (double)qf[0], (double)qf[1], (double)qf[2] };
-            dv[0] += (double)__uint_as_float(key);
-            for (int c = 0; c < 3; ++c) {
-                dv[1 + c] += p[c];
-                dv[4 + c] += q[c];
-            }
-            dv[7] += 1.0;
-            dv[8] += p[0] * p[0]; dv[9] += p[0] * p[1]; dv[10] += p[0] * p[2];
-            dv[11] += p[1] * p[1]; dv[12] += p[1] * p[2]; dv[13] += p[2] * p[2];
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) dv[14 + a * 3 + b] += p[a] * q[b];
-        };
-        auto add_kept = [&](int i, uint32_t key) { add_point(P + 3 * i, Q + 3 * i, key); };
-        if ((uint32_t)k == eqCount) {
-            for (int i0 = tid; i0 < n; i0 += kLtsUnroll * kLtsThreads) {
-                float pq[kLtsUnroll][6];
+        volatile uint32_t *list = s.list[wv];
+        int listed = 0, seenEqual = 0;
+        const bool allEqual = (uint32_t)k == eqCount;
+        for (int base = 0; base < n; base += kLtsUnroll * NT) {
+            uint32_t key[kLtsUnroll];
+            bool kept[kLtsUnroll], was[kLtsUnroll];
 #pragma unroll
-                for (int u = 0; u < kLtsUnroll; ++u) {
-                    const int i = min(i0 + u * kLtsThreads, n - 1);
-                    for (int c = 0; c < 3; ++c) {
-                        pq[u][c] = P[3 * i + c];
-                        pq[u][3 + c] = Q[3 * i + c];
-                    }
-                }
-                batch_loaded(pq);
-#pragma unroll
-                for (int u = 0; u < kLtsUnroll; ++u) {
-                    const int i = i0 + u * kLtsThreads;
-                    if (i >= n) break;
-                    const uint32_t key = res[i];
-                    const bool kept = key <= prefix;
-                    keepFlag[i] = kept ? 1 : 0;
-                    if (kept) add_point(pq[u], pq[u] + 3, key);
-                }
+            for (int u = 0; u < kLtsUnroll; ++u) {
+                const int i = base + u * NT + tid;
+                key[u] = res[(uint32_t)min(i, n - 1)];
+                was[u] = !LDS && it > 0 && keepFlag[(uint32_t)min(i, n - 1)] != 0;
+                kept[u] = i < n && key[u] <= prefix;
+                if (i >= n) was[u] = false;
             }
-        } else {
-            int seenEqual = 0;
-            for (int base = 0; base < n; base += kLtsThreads) {
-                const int i = base + tid;
-                const uint32_t key = i < n ? res[i] : 0xffffffffu;
-                int total;
-                const int eqPos = seenEqual + wg_scan(i < n && key == prefix, s, &total);
-                const bool kept = i < n && (key < prefix || (key == prefix && eqPos < k));
-                if (i < n) keepFlag[i] = kept ? 1 : 0;
-                if (kept) add_kept(i, key);
+            if (!allEqual) {
+                bool equal[kLtsUnroll];
+                int eqPos[kLtsUnroll];
+#pragma unroll
+                for (int u = 0; u < kLtsUnroll; ++u) equal[u] = kept[u] && key[u] == prefix;
+                const int total = wg_scan(equal, eqPos, s);
+#pragma unroll
+                for (int u = 0; u < kLtsUnroll; ++u)
+                    kept[u] = kept[u] && (key[u] < prefix || seenEqual + eqPos[u] < k);
                 seenEqual += total;
             }
+#pragma unroll
+            for (int u = 0; u < kLtsUnroll; ++u) {
+                const int i = base + u * NT + tid;
+                if (kept[u]) dv[22] += (double)__uint_as_float(key[u]);
+                if (LDS) {
+                    was[u] = keptBits & 1u;
+                    keptBits = keptBits >> 1 | (kept[u] ? 0x80000000u : 0u);
+                } else if (i < n && (it == 0 || kept[u] != was[u])) {
+                    keepFlag[i] = kept[u] ? 1 : 0;
+                }
+                const bool flip = kept[u] != was[u];
+                const unsigned long long flips = __ballot(flip);
+                if (flips) {  // uniform over the wave; its lanes' accesses to the list are in program order
+                    if (flip)
+                        list[listed + __popcll(flips & ((1ull << lane) - 1ull))] =
+                            (uint32_t)i | (kept[u] ? 0u : 0x80000000u);
+                    listed += __popcll(flips);
+                    if (listed >= 64) {
+                        lts_add_listed(P, Q, stride, list, 64, dv);
+                        listed -= 64;
+                        if (lane < listed) list[lane] = list[64 + lane];
+                    }
+                }
+            }
         }
-        wg_sum<23>(dv, s);
-        const double distance = s.out[0];
+        if (LDS) keptBits >>= (32 - kLtsUnroll * ((n + kLtsUnroll * NT - 1) / (kLtsUnroll * NT))) & 31;
+        lts_add_listed(P, Q, stride, list, listed, dv);
+        wg_sum(dv, s);
+        const double distance = s.out[22];
         if (distance > lastDistance || (lastDistance - distance) < 1e-3) {
             if (tid < 16) s.M[tid] = s.last[tid];
             __syncthreads();
@@ -919,8 +1059,10 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
         }
         lastDistance = distance;
         if (tid < 16) s.last[tid] = s.M[tid];
+        if (tid < 22) s.kept[tid] += s.out[tid];
         __syncthreads();
-        if (!lts_fit(P, Q, keepFlag, n, affine != 0, s, true)) {
+        lts_kept_moments(s);
+        if (!lts_fit(affine != 0, s)) {
             if (tid == 0) *status = 2;
             return;
         }
@@ -928,34 +1070,39 @@ lts_body(const float *__restrict__ refPos, const float *__restrict__ warpPos, in
     if (tid < 16) matrix[tid] = s.M[tid];
 }
 
+// Past the LDS: the residuals and the kept flags in memory.
 __global__ void __launch_bounds__(kLtsThreads)
 k_lts(const float *__restrict__ refPos, const float *__restrict__ warpPos, int nActive, float *__restrict__ matrix,
       float *__restrict__ P, float *__restrict__ Q, uint32_t *__restrict__ res, int percent, int affine,
       int *__restrict__ status) {
-    __shared__ LtsShared s;
-    lts_body(refPos, warpPos, nActive, matrix, P, Q, res, percent, affine, status, s);
+    __shared__ LtsShared<kLtsThreads> s;
+    lts_body<kLtsThreads, false>(refPos, warpPos, nActive, matrix, P, Q, res, percent, affine, status, s);
 }
 
-// The same fit with the residuals and keep flags of up to kLtsLdsN correspondences in LDS (the
-// radix passes and the fits then read them from LDS instead of memory).
-constexpr int kLtsLdsN = 16384;
-
-__global__ void __launch_bounds__(kLtsThreads)
+// The same fit with the residuals of up to N correspondences in LDS.  Few of them go to 256 threads:
+// what an iteration over 1000 points takes is its barriers and the sums over the workgroup's waves.
+template<int NT, int N>
+__global__ void __launch_bounds__(NT)
 k_lts_lds(const float *__restrict__ refPos, const float *__restrict__ warpPos, int nActive, float *__restrict__ matrix,
           float *__restrict__ P, float *__restrict__ Q, int percent, int affine, int *__restrict__ status) {
-    __shared__ LtsShared s;
-    __shared__ uint32_t sRes[kLtsLdsN];
-    __shared__ uint8_t sKeep[kLtsLdsN];
-    lts_body(refPos, warpPos, nActive, matrix, P, Q, sRes, percent, affine, status, s, sKeep);
+    static_assert(N <= 32 * NT, "a thread's kept flags are a word");
+    __shared__ LtsShared<NT> s;
+    __shared__ uint32_t sRes[N];
+    lts_body<NT, true>(refPos, warpPos, nActive, matrix, P, Q, sRes, percent, affine, status, s);
 }
+
+constexpr int kLtsSmallThreads = 256, kLtsSmallN = 4096, kLtsLdsN = 16384;
 
 // One LTS fit of nActive correspondences on `stream`: in LDS when they fit, else with the
 // residual scratch `res` (nActive + nActive / 4 words) in memory.
 void launch_lts(hipStream_t stream, const float *refPos, const float *warpPos, int nActive, float *matrix, float *P,
                 float *Q, uint32_t *res, int percent, int affine, int *status) {
-    if (nActive <= kLtsLdsN)
-        hipLaunchKernelGGL(k_lts_lds, dim3(1), dim3(kLtsThreads), 0, stream, refPos, warpPos, nActive, matrix, P, Q,
-                           percent, affine, status);
+    if (nActive <= kLtsSmallN)
+        hipLaunchKernelGGL((k_lts_lds<kLtsSmallThreads, kLtsSmallN>), dim3(1), dim3(kLtsSmallThreads), 0, stream, refPos,
+                           warpPos, nActive, matrix, P, Q, percent, affine, status);
+    else if (nActive <= kLtsLdsN)
+        hipLaunchKernelGGL((k_lts_lds<kLtsThreads, kLtsLdsN>), dim3(1), dim3(kLtsThreads), 0, stream, refPos, warpPos,
+                           nActive, matrix, P, Q, percent, affine, status);
     else
         hipLaunchKernelGGL(k_lts, dim3(1), dim3(kLtsThreads), 0, stream, refPos, warpPos, nActive, matrix, P, Q, res,
                            percent, affine, status);
@@ -972,9 +1119,9 @@ struct LtsArgs {
 };
 
 __global__ void __launch_bounds__(kLtsThreads) k_lts_batch(const LtsArgs *__restrict__ A, int affine) {
-    __shared__ LtsShared s;
+    __shared__ LtsShared<kLtsThreads> s;
     const LtsArgs& a = A[blockIdx.x];
-    lts_body(a.refPos, a.warpPos, a.nActive, a.matrix, a.P, a.Q, a.res, a.percent, affine, a.status, s);
+    lts_body<kLtsThreads, false>(a.refPos, a.warpPos, a.nActive, a.matrix, a.P, a.Q, a.res, a.percent, affine, a.status, s);
 }
 
 // Empties the defined-block count before a block matching (a kernel, so that an iteration can be
