@@ -18,7 +18,9 @@
 #include "f3d_handle.hpp"
 #include "host.hpp"
 #include "m33.hpp"
+#include <climits>
 #include <cmath>
+#include <type_traits>
 
 namespace nrh {
 
@@ -355,6 +357,145 @@ __global__ void __launch_bounds__(kBlock) k_vel_affine_parts(float *fields, int 
     }
 }
 
+// ------------------------------------------------------------------ gathers through LDS
+typedef float Float2 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ Float2 ld32x2(const float *base, uint32_t byteOff) {
+    return *reinterpret_cast<const Float2 *>(reinterpret_cast<const char *>(base) + byteOff);
+}
+__device__ __forceinline__ float ld32(const float *base, uint32_t byteOff) {
+    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + byteOff);
+}
+
+// A vector image gathered at smooth positions takes nearly the same 8 neighbours for adjacent voxels, so a
+// workgroup of 512 takes a tile of 32 x 8 x (2 VPT) voxels, finds the box of the voxels that its
+// taps reach, copies the box's three components into LDS with coalesced loads and gathers there.
+// Voxels with a tap outside the image, and all those of a tile whose box does not fit, gather from
+// memory; every sum keeps its order.  What is left is bound by vector instructions, so addresses are
+// uniform bases with 32-bit offsets and a tap's three components lie side by side in LDS.
+constexpr int kTileX = 32, kTileY = 8, kTileThreads = 512;
+constexpr int kTileCap = 3300;  // voxels of a box: four workgroups a compute unit
+
+struct TileBox {
+    int sLo[3], sHi[3];
+    float v[3 * kTileCap];
+};
+
+// Minimum over the wave, valid in lane 63: shifts by 1, 2, 4 and 8 lanes inside each row of 16, then
+// the rows' last lanes (lanes with no source keep their own value).
+typedef short Short2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ Short2 wave_min(Short2 v) {
+    auto step = [&](auto ctrl, auto rows) {
+        int b;
+        __builtin_memcpy(&b, &v, 4);
+        b = __builtin_amdgcn_update_dpp(b, b, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+        Short2 o;
+        __builtin_memcpy(&o, &b, 4);
+        v = __builtin_elementwise_min(v, o);
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return v;
+}
+
+// Stages the box of all threads' taps [lo, hi] (lo = 32767, hi = -32767: a thread without any) of D
+// (planar [3][n], rows of nx, slices of ny) into S; returns whether it fits, its first voxel and its
+// row and slice strides.  Every thread of the workgroup calls it; the taps lie inside D.
+__device__ __forceinline__ bool stage_box(TileBox& S, const float *__restrict__ D, size_t n, int nx, int ny, int nz,
+                                          const int (&lo)[3], const int (&hi)[3], int (&org)[3], int& sy, int& sz) {
+    const int tid = threadIdx.x;
+    // coordinates and offsets in 16 and 32 bits; larger fields gather from memory
+    if (nx > 32767 || ny > 32767 || nz > 32767 || (size_t)nx * ny > (1u << 24)) return false;
+    if (tid < 3) {
+        S.sLo[tid] = INT_MAX;
+        S.sHi[tid] = INT_MIN;
+    }
+    __syncthreads();
+    const Short2 a = wave_min(Short2{ (short)lo[0], (short)lo[1] });
+    const Short2 b = wave_min(Short2{ (short)lo[2], (short)-hi[0] });
+    const Short2 c = wave_min(Short2{ (short)-hi[1], (short)-hi[2] });
+    if ((tid & 63) == 63) {
+        atomicMin(&S.sLo[0], (int)a.x);
+        atomicMin(&S.sLo[1], (int)a.y);
+        atomicMin(&S.sLo[2], (int)b.x);
+        atomicMax(&S.sHi[0], -(int)b.y);
+        atomicMax(&S.sHi[1], -(int)c.x);
+        atomicMax(&S.sHi[2], -(int)c.y);
+    }
+    __syncthreads();
+    int d[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        org[k] = __builtin_amdgcn_readfirstlane(S.sLo[k]);
+        d[k] = __builtin_amdgcn_readfirstlane(S.sHi[k]) - org[k] + 1;
+    }
+    sy = d[0];
+    sz = d[0] * d[1];
+    if (d[0] <= 0) return true;  // no voxel of the tile has its taps inside
+    if (d[0] > 64 || d[1] > 64 || d[2] > 64 || sz * d[2] > kTileCap) return false;
+    // element e of the box is row e / d0, its slice that / d1: products with the rounded-up reciprocal
+    // in 20 bits are exact for e d < 2^20
+    const uint32_t mx = (1u << 20) / (uint32_t)d[0] + 1u, my = (1u << 20) / (uint32_t)d[1] + 1u;
+    const int total = sz * d[2];
+    const float *D0 = D + ((size_t)org[2] * ny + org[1]) * nx + org[0], *D1 = D0 + n, *D2 = D1 + n;
+    // offset of e: z ny nx + (row - z d1) nx + e - row d0
+    const uint32_t perZ = (uint32_t)(ny - d[1]) * (uint32_t)nx, perRow = (uint32_t)(nx - d[0]);
+    constexpr int U = 4;
+    for (int e0 = tid; e0 < total; e0 += U * kTileThreads) {
+        float v[U][3];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // clamped, unconditional loads: all in flight before the first is stored
+            const uint32_t e = (uint32_t)min(e0 + u * kTileThreads, total - 1);
+            const uint32_t row = (e * mx) >> 20, z = (row * my) >> 20;
+            const uint32_t o = (e + row * perRow + z * perZ) * 4u;
+            v[u][0] = ld32(D0, o);
+            v[u][1] = ld32(D1, o);
+            v[u][2] = ld32(D2, o);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = e0 + u * kTileThreads;
+            if (e < total) {
+                S.v[3 * e] = v[u][0];
+                S.v[3 * e + 1] = v[u][1];
+                S.v[3 * e + 2] = v[u][2];
+            }
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
+// This thread's column of a tile: x, y, its byte offset in a slice, and the first slice (uniform over
+// the wave; slot u is 2 u slices on).
+struct TileColumn {
+    int x, y, z;
+    uint32_t off;
+    bool in;
+};
+
+template<int VPT>
+__device__ __forceinline__ TileColumn tile_column(int nx, int ny) {
+    const uint32_t t = (uint32_t)xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t tilesX = (uint32_t)(nx + kTileX - 1) / kTileX, tilesY = (uint32_t)(ny + kTileY - 1) / kTileY;
+    const uint32_t row = t / tilesX;
+    TileColumn c;
+    c.x = (int)(t - row * tilesX) * kTileX + (threadIdx.x & 31);
+    c.y = (int)(row % tilesY) * kTileY + ((threadIdx.x >> 5) & 7);
+    c.z = __builtin_amdgcn_readfirstlane((int)(row / tilesY) * 2 * VPT + (int)(threadIdx.x >> 8));
+    c.in = c.x < nx && c.y < ny;
+    c.off = c.in ? ((uint32_t)c.y * (uint32_t)nx + (uint32_t)c.x) * 4u : 0u;
+    return c;
+}
+
+__device__ __forceinline__ void st32(float *base, uint32_t byteOff, float v) {
+    *reinterpret_cast<float *>(reinterpret_cast<char *>(base) + byteOff) = v;
+}
+
 // reg_defField_compose3D without a mask (reg-lib/cpu/_reg_localTrans.cpp:2333-2457): out[i] is
 // the trilinear interpolation of field D (geometry d) at position pos[i], with sliding outside
 // D.  out may alias pos (each thread reads only its own position) but not D.
@@ -601,41 +742,19 @@ __global__ void __launch_bounds__(kBlock) k_resample_gradient(ResampleGradArgs r
 //   difference aside);
 // * a / sp is q + (a - q sp) / sp with q = a rsp and the residual taken by fused multiply-adds,
 //   rsp = 1 / sp rounded to float: Markstein's correction, correctly rounded;
-// * the division by the power of two 2^s is the product with its exact reciprocal;
-// * neighbours along x are fetched as one 8-byte load (4-byte aligned): the two taps of each row
-//   where no lane of the wave sits on an integer x (there the second tap is the first again), and a
-//   voxel's position with its x neighbour's.  24 loads a voxel instead of 42: the gathers' requests
-//   to the L1 bound the kernel, 214 -> 189 us a launch at 256 x 256 x 160 with both directions'
-//   launches overlapping.
-typedef float Float2 __attribute__((ext_vector_type(2), aligned(4)));
-__device__ __forceinline__ Float2 ld32x2(const float *base, uint32_t byteOff) {
-    return *reinterpret_cast<const Float2 *>(reinterpret_cast<const char *>(base) + byteOff);
-}
-__device__ __forceinline__ float ld32(const float *base, uint32_t byteOff) {
-    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + byteOff);
-}
-
-__global__ void __launch_bounds__(kBlock) k_resample_gradient32(ResampleGradArgs r) {
+// * the sum with accum and the division by the power of two 2^s, in double rounded to float, are the
+//   float sum and the float product with the exact reciprocal (53 bits are more than twice 24 and 2);
+// * the vector image's taps are gathered through LDS, a tile at a time; voxels that cannot be take the
+//   two taps of each row in one 8-byte load (4-byte aligned) where no lane of the wave sits on an
+//   integer x (there the second tap is the first again), as a voxel's position is with its x
+//   neighbour's.  256 x 256 x 160, both directions' launches overlapping: 42 loads a voxel 214 us a
+//   launch, 24 with pairs 189, 172 so (the
+//   field composition, with little else to do per voxel, got slower: 102 -> 120).
+// Taps, weights and the taps' box of position fc of the vector image; whether all lie inside it.
+__device__ __forceinline__ bool gradient_taps32(const ResampleGradArgs& r, float3 fc, int (&lo)[3], int (&hi)[3],
+                                                float (&bw)[3][2]) {
 #pragma clang fp contract(off)
-    const size_t ib = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (ib >= r.n) return;
-    const uint32_t i = (uint32_t)ib;
-    int x, y, z;
-    index_xyz(i, r.nx, r.ny, x, y, z);
-    const float *D0 = r.def, *D1 = r.def + r.n, *D2 = r.def + 2 * r.n;
-    const float *G0 = r.grad, *G1 = r.grad + r.gn, *G2 = r.grad + 2 * r.gn;
-    const uint32_t io = i * 4u;
-    // the Jacobian's corner o0: the voxel, one back along the axes where it is the last
-    const int ax = x == r.nx - 1, ay = y == r.ny - 1, az = z == r.nz - 1;
-    const uint32_t dsx = 4u, dsy = (uint32_t)r.nx * 4u, dsz = (uint32_t)r.nx * (uint32_t)r.ny * 4u;
-    const uint32_t o0 = io - (ax ? dsx : 0u) - (ay ? dsy : 0u) - (az ? dsz : 0u);
-    const Float2 c0 = ld32x2(D0, o0), c1 = ld32x2(D1, o0), c2 = ld32x2(D2, o0);
-    float3 pos = make_float3(c0.x, c1.x, c2.x);
-    if (ax | ay | az) pos = make_float3(ld32(D0, io), ld32(D1, io), ld32(D2, io));
-    const float3 fc = to_vox(r.gradIjk, pos);
     const float fcv[3] = { fc.x, fc.y, fc.z };
-    int lo[3], hi[3];
-    float bw[3][2];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         lo[k] = floor_int(fcv[k]);
@@ -644,9 +763,15 @@ __global__ void __launch_bounds__(kBlock) k_resample_gradient32(ResampleGradArgs
         bw[k][1] = fabsf(fcv[k] - (float)lo[k]);
         bw[k][0] = 1.f - bw[k][1];
     }
-    const int gdim[3] = { r.gnx, r.gny, r.gnz };
-    float vx = 0.f, vy = 0.f, vz = 0.f;
-    const bool inside = lo[0] > -1 && hi[0] < gdim[0] && lo[1] > -1 && hi[1] < gdim[1] && lo[2] > -1 && hi[2] < gdim[2];
+    return lo[0] > -1 && hi[0] < r.gnx && lo[1] > -1 && hi[1] < r.gny && lo[2] > -1 && hi[2] < r.gnz;
+}
+
+// The sum of the weighted taps from memory, padding outside.
+__device__ __forceinline__ void gradient_gather32(const ResampleGradArgs& r, bool inside, const int (&lo)[3],
+                                                  const int (&hi)[3], const float (&bw)[3][2], float& vx, float& vy,
+                                                  float& vz) {
+#pragma clang fp contract(off)
+    const float *G0 = r.grad, *G1 = r.grad + r.gn, *G2 = r.grad + 2 * r.gn;
     if (__all(inside && hi[0] == lo[0] + 1)) {
         const uint32_t sy = (uint32_t)r.gnx, sz = (uint32_t)r.gnx * (uint32_t)r.gny, xo = (uint32_t)lo[0];
         const uint32_t yo[2] = { (uint32_t)lo[1] * sy, (uint32_t)hi[1] * sy };
@@ -690,16 +815,16 @@ __global__ void __launch_bounds__(kBlock) k_resample_gradient32(ResampleGradArgs
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int Z = c ? hi[2] : lo[2];
-            if (Z > -1 && Z < gdim[2]) {
+            if (Z > -1 && Z < r.gnz) {
 #pragma unroll
                 for (int b = 0; b < 2; ++b) {
                     const int Y = b ? hi[1] : lo[1];
-                    if (Y > -1 && Y < gdim[1]) {
+                    if (Y > -1 && Y < r.gny) {
 #pragma unroll
                         for (int a = 0; a < 2; ++a) {
                             const int X = a ? hi[0] : lo[0];
                             const float w = bw[0][a] * bw[1][b] * bw[2][c];
-                            if (X > -1 && X < gdim[0]) {
+                            if (X > -1 && X < r.gnx) {
                                 const uint32_t o = (((uint32_t)Z * (uint32_t)r.gny + (uint32_t)Y) * (uint32_t)r.gnx +
                                                     (uint32_t)X) * 4u;
                                 vx += ld32(G0, o) * w;
@@ -726,37 +851,100 @@ __global__ void __launch_bounds__(kBlock) k_resample_gradient32(ResampleGradArgs
             }
         }
     }
-    const float d0v[3] = { c0.x, c1.x, c2.x };
-    const float dxv[3] = { c0.y, c1.y, c2.y };
-    const float dyv[3] = { ld32(D0, o0 + dsy), ld32(D1, o0 + dsy), ld32(D2, o0 + dsy) };
-    const float dzv[3] = { ld32(D0, o0 + dsz), ld32(D1, o0 + dsz), ld32(D2, o0 + dsz) };
-    float J[3][3];
+}
+
+template<int VPT>
+__global__ void __launch_bounds__(kTileThreads) k_resample_gradient32(ResampleGradArgs r) {
+#pragma clang fp contract(off)
+    __shared__ TileBox S;
+    const TileColumn col = tile_column<VPT>(r.nx, r.ny);
+    const size_t slice = (size_t)r.nx * r.ny;
+    float3 fc[VPT];
+    bool in[VPT];
+    int blo[3] = { 32767, 32767, 32767 }, bhi[3] = { -32767, -32767, -32767 };
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
-        J[m][0] = dxv[m] - d0v[m];
-        J[m][1] = dyv[m] - d0v[m];
-        J[m][2] = dzv[m] - d0v[m];
+    for (int u = 0; u < VPT; ++u) {
+        const float *p = r.def + (size_t)min(col.z + 2 * u, r.nz - 1) * slice;
+        fc[u] = make_float3(ld32(p, col.off), ld32(p + r.n, col.off), ld32(p + 2 * r.n, col.off));
     }
-    float R[3][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int u = 0; u < VPT; ++u) {
+        fc[u] = to_vox(r.gradIjk, fc[u]);
+        int lo[3], hi[3];
+        float bw[3][2];
+        in[u] = gradient_taps32(r, fc[u], lo, hi, bw) && col.in && col.z + 2 * u < r.nz;
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const float num = r.reo[a * 3] * J[0][b] + r.reo[a * 3 + 1] * J[1][b] + r.reo[a * 3 + 2] * J[2][b];
-            const float q = num * r.rsp[b];
-            R[a][b] = fmaf(fmaf(-q, r.sp[b], num), r.rsp[b], q);
+        for (int k = 0; k < 3; ++k) {
+            blo[k] = in[u] ? min(blo[k], lo[k]) : blo[k];
+            bhi[k] = in[u] ? max(bhi[k], hi[k]) : bhi[k];
         }
-    float o[3];
+    }
+    int org[3], sy, sz;
+    const bool fits = stage_box(S, r.grad, r.gn, r.gnx, r.gny, r.gnz, blo, bhi, org, sy, sz);
+    if (!col.in) return;
+    const uint32_t dsy = (uint32_t)r.nx * 4u;
+    // the Jacobian's corner: the voxel, one back along the axes where it is the last
+    const uint32_t o0 = col.off - (col.x == r.nx - 1 ? 4u : 0u) - (col.y == r.ny - 1 ? dsy : 0u);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) o[a] = R[a][0] * vx + R[a][1] * vy + R[a][2] * vz;
-    float *O[3] = { r.out, r.out + r.n, r.out + 2 * r.n };
-    const float *A[3] = { r.accum, r.accum + r.n, r.accum + 2 * r.n };
+    for (int u = 0; u < VPT; ++u) {
+        const int z = col.z + 2 * u;
+        if (z >= r.nz) break;
+        const float *D0 = r.def + (size_t)(z == r.nz - 1 ? z - 1 : z) * slice, *D1 = D0 + r.n, *D2 = D1 + r.n;
+        const Float2 c0 = ld32x2(D0, o0), c1 = ld32x2(D1, o0), c2 = ld32x2(D2, o0);
+        const float dyv[3] = { ld32(D0, o0 + dsy), ld32(D1, o0 + dsy), ld32(D2, o0 + dsy) };
+        const float dzv[3] = { ld32(D0 + slice, o0), ld32(D1 + slice, o0), ld32(D2 + slice, o0) };
+        const size_t zo = (size_t)z * slice;
+        float acc[3] = { 0.f, 0.f, 0.f };
+        if (r.accum)
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        float v = o[a];
-        if (r.accum) v = (float)((double)v + (double)ld32(A[a], io));
-        if (r.divisor > 0.0) v = (float)((double)v * r.invDivisor);
-        *reinterpret_cast<float *>(reinterpret_cast<char *>(O[a]) + io) = v;
+            for (int a = 0; a < 3; ++a) acc[a] = ld32(r.accum + zo + a * r.n, col.off);
+        int lo[3], hi[3];
+        float bw[3][2];
+        const bool inside = gradient_taps32(r, fc[u], lo, hi, bw);
+        float vx = 0.f, vy = 0.f, vz = 0.f;
+        if (fits && inside) {
+            const float *e = S.v + 3 * ((lo[2] - org[2]) * sz + (lo[1] - org[1]) * sy + lo[0] - org[0]);
+            const int ex = 3 * (hi[0] - lo[0]), ey = (hi[1] - lo[1]) * 3 * sy, ez = (hi[2] - lo[2]) * 3 * sz;
+            const float *row[4] = { e, e + ey, e + ez, e + ey + ez };
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float *t = row[k >> 1] + (k & 1 ? ex : 0);
+                const float w = bw[0][k & 1] * bw[1][(k >> 1) & 1] * bw[2][k >> 2];
+                vx += t[0] * w;
+                vy += t[1] * w;
+                vz += t[2] * w;
+            }
+        } else {
+            gradient_gather32(r, inside, lo, hi, bw, vx, vy, vz);
+        }
+        const float d0v[3] = { c0.x, c1.x, c2.x };
+        const float dxv[3] = { c0.y, c1.y, c2.y };
+                float J[3][3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            J[m][0] = dxv[m] - d0v[m];
+            J[m][1] = dyv[m] - d0v[m];
+            J[m][2] = dzv[m] - d0v[m];
+        }
+        float R[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                const float num = r.reo[a * 3] * J[0][b] + r.reo[a * 3 + 1] * J[1][b] + r.reo[a * 3 + 2] * J[2][b];
+                const float q = num * r.rsp[b];
+                R[a][b] = fmaf(fmaf(-q, r.sp[b], num), r.rsp[b], q);
+            }
+        float o[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) o[a] = R[a][0] * vx + R[a][1] * vy + R[a][2] * vz;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            float w = o[a];
+            if (r.accum) w = w + acc[a];
+            if (r.divisor > 0.0) w = w * (float)r.invDivisor;
+            st32(r.out + zo + a * r.n, col.off, w);
+        }
     }
 }
 
@@ -798,16 +986,29 @@ inline dim3 blocks_for(size_t n) { return dim3((unsigned)((n + kBlock - 1) / kBl
 // grid of a kernel indexed through xcd_block: a multiple of 8 workgroups
 inline dim3 blocks8_for(size_t n) { return dim3((unsigned)(((n + kBlock - 1) / kBlock + 7) / 8 * 8)); }
 
+inline dim3 blocks8(size_t blocks) { return dim3((unsigned)((blocks + 7) / 8 * 8)); }
+
+// Tiles of the gathers through LDS.  Four voxels a thread read the least around a tile; a launch of
+// fewer than kTileMinimum such tiles (two a compute unit are resident) takes a voxel a thread.
+template<int VPT>
+size_t tiles_of(int nx, int ny, int nz) {
+    return (size_t)((nx + kTileX - 1) / kTileX) * ((ny + kTileY - 1) / kTileY) * ((nz + 2 * VPT - 1) / (2 * VPT));
+}
+constexpr size_t kTileMinimum = 512;
+
 // k_resample_gradient32 when its conditions hold (planes below 4 GiB, at least two voxels per axis,
 // a power-of-two divisor), else k_resample_gradient.
 void launch_resample_gradient(ResampleGradArgs r, hipStream_t s) {
     const size_t lim = 0xffffffffull / 4;
     int e = 0;
-    const bool pow2 = r.divisor <= 0.0 || std::frexp(r.divisor, &e) == 0.5;
+    const bool pow2 = r.divisor <= 0.0 || (std::frexp(r.divisor, &e) == 0.5 && r.divisor < 1e30);
     if (3 * r.n <= lim && 3 * r.gn <= lim && r.nx >= 2 && r.ny >= 2 && r.nz >= 2 && pow2) {
         for (int k = 0; k < 3; ++k) r.rsp[k] = (float)(1.0 / (double)r.sp[k]);
         r.invDivisor = r.divisor > 0.0 ? 1.0 / r.divisor : 0.0;
-        hipLaunchKernelGGL(k_resample_gradient32, blocks8_for(r.n), dim3(kBlock), 0, s, r);
+        if (tiles_of<2>(r.nx, r.ny, r.nz) >= kTileMinimum)
+            hipLaunchKernelGGL(k_resample_gradient32<2>, blocks8(tiles_of<2>(r.nx, r.ny, r.nz)), dim3(kTileThreads), 0, s, r);
+        else
+            hipLaunchKernelGGL(k_resample_gradient32<1>, blocks8(tiles_of<1>(r.nx, r.ny, r.nz)), dim3(kTileThreads), 0, s, r);
     } else {
         hipLaunchKernelGGL(k_resample_gradient, blocks8_for(r.n), dim3(kBlock), 0, s, r);
     }
