@@ -48,8 +48,7 @@ static void lncc_gradient(nrh_f3d *h, float weight) {
 static void nmi_chain_gradient(nrh_f3d *h, float weight) {
     if (h->evalVersion != h->cppVersion) histogram_at_current_points(h);
     op_image_gradient(h);
-    zero_voxel_gradient(h);
-    op_nmi_voxel_gradient(h, 1.0);
+    op_nmi_voxel_gradient_eval(h);
     op_voxel_gradient_to_nodes(h, weight);
 }
 

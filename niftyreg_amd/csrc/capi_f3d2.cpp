@@ -113,14 +113,16 @@ int nrh_f3d2_gradient(nrh_f3d *fw, nrh_f3d *bw, double *max_length) {
             // reg_f3d2::GetVoxelBasedGradient (reg-lib/_reg_f3d2.cpp:246-301)
             warp_and_histograms(fw, bw);
             for (nrh_f3d *h : { fw, bw }) {
-                ensure_voxel_grad(h);
-                op_fill_f32(h->voxelGrad.p, 3 * h->N, 0.f, h->stream);
-                h->voxelGradPending = false;
                 op_image_gradient(h);
+                if (p.measure == NRH_MEASURE_LNCC) {
+                    ensure_voxel_grad(h);
+                    op_fill_f32(h->voxelGrad.p, 3 * h->N, 0.f, h->stream);
+                    h->voxelGradPending = false;
+                }
             }
             for (nrh_f3d *h : { fw, bw }) {
                 if (p.measure == NRH_MEASURE_LNCC) op_lncc_voxel_gradient(h, 1.0);
-                else op_nmi_voxel_gradient(h, 1.0);
+                else op_nmi_voxel_gradient_eval(h);
             }
             // ExponentiateGradient (reg-lib/_reg_f3d2.cpp:597-610): each direction reads the
             // other's grid (unchanged until the join before the penalty gradients) and, on a

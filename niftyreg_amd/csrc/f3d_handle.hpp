@@ -141,6 +141,8 @@ void op_joint_histogram(nrh_f3d *h, const float *warped);
 void op_nmi_finalize(nrh_f3d *h, float *kTab = nullptr, const double *pubS1 = nullptr, int pubN1 = -1,
                      int bePartials = 0);
 void op_nmi_voxel_gradient(nrh_f3d *h, double weight);
+// voxelGrad = the NMI voxel gradient, for an evaluation's gradient
+void op_nmi_voxel_gradient_eval(nrh_f3d *h);
 void op_convolve_voxel_gradient(nrh_f3d *h);
 void op_voxel_to_node(nrh_f3d *h, float weight);
 // op_convolve_voxel_gradient + op_voxel_to_node, convolving only what the nodes read where that is
