@@ -8,7 +8,7 @@ plus one objective gradient at the same control points (the unit "obj+grad eval"
 through libnrhip's fused sweeps with the images and control points resident in HBM.
 
 Prints one JSON line.  The roofline entry covers the dominant kernel (the gradient sweep,
-k_sweep<float, true>), timed with HIP events on the stream it runs on; its algorithmic bytes are
+k_sweep<float, kSweepGrad, depth>), timed with HIP events on the stream it runs on; its algorithmic bytes are
 the reference and floating images read once (8 B per voxel), its measured traffic also counts
 the voxel-gradient image it writes for the projection passes.  The CPU baseline times the
 reference CPU path (oracle/_ref, OpenMP) on a bounded sample of the same workload.
@@ -590,7 +590,7 @@ def main():
             "valu_source": "profiles/f3d_sweeps_256x256x160_counters.md (rocprofv3 SQ_INSTS_VALU per launch) over "
                            "the launch time, against 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction",
             "traffic_source": "profiles/f3d_eval_256x256x160_hbm_traffic.md (rocprofv3 FETCH_SIZE, WRITE_SIZE)",
-            "kernel": "k_sweep<float,true> (gradient sweep)",
+            "kernel": "k_sweep<float,kSweepGrad,8> (gradient sweep)",
             "kernel_ms": grad_ms, "histogram_sweep_ms": hist_ms, "algorithmic_bytes_per_launch": algo_bytes,
         },
         "cpu_baseline": None,

@@ -36,8 +36,8 @@ struct nrh_batch {
 
     // small kernels (f3d_ops.hip): per-pair descriptors and item tables (pair, block)
     nrh::DevBuf<uint8_t> pairOps;     // PairOps[P]
-    nrh::DevBuf<int2> itBE, itG, itG3, itCg;
-    int nBE = 0, nG = 0, nG3 = 0, nCg = 0;
+    nrh::DevBuf<int2> itBE, itG3, itCg;
+    int nBE = 0, nG3 = 0, nCg = 0;
 
     // results: per pair [NMI, H_r, H_f, H_rf, total, bending energy, value, max length]
     nrh::DevBuf<double> results;

@@ -985,7 +985,6 @@ struct PairOps {
     Affine xyz;
     BrickGrid bg;
     int beBlocks, cgBlocks;
-    float beRatio;         // bending-energy weight / G
     double beScale;        // 1 / (3 G)
     double *partials;      // bending-energy value and CG dot partials
     float *beGrad;
@@ -1658,7 +1657,7 @@ k_batch_values(const PairOps *__restrict__ P, const int *active, int sumBe, cons
 
 void batch_ops_setup(nrh_batch *b) {
     std::vector<PairOps> ops(b->P);
-    std::vector<int2> itBE, itG, itG3, itCg;
+    std::vector<int2> itBE, itG3, itCg;
     std::vector<float> w(2 * b->P);
     for (int q = 0; q < b->P; ++q) {
         nrh_f3d *h = b->pairs[q];
@@ -1685,7 +1684,6 @@ void batch_ops_setup(nrh_batch *b) {
         o.bg = bg;
         o.beBlocks = nb;
         o.cgBlocks = cgBlocks;
-        o.beRatio = h->params.be_weight / (float)h->G;
         o.beScale = 1.0 / (double)(3 * h->G);
         o.partials = h->partials.p;
         o.beGrad = h->beGrad.p;
@@ -1704,7 +1702,6 @@ void batch_ops_setup(nrh_batch *b) {
         w[2 * q] = h->params.similarity_weight;
         w[2 * q + 1] = h->params.be_weight;
         for (int k = 0; k < nb; ++k) itBE.push_back(make_int2(q, k));
-        for (unsigned k = 0; k < blocks_for(h->G); ++k) itG.push_back(make_int2(q, (int)k));
         for (unsigned k = 0; k < blocks_for(n3); ++k) itG3.push_back(make_int2(q, (int)k));
         for (int k = 0; k < cgBlocks; ++k) itCg.push_back(make_int2(q, k));
     }
@@ -1718,7 +1715,6 @@ void batch_ops_setup(nrh_batch *b) {
         n = (int)v.size();
     };
     up(b->itBE, itBE, b->nBE);
-    up(b->itG, itG, b->nG);
     up(b->itG3, itG3, b->nG3);
     up(b->itCg, itCg, b->nCg);
     b->results.alloc((size_t)kBatchResults * b->P);
