@@ -19,14 +19,12 @@ static void histogram_at_current_points(nrh_f3d *h) {
     }
 }
 
-// reg_f3d::WarpFloatingImage and reg_lncc's convolved sums
+// reg_f3d::WarpFloatingImage and reg_lncc's convolved sums.  The field and the warp are the
+// per-operation ones: the fused sweep's field sums and its float mm -> voxel product move single
+// positions by some ulps, which the local variances amplify.
 static void lncc_at_current_points(nrh_f3d *h) {
-    if (fused_warp_supported(h)) {
-        fused_warp(h);
-    } else {
-        op_spline_field(h);
-        op_resample(h);
-    }
+    op_spline_field(h);
+    op_resample(h);
     op_lncc_eval(h);
     h->evalVersion = h->cppVersion;
 }

@@ -68,9 +68,7 @@ struct FusedArgs {
     const double *ent;
     const float *kTab;  // gradient sweep: K[r + w rb] = log p_r + log p_w - NMI log p_rw (padded to 4)
     float *gvox;      // gradient sweep: the NMI voxel gradient (planar [3][N])
-    float *fieldOut;  // the deformation field of the sweep (planar [3][N]): warp sweep; optional in the
-                      // histogram sweep, for checking
-    float *warpOut;   // warp sweep: the warped image
+    float *fieldOut;  // histogram sweep, optional: the deformation field (planar [3][N]), for checking
     // voxels left to the exact pass: positions within ambTol (floating voxels) of a voxel plane;
     // tile t lists its voxels in ambList[t * tileVoxels ..] and their number in ambCounts[t]
     uint32_t *ambList;
@@ -81,9 +79,8 @@ struct FusedArgs {
     const double *logh;  // the reference's jointHistogramLog (exact pass of the gradient sweep)
 };
 
-// What a sweep makes of its voxels: the joint histogram, the NMI voxel gradient, or the warped image
-// (with the field in fieldOut).
-enum { kSweepHist = 0, kSweepGrad = 1, kSweepWarp = 2 };
+// What a sweep makes of its voxels: the joint histogram or the NMI voxel gradient.
+enum { kSweepHist = 0, kSweepGrad = 1 };
 
 template<class T> __device__ __forceinline__ float ld(const T *p, size_t i);
 template<> __device__ __forceinline__ float ld<float>(const float *p, size_t i) { return p[i]; }
@@ -218,9 +215,7 @@ __device__ __forceinline__ void sweep_finish(const FusedArgs& a, VoxelTaps t, fl
     const float f0 = e00 * y0b + e01 * ry, f1 = e10 * y0b + e11 * ry;
     const float war = f0 * z0b + f1 * rz;
     const float rv = t.rv;
-    if (MODE == kSweepWarp) {
-        if (t.active) a.warpOut[idx] = war;
-    } else if (MODE == kSweepHist) {
+    if (MODE == kSweepHist) {
         bool edge = false;
         if (t.active && rv == rv && war == war) {
             float lo = t.v[0][0][0], hi = lo;
@@ -363,7 +358,7 @@ __device__ __forceinline__ float3 gradient_taps(const float v[2][2][2], float3 p
 }
 
 // One listed voxel idx of pair a: the histogram pass counts it into the tile's LDS histogram h,
-// the gradient pass writes its voxel gradient, the warp pass its field and warped value.
+// the gradient pass writes its voxel gradient.
 template<class TImg, int MODE>
 __device__ __forceinline__ void fixup_voxel(const FusedArgs& a, const uint32_t idx, uint32_t *h) {
     const TImg *__restrict__ ref = (const TImg *)a.ref;
@@ -381,13 +376,7 @@ __device__ __forceinline__ void fixup_voxel(const FusedArgs& a, const uint32_t i
     exact_taps(flo, a.fnx, a.fny, a.fnz, px, py, pz, a.pad, v);
     const float rv = ld(ref, idx);
     const float war = sample_taps(v, p, px, py, pz);
-    if (MODE == kSweepWarp) {
-        const uint32_t N = (uint32_t)a.nx * a.ny * a.nz;
-        a.fieldOut[idx] = w.x;
-        a.fieldOut[idx + N] = w.y;
-        a.fieldOut[idx + 2 * N] = w.z;
-        a.warpOut[idx] = war;
-    } else if (MODE == kSweepHist) {
+    if (MODE == kSweepHist) {
         if (rv == rv && war == war && rv >= 0.f && rv < (float)a.rb && war >= 0.f && war < (float)a.fb)
             atomicAdd(&h[(int)rv + (int)war * a.rb], 1u);
     } else {
@@ -667,7 +656,7 @@ __device__ __forceinline__ void sweep_tile(const FusedArgs& a, const int t, cons
                 t[k].rx = pos[k].rx;
                 t[k].ry = pos[k].ry;
                 t[k].rz = pos[k].rz;
-                t[k].rv = MODE == kSweepWarp ? 0.f : ld(ref, idx[k]);
+                t[k].rv = ld(ref, idx[k]);
             }
 #pragma unroll
             for (int k = 0; k < kRowsPerWave; ++k) {
@@ -1289,10 +1278,9 @@ static void launch_sweep(const FusedArgs& a, int depth, size_t lds, hipStream_t 
 
 // Dynamic LDS of a sweep: the control-point window and its z contraction, then the histogram / NMI
 // table in their place.
-static size_t window_lds(int depth) { return (size_t)3 * (WZM + depth) * WYM * WXM * sizeof(float); }
 static size_t sweep_lds(const FusedArgs& a, int depth) {
     // window [3][WZM][WYM][WXM] + its z contraction [3][depth][WYM][WXM]; then histogram / table K
-    return std::max<size_t>(((size_t)a.rb * a.fb + 3) / 4 * 4 * sizeof(float), window_lds(depth));
+    return std::max<size_t>(((size_t)a.rb * a.fb + 3) / 4 * 4, (size_t)3 * (WZM + depth) * WYM * WXM) * sizeof(float);
 }
 
 static BeArgs be_args(nrh_f3d *h) {
@@ -1346,31 +1334,6 @@ void fused_histogram(nrh_f3d *h, float *fieldOut, bool beValue, const double *pu
     p->kTab.alloc((size_t)(a.rb * a.fb + 3) / 4 * 4);
     op_nmi_finalize(h, p->kTab.p, pubS1, pubN1, bePartials);
     h->histVersion = h->cppVersion;
-}
-
-// The warped image and the field of the current points (the exact pass's voxels in the reference's
-// order, as everywhere on the fused path): one sweep without histogram in place of a kernel for the
-// field's 64 sums per voxel and one for the resampling.  float32 images, whatever the storage.
-bool fused_warp_supported(nrh_f3d *h) {
-    return plan_of(h)->ok && 3 * (size_t)h->N <= 0xffffffffull && (size_t)h->Nf <= 0xffffffffull;
-}
-
-void fused_warp(nrh_f3d *h) {
-    FusedPlan *p = plan_of(h);
-    NRH_REQUIRE(fused_warp_supported(h), NRH_ERR_UNSUPPORTED, "fused path unavailable for this geometry");
-    ensure_field(h);
-    ensure_warped(h);
-    h->velFieldVersion = 0;
-    h->touch();
-    FusedArgs a = make_args(h, p);
-    a.ref = h->refImg.p;
-    a.flo = h->floImg.p;
-    a.fieldOut = h->field.p;
-    a.warpOut = h->warped.p;
-    launch_sweep<float, kSweepWarp>(a, p->depth, window_lds(p->depth), h->stream);
-    hipLaunchKernelGGL((k_sweep_fixup<float, kSweepWarp>), dim3((unsigned)((a.numTiles + kFixChunk - 1) / kFixChunk)),
-                       dim3(256), 0, h->stream, a);
-    NRH_HIP(hipGetLastError());
 }
 
 // Arguments of the three projection passes of the voxel gradient g (planar [3][N]) onto the

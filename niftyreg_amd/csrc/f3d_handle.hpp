@@ -208,8 +208,6 @@ void op_symmetrise_velocity(nrh_f3d *fw, nrh_f3d *bw);
 // fused evaluation (f3d_fused.hip)
 bool fused_supported(nrh_f3d *h);
 void fused_release(const nrh_f3d *h);
-bool fused_warp_supported(nrh_f3d *h);
-void fused_warp(nrh_f3d *h);
 // beValue: also the bending energy (into scalars[0]), in the exact pass's launch
 // pubN1 >= 0: the finalisation also publishes the entropies and NMI followed by pubS1[0..pubN1)
 // (op_publish's layout, the sequence number advanced)

@@ -72,3 +72,39 @@ def test_evaluation_matches_per_operation_measure(gpu, dims, spacing, sigma, mas
         assert np.array_equal(got, want)
     else:
         assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("dims,spacing,masked", [
+    ((65, 33, 41), 5.0, True),    # the tabulated spacing: masked voxels of the field are not written
+    ((64, 40, 32), 4.0, True),    # zeros there
+    ((66, 37, 35), 6.0, False),
+])
+def test_evaluation_warps_as_the_per_operation_chain(gpu, dims, spacing, masked):
+    """The field and the warped image behind a value and a gradient: those of the per-operation calls,
+    bit for bit, on grids that the fused sweeps take too."""
+    g = Geom.identity(dims)
+    rng = np.random.default_rng(sum(dims))
+    ref = phantoms.blob_phantom(dims, 1).ravel()
+    flo = phantoms.blob_phantom(dims, 2).ravel()
+    cg, cpp = create_control_point_grid(g, [spacing] * 3)
+    cpp = (cpp + rng.uniform(-1.5, 1.5, cpp.size)).astype(np.float32)
+    mask = (rng.uniform(size=g.nvox) > 0.2).astype(np.int32) - 1 if masked else None
+    keep = mask > -1 if masked else np.ones(g.nvox, bool)
+    p = default_params(similarity_weight=0.99, be_weight=0.01, measure=_lib.MEASURE_LNCC, lncc_sigma=-3.0)
+    h = F3dContent(g, ref, g, flo, cg, cpp, mask=mask, params=p)
+    h.rescale_intensities((0, 1), (0, 1))
+    got = []
+    for call in (h.objective, h.gradient):
+        h.set_control_points(cpp)
+        call()
+        got.append((h.deformation_field().reshape(3, -1), h.warped().ravel()))
+    h.set_control_points(cpp)
+    h.GetDeformationField()
+    h.ResampleImage()
+    field, warped = h.deformation_field().reshape(3, -1), h.warped().ravel()
+    h.close()
+    for f, w in got:
+        assert np.array_equal(f[:, keep], field[:, keep])
+        assert np.array_equal(w[keep], warped[keep], equal_nan=True)
+        if masked and spacing != 5.0:
+            assert not f[:, ~keep].any()
