@@ -60,7 +60,6 @@ struct nrh_f3d {
 
     // LNCC: two ping-pong sets of planar numerators + density, combined mask, reductions
     nrh::DevBuf<float> lnccA, lnccB, lnccKern;
-    nrh::DevBuf<double> lnccKernD;  // the kernels as double
     nrh::DevBuf<uint8_t> lnccComb;
     nrh::DevBuf<double> lnccPart, lnccScalars;  // scalars: adjusted weight, -, value, active count
     float lnccSigma = 0.f;
@@ -184,7 +183,7 @@ void wait_published(nrh_f3d *h);
 // LNCC measure (lncc.hip); value = mean |local correlation| into out_device[0] (count in [1])
 void op_lncc_value(nrh_f3d *h, double *out_device);
 void op_lncc_voxel_gradient(nrh_f3d *h, double weight);
-// The same for the evaluations, in fewer passes and with sums that differ in rounding (lncc.hip):
+// The same for the evaluations, in fewer passes (lncc.hip):
 // op_lncc_eval leaves the convolved sums of the warped image, from which the value and the gradient
 // are formed; the gradient is written over voxelGrad and uses the sums up.
 void op_lncc_eval(nrh_f3d *h);

@@ -9,11 +9,12 @@
 // products added in double, reg-lib/cpu/_reg_tools.cpp:1047-1053), so the results equal the
 // reference's scalar build bit for bit.  That is the per-operation measure (op_lncc_value,
 // op_lncc_voxel_gradient).  The evaluations take the passes at the end of the kernels below, which
-// form the same sums without rounding the products and in fewer trips to memory.
+// form the same sums in fewer trips to memory.
 
 #include "f3d_handle.hpp"
 #include "device.hpp"
 #include <cmath>
+#include <type_traits>
 
 namespace nrh {
 
@@ -338,51 +339,62 @@ k_lncc_apply(const float *__restrict__ T, const uint8_t *__restrict__ comb, cons
 }
 
 // ------------------------------------------------------------------ evaluation passes
-// The evaluations' convolutions.  Per tap a fused multiply-add in double of the exact product, where
-// the per-operation passes round the product to float, widen it and add (three instructions, the
-// widening at a quarter of the rate): the sums are closer to exact, and each axis still ends in one
-// rounding to float.  The lines lie in LDS as doubles, widened once per sample; a lane holds a sliding
-// window of 16 samples in registers for 8 outputs, so a sample is read from LDS about 5 times, not 31.
-// The x pass forms the six numerators from the two images as it stages them, and the z pass ends in
-// the value or the derivative terms, so that the six arrays cross memory four times instead of ten.
-// At 256 x 256 x 160, sigma 5 voxels (31 taps): the x, y and z passes of the six sums take 137, 175
-// and 205 us, about 300 each before, with a preparing and a reducing pass of 52 and 70 us; the
-// derivative's three arrays 78, 87 and 139 us.  The sums themselves are 50 us of each six-array pass
-// (double multiply-adds at the vector rate), its bytes 64, 97 and 48; the z pass also takes five
-// divisions and two square roots a voxel.
+// The evaluations' convolutions: the sums of the per-operation passes, product by product, in fewer
+// trips to memory.  The x pass forms the six numerators from the two images as it stages them, with a
+// sliding window of samples in registers for eight neighbouring outputs, and the z pass ends in the value
+// or the derivative terms, so that the six arrays cross memory four times instead of ten.
+// At 256 x 256 x 160, sigma 5 voxels (31 taps): the x, y and z passes of the six sums take 225, 219 and
+// 278 us (with the derivative's terms 305), about 300 each by the per-operation passes, with a preparing
+// and a reducing pass of 52 and 70 us; the derivative's three arrays 109, 110 and 152 us.  A tap is a
+// float product, its widening and an addition in double: bound by these.  Two shifts of the product's bits
+// in place of the widening, 2^-896 scaled, took longer (281, about 305 and 314 us).  Fused multiply-adds
+// in double took 137, 175 and 205 us, but an unrounded product moves the node gradient by 1e-4.
 constexpr int kEvalRadius = 30;  // radii above take the per-operation passes (LDS rows of 64 KB)
 constexpr int kColOut = 32;      // outputs along y / z per workgroup: four waves of 8
 constexpr int kEvalRows = 32;    // rows per workgroup of the x pass
 
-// chunks of 8 samples that 8 outputs over `taps` taps touch
-__host__ __device__ constexpr int eval_chunks(int taps) { return taps / 8 + 2; }
-size_t eval_lds_cols(int radius) {
-    return (size_t)8 * (kColOut / 8 - 1 + eval_chunks(2 * radius + 1)) * 64 * sizeof(double);
-}
-// x rows: chunk k of a row starts at 9 k doubles (the ninth unused), rows at a stride of 1 modulo 32:
-// the 8 segments of neighbouring rows then read distinct bank pairs but for one
-__host__ __device__ constexpr int eval_row_stride(int taps) { return (9 * (7 + eval_chunks(taps)) + 30) / 32 * 32 + 1; }
-size_t eval_lds_rows(int radius) { return (size_t)kEvalRows * eval_row_stride(2 * radius + 1) * sizeof(double); }
+size_t eval_lds_cols(int radius) { return (size_t)(kColOut + 2 * radius) * 64 * sizeof(float); }
+// x rows: chunk k of a row starts at 9 k (the ninth unused), rows at a stride of 1 modulo 64: the
+// 8 segments of 8 neighbouring rows then read distinct banks but for seven.  8 outputs over `taps`
+// taps touch taps / 8 + 2 chunks
+__host__ __device__ constexpr int eval_row_stride(int taps) { return (9 * (9 + taps / 8) + 62) / 64 * 64 + 1; }
+size_t eval_lds_rows(int radius) { return (size_t)kEvalRows * eval_row_stride(2 * radius + 1) * sizeof(float); }
 
-// acc[o] = sum_k kern[k] s[o + k], o < 8, in ascending k, where sample 8 c + e lies at
-// base[c * CHUNK + e * STEP].  Samples past o + k = 7 + taps - 1 are loaded, not used.
-template<int CHUNK, int STEP>
-__device__ __forceinline__ void conv8(const double *base, const double *__restrict__ kern, int taps, double (&acc)[8]) {
-    double w[16];
+// out[o] = sum_k (double)(kern[k] s[o + k]), o < 8, in ascending k.  Column: sample p at base[64 p],
+// which the lanes read without conflicts, so a tap reads its eight samples.
+__device__ __forceinline__ void conv8_column(const float *base, const float *__restrict__ kern, int taps,
+                                             float (&out)[8]) {
+#pragma clang fp contract(off)
+    double acc[8] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
+    for (int k = 0; k < taps; ++k) {
+        const float kv = kern[k];
+#pragma unroll
+        for (int o = 0; o < 8; ++o) acc[o] += (double)(kv * base[(o + k) * 64]);
+    }
+#pragma unroll
+    for (int o = 0; o < 8; ++o) out[o] = (float)acc[o];
+}
+
+// The same along a row in chunks of 8 samples, sample 8 c + e at base[9 c + e], from a window of 16 in
+// registers.  Samples past o + k = 7 + taps - 1 are loaded, not used.
+__device__ __forceinline__ void conv8_row(const float *base, const float *__restrict__ kern, int taps, float (&out)[8]) {
+#pragma clang fp contract(off)
+    float w[16];
+    double acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        w[e] = base[e * STEP];
+        w[e] = base[e];
         acc[e] = 0.0;
     }
     int c = 0;
     for (; 8 * c + 8 <= taps; ++c) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * CHUNK + e * STEP];
+        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * 9 + e];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const double kv = kern[8 * c + k];
+            const float kv = kern[8 * c + k];
 #pragma unroll
-            for (int o = 0; o < 8; ++o) acc[o] = fma(kv, w[o + k], acc[o]);
+            for (int o = 0; o < 8; ++o) acc[o] += (double)(kv * w[o + k]);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) w[e] = w[8 + e];
@@ -390,15 +402,17 @@ __device__ __forceinline__ void conv8(const double *base, const double *__restri
     const int rest = taps - 8 * c;
     if (rest > 0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * CHUNK + e * STEP];
+        for (int e = 0; e < 8; ++e) w[8 + e] = base[(c + 1) * 9 + e];
 #pragma unroll
         for (int k = 0; k < 7; ++k)
             if (k < rest) {  // uniform
-                const double kv = kern[8 * c + k];
+                const float kv = kern[8 * c + k];
 #pragma unroll
-                for (int o = 0; o < 8; ++o) acc[o] = fma(kv, w[o + k], acc[o]);
+                for (int o = 0; o < 8; ++o) acc[o] += (double)(kv * w[o + k]);
             }
     }
+#pragma unroll
+    for (int o = 0; o < 8; ++o) out[o] = (float)acc[o];
 }
 
 // x pass.  A lane takes 8 neighbouring outputs of one row (8 segments by 32 rows a workgroup).
@@ -408,9 +422,9 @@ template<bool FIRST>
 __global__ void __launch_bounds__(kB)
 k_eval_x(const float *__restrict__ ref, const float *__restrict__ war, const int *__restrict__ mask,
          const float *__restrict__ in, float *__restrict__ out, uint8_t *__restrict__ comb, size_t N, int nx, int nrows,
-         const double *__restrict__ kern, int radius) {
+         const float *__restrict__ kern, int radius) {
 #pragma clang fp contract(off)
-    extern __shared__ double rowsD[];
+    extern __shared__ float rowsF[];
     const int taps = 2 * radius + 1, W = 64 + 2 * radius, S = eval_row_stride(taps);
     const int x0 = blockIdx.y * 64, row0 = blockIdx.x * kEvalRows;
     // a wave stages every fourth row, a lane its samples `lane` and 64 + lane: every load in flight
@@ -447,7 +461,6 @@ k_eval_x(const float *__restrict__ ref, const float *__restrict__ war, const int
     }
     const int seg = threadIdx.x & 7, r = threadIdx.x >> 3, row = row0 + r, x = x0 + 8 * seg;
     const int at0 = (lane >> 3) * 9 + (lane & 7);
-#pragma unroll
     for (int q = 0; q < (FIRST ? 6 : 1); ++q) {
 #pragma unroll
         for (int e = 0; e < kEl; ++e)
@@ -455,22 +468,21 @@ k_eval_x(const float *__restrict__ ref, const float *__restrict__ war, const int
             for (int h = 0; h < 2; ++h) {
                 const float u = a[e][h], t = b[e][h];
                 const float v = !FIRST ? u : q == 0 ? u : q == 1 ? u * u : q == 2 ? t : q == 3 ? t * t : q == 4 ? u * t : 1.f;
-                if (lane + 64 * h < W)
-                    rowsD[(w + e * (kB / 64)) * S + at0 + 72 * h] = ok[e][h] ? (double)v : 0.0;
+                if (lane + 64 * h < W) rowsF[(w + e * (kB / 64)) * S + at0 + 72 * h] = ok[e][h] ? v : 0.f;
             }
         __syncthreads();
-        double acc[8];
-        conv8<9, 1>(rowsD + r * S + 9 * seg, kern, taps, acc);
+        float acc[8];
+        conv8_row(rowsF + r * S + 9 * seg, kern, taps, acc);
         float *dst = out + (size_t)(FIRST ? q : blockIdx.z) * N + (size_t)row * nx + x;
         if (row < nrows && x + 8 <= nx) {
             // two 16-byte stores (4-byte aligned)
             typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
-            *reinterpret_cast<Float4 *>(dst) = Float4{ (float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3] };
-            *reinterpret_cast<Float4 *>(dst + 4) = Float4{ (float)acc[4], (float)acc[5], (float)acc[6], (float)acc[7] };
+            *reinterpret_cast<Float4 *>(dst) = Float4{ acc[0], acc[1], acc[2], acc[3] };
+            *reinterpret_cast<Float4 *>(dst + 4) = Float4{ acc[4], acc[5], acc[6], acc[7] };
         } else {
 #pragma unroll
             for (int o = 0; o < 8; ++o)
-                if (row < nrows && x + o < nx) dst[o] = (float)acc[o];
+                if (row < nrows && x + o < nx) dst[o] = acc[o];
         }
         __syncthreads();
     }
@@ -490,7 +502,7 @@ __device__ __forceinline__ size_t column_base(const Columns& c, size_t col) {
 }
 
 // One array's tile of 64 columns, positions t0 - radius ..: loaded (every load in flight before one is
-// used, addresses clamped to the line), then widened into LDS with zeros outside the line.  A pass
+// used, addresses clamped to the line), then stored into LDS with zeros outside the line.  A pass
 // over several arrays loads the next while it sums the last.
 constexpr int kStage = (kColOut + 2 * kEvalRadius + kB / 64 - 1) / (kB / 64);
 
@@ -505,21 +517,21 @@ __device__ __forceinline__ void load_columns(const float *__restrict__ src, cons
 }
 
 __device__ __forceinline__ void store_columns(const float (&v)[kStage], const Columns& c, bool col, int t0, int radius,
-                                              double *tile) {
+                                              float *tile) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rows = kColOut + 2 * radius;
 #pragma unroll
     for (int u = 0; u < kStage; ++u) {
         const int p = w + u * (kB / 64), pos = t0 - radius + p;
-        if (p < rows) tile[p * 64 + lane] = col && pos >= 0 && pos < c.L ? (double)v[u] : 0.0;
+        if (p < rows) tile[p * 64 + lane] = col && pos >= 0 && pos < c.L ? v[u] : 0.f;
     }
 }
 
 // y pass of array blockIdx.z.
 __global__ void __launch_bounds__(kB)
-k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Columns c, const double *__restrict__ kern,
+k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Columns c, const float *__restrict__ kern,
             int radius) {
-    extern __shared__ double tileD[];
+    extern __shared__ float tileF[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
     const bool col = colIdx < c.count;
@@ -527,14 +539,14 @@ k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Col
     const int t0 = blockIdx.y * kColOut;
     float v[kStage];
     load_columns(in + base, c, t0, radius, v);
-    store_columns(v, c, col, t0, radius, tileD);
+    store_columns(v, c, col, t0, radius, tileF);
     __syncthreads();
-    double acc[8];
-    conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
+    float acc[8];
+    conv8_column(tileF + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
         const int pos = t0 + w * 8 + o;
-        if (col && pos < c.L) out[base + (size_t)pos * c.lineStride] = (float)acc[o];
+        if (col && pos < c.L) out[base + (size_t)pos * c.lineStride] = acc[o];
     }
 }
 
@@ -543,9 +555,9 @@ k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Col
 template<bool GRAD>
 __global__ void __launch_bounds__(kB)
 k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, size_t N, Columns c,
-             const double *__restrict__ kern, int radius, float *__restrict__ T, double *__restrict__ partSum,
+             const float *__restrict__ kern, int radius, float *__restrict__ T, double *__restrict__ partSum,
              unsigned long long *__restrict__ partCnt) {
-    extern __shared__ double tileD[];
+    extern __shared__ float tileF[];
     __shared__ double sS[kB / 64];
     __shared__ unsigned long long sC[kB / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -555,17 +567,20 @@ k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, siz
     const int t0 = blockIdx.y * kColOut;
     float sum[6][8], v[kStage];
     load_columns(in + base, c, t0, radius, v);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        store_columns(v, c, col, t0, radius, tileD);
+    // one call an array: unrolled, so that the sums stay in registers
+    auto array = [&](auto q) __attribute__((always_inline)) {
+        store_columns(v, c, col, t0, radius, tileF);
         __syncthreads();
         if (q < 5) load_columns(in + (q + 1) * N + base, c, t0, radius, v);
-        double acc[8];
-        conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
-#pragma unroll
-        for (int o = 0; o < 8; ++o) sum[q][o] = (float)acc[o];
+        conv8_column(tileF + w * 8 * 64 + lane, kern, 2 * radius + 1, sum[q]);
         __syncthreads();
-    }
+    };
+    array(std::integral_constant<int, 0>{});
+    array(std::integral_constant<int, 1>{});
+    array(std::integral_constant<int, 2>{});
+    array(std::integral_constant<int, 3>{});
+    array(std::integral_constant<int, 4>{});
+    array(std::integral_constant<int, 5>{});
     double s = 0.0;
     unsigned long long cnt = 0;
 #pragma unroll
@@ -614,11 +629,11 @@ k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, siz
 // (not added to); the density is the one of the six sums, convolved already.
 __global__ void __launch_bounds__(kB)
 k_eval_apply(const float *__restrict__ in, const uint8_t *__restrict__ comb, const float *__restrict__ dens, size_t N,
-             Columns c, const double *__restrict__ kern, int radius, const float *__restrict__ ref,
+             Columns c, const float *__restrict__ kern, int radius, const float *__restrict__ ref,
              const float *__restrict__ war, const float *__restrict__ wgrad, const double *__restrict__ adjusted,
              float *__restrict__ grad) {
 #pragma clang fp contract(off)
-    extern __shared__ double tileD[];
+    extern __shared__ float tileF[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
     const bool col = colIdx < c.count;
@@ -628,13 +643,10 @@ k_eval_apply(const float *__restrict__ in, const uint8_t *__restrict__ comb, con
     load_columns(in + base, c, t0, radius, v);
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        store_columns(v, c, col, t0, radius, tileD);
+        store_columns(v, c, col, t0, radius, tileF);
         __syncthreads();
         if (q < 2) load_columns(in + (q + 1) * N + base, c, t0, radius, v);
-        double acc[8];
-        conv8<8 * 64, 64>(tileD + w * 8 * 64 + lane, kern, 2 * radius + 1, acc);
-#pragma unroll
-        for (int o = 0; o < 8; ++o) sum[q][o] = (float)acc[o];
+        conv8_column(tileF + w * 8 * 64 + lane, kern, 2 * radius + 1, sum[q]);
         __syncthreads();
     }
     const double aw = adjusted[0];
@@ -718,11 +730,7 @@ void ensure_lncc(nrh_f3d *h) {
             h->lnccKernOff[a] = (int)all.size();
             all.insert(all.end(), k.begin(), k.end());
         }
-        std::vector<double> wide(all.begin(), all.end());
-        wide.push_back(1.0);  // the kernel of an axis that is not smoothed
-        h->lnccKernD.alloc(wide.size());
-        NRH_HIP(hipMemcpyAsync(h->lnccKernD.p, wide.data(), wide.size() * sizeof(double), hipMemcpyHostToDevice,
-                               h->stream));
+        all.push_back(1.f);  // the evaluations' kernel of an axis that is not smoothed
         h->lnccKern.alloc(all.size());
         NRH_HIP(hipMemcpyAsync(h->lnccKern.p, all.data(), all.size() * sizeof(float), hipMemcpyHostToDevice,
                                h->stream));
@@ -774,14 +782,14 @@ float *lncc_statistics(nrh_f3d *h) {
 
 // Radius and kernel of one axis of the evaluation's passes: an axis that is not smoothed has the
 // single tap 1.
-int eval_axis(const nrh_f3d *h, int axis, const double **kern) {
+int eval_axis(const nrh_f3d *h, int axis, const float **kern) {
     const int dims[3] = { h->ref.nx, h->ref.ny, h->ref.nz };
     const int r = h->lnccRadius[axis];
     if (dims[axis] <= 1 || r <= 0) {
-        *kern = h->lnccKernD.p + (h->lnccKernD.n - 1);
+        *kern = h->lnccKern.p + (h->lnccKern.n - 1);
         return 0;
     }
-    *kern = h->lnccKernD.p + h->lnccKernOff[axis];
+    *kern = h->lnccKern.p + h->lnccKernOff[axis];
     return r;
 }
 
@@ -793,7 +801,7 @@ bool eval_tiled(const nrh_f3d *h) {
 // x then y pass of `arrays` planar arrays: in (null: the six numerators of the images) -> mid -> out.
 void eval_xy(nrh_f3d *h, const float *in, float *mid, float *out, int arrays) {
     const int nx = h->ref.nx, ny = h->ref.ny, nz = h->ref.nz, nrows = ny * nz;
-    const double *kern;
+    const float *kern;
     int r = eval_axis(h, 0, &kern);
     const dim3 rows((nrows + kEvalRows - 1) / kEvalRows, (nx + 63) / 64, in ? arrays : 1);
     if (in)
@@ -825,7 +833,7 @@ void op_lncc_eval_value(nrh_f3d *h, double *out_device) {
         h->evalVersion = keep;
         return;
     }
-    const double *kern;
+    const float *kern;
     const int r = eval_axis(h, 2, &kern);
     const Columns c = z_columns(h);
     const dim3 grid = column_grid(c, 1);
@@ -849,7 +857,7 @@ void op_lncc_eval_voxel_gradient(nrh_f3d *h, double weight) {
     ensure_voxel_grad(h);
     h->voxelGradPending = false;
     NRH_REQUIRE(!h->warpedGrad.empty(), NRH_ERR_STATE, "LNCC gradient needs the warped image gradient");
-    const double *kern;
+    const float *kern;
     const int r = eval_axis(h, 2, &kern);
     const Columns c = z_columns(h);
     const dim3 grid = column_grid(c, 1);

@@ -1,12 +1,10 @@
 """The LNCC evaluation's passes against the per-operation measure.
 
-objective / gradient convolve with fused multiply-adds and warp with the fused sweep where the grid
-allows it; the per-operation calls round every product to float as the reference does.  Bounds: a
-product rounded to float is off by 2^-24, so a convolved sum of positive terms by at most 6e-8 an
-axis, and a local variance by that times mean^2 / variance, up to about 2.5e3 on these images
-(noise 0.01 on intensities in [0, 1]): 5e-4 at single voxels.  The mean value is far closer (1e-5
-allowed), the gradient's L2 error is bounded by 1e-3.  Kernels too long for the tiled passes take
-the per-operation ones: on a grid off the voxels the results are then equal.
+objective / gradient form the same sums as the per-operation calls, every product rounded to float, in
+fewer passes: the voxel gradient is equal bit for bit, and so is the node gradient on a grid off the
+voxels.  The value adds the same per-voxel terms in another order (1e-12), and the projection onto
+nodes that lie on voxels is separable where the calls convolve the image axis by axis (1e-5, float
+sums of a few hundred terms).
 """
 import numpy as np
 import pytest
@@ -65,13 +63,38 @@ def test_evaluation_matches_per_operation_measure(gpu, dims, spacing, sigma, mas
     assert np.array_equal(got, h.node_gradient())
     want_value, want_voxel, want = _chain(h, cpp, 0.99)
     h.close()
-    exact = sigma == -11.0
-    assert abs(terms[0] / np.float32(0.99) - want_value) <= (1e-12 if exact else 1e-5) * abs(want_value)
+    assert abs(terms[0] / np.float32(0.99) - want_value) <= 1e-12 * abs(want_value)
     assert np.isfinite(got).all() and np.isfinite(vox).all() and np.abs(want).max() > 0
-    if exact:
+    if spacing == 4.6:
         assert np.array_equal(got, want)
     else:
-        assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+        assert np.array_equal(vox, want_voxel)
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("huge", [0.0, 3e15, 1e25, 3e38, np.inf])
+def test_evaluation_of_signed_and_huge_intensities(gpu, huge):
+    """Negative values, and values whose squares grow large or overflow, as they are (no rescaling)."""
+    dims = (41, 37, 35)
+    g = Geom.identity(dims)
+    rng = np.random.default_rng(11)
+    ref = phantoms.blob_phantom(dims, 1).ravel() - np.float32(0.4)
+    flo = phantoms.blob_phantom(dims, 2).ravel() - np.float32(0.6)
+    if huge:
+        ref[rng.integers(0, ref.size, 2)] = [huge, -huge]
+        flo[rng.integers(0, flo.size, 2)] = [-huge, huge]
+    cg, cpp = create_control_point_grid(g, [5.0] * 3)
+    cpp = (cpp + rng.uniform(-1, 1, cpp.size)).astype(np.float32)
+    p = default_params(similarity_weight=0.99, be_weight=0.01, measure=_lib.MEASURE_LNCC, lncc_sigma=-2.0)
+    h = F3dContent(g, ref, g, flo, cg, cpp, params=p)
+    value, terms = h.objective()
+    h.gradient()
+    vox = h.voxel_gradient()
+    want_value, want_voxel, _ = _chain(h, cpp, 0.99)
+    h.close()
+    assert abs(terms[0] / np.float32(0.99) - want_value) <= 1e-12 * abs(want_value)
+    assert np.abs(want_voxel).max() > 0
+    assert np.array_equal(vox, want_voxel, equal_nan=True)
 
 
 @pytest.mark.parametrize("dims,spacing,masked", [
