@@ -349,7 +349,10 @@ k_lncc_apply(const float *__restrict__ T, const uint8_t *__restrict__ comb, cons
 // float product, its widening and an addition in double: bound by these.  Two shifts of the product's bits
 // in place of the widening, 2^-896 scaled, took longer (281, about 305 and 314 us).  Fused multiply-adds
 // in double took 137, 175 and 205 us, but an unrounded product moves the node gradient by 1e-4.
-constexpr int kEvalRadius = 30;  // radii above take the per-operation passes (LDS rows of 64 KB)
+// Radii above take the per-operation passes.  The x pass stages two samples of a row a lane, 64 outputs and
+// the radius on each side; 30 is a sigma of 10 voxels, whose tiles take 25 KB (x) and 23.5 KB of LDS.
+constexpr int kEvalRadius = 30;
+static_assert(64 + 2 * kEvalRadius <= 128, "a row's samples are two a lane");
 constexpr int kColOut = 32;      // outputs along y / z per workgroup: four waves of 8
 constexpr int kEvalRows = 32;    // rows per workgroup of the x pass
 
