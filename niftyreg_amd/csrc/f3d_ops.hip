@@ -889,13 +889,12 @@ __global__ void k_fill_f32(float *p, size_t n, float v) {
 // and s1[0..n1) to coherent host memory followed by the sequence number seq (k_publish's
 // layout), so the objective needs no publishing kernel of its own.
 // be (may be null): the bending-energy partials of the launch before, summed into *beOut as k_be_sum
-// does.
+// does.  beOut may lie in s1, whose value is then the one published: neither is __restrict__.
 __global__ void __launch_bounds__(1024)
 k_nmi_finalize_lds(uint32_t *__restrict__ counts, int rb, int fb, double *__restrict__ pro,
                    double *__restrict__ logh, float *__restrict__ logf, double *__restrict__ ent,
                    float *__restrict__ kTab, const double *__restrict__ be, int nBe, double beScale,
-                   double *__restrict__ beOut, double *__restrict__ pub, const double *__restrict__ s1, int n1,
-                   uint64_t seq) {
+                   double *beOut, double *__restrict__ pub, const double *s1, int n1, uint64_t seq) {
     __shared__ double redBe[16];
     if (be) {
         const double t = sum_partials_256(be, nBe, redBe);

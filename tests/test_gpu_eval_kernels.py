@@ -49,6 +49,21 @@ def test_bending_energy_at_brick_edges(gpu, dims):
         h.close()
 
 
+@pytest.mark.parametrize("bins", [24, 68])
+def test_published_bending_energy_follows_the_points(gpu, bins):
+    """The finalisation sums the bending energy and publishes it from the same address: each objective
+    has the energy of its own points, not of the last ones."""
+    h, g, cg, cpp = content((40, 36, 32), bins, bins)
+    try:
+        for scale in (1.0, 3.0, 0.25, 2.0):
+            points = (cpp * np.float32(scale)).astype(np.float32)
+            h.set_control_points(points)
+            want = O.orc_be(cg, points)
+            assert abs(h.objective()[1][1] - np.float32(0.001) * want) <= 1e-9 * want
+    finally:
+        h.close()
+
+
 @pytest.mark.parametrize("rb,fb", [(8, 8), (9, 113), (113, 9), (32, 32), (33, 31), (64, 65), (88, 88), (87, 89), (90, 90)])
 def test_finalisation_over_bins(gpu, rb, fb):
     h, g, cg, cpp = content((23, 22, 21), rb, fb)
