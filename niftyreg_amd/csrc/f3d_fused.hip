@@ -1028,16 +1028,17 @@ struct FusedPlan {
     int tiles(int d) const { return tilesX * tilesY * ((nz + d - 1) / d); }
 };
 
-// Depth of a pair's own tiles, from the number of tiles across a slice and of slices.  A tile stages
-// and contracts its window before its voxels run one wave a row, so deep tiles cost least per voxel,
-// but an image of fewer 8-deep tiles than compute units leaves most of the chip idle through a long
-// tile, and one of a few tiles per unit ends in a nearly empty last round.  Histogram / gradient sweep
-// in us at depth 8, 4, 2: 64^3 (64 tiles) 31 / 34, 22 / 23, 18 / 17; 96^3 (288) 35 / 40, 31 / 35,
-// 30 / 31; 128 x 144 x 112 (504) 40 / 44, 36 / 40, 44 / 43; 160^3 (1200) 66 / 75, 59 / 73, 71 / 78;
-// 192^3 (1728) 82 / 97, 82 / 99, 96 / 109; 256 x 256 x 160 (2560) 108 / 131, 110 / 136, 133 / 154.
+// Depth of a pair's own tiles, from the number of 8-deep ones.  A tile stages and contracts its window
+// before its voxels run one wave a row, so deep tiles cost least per voxel, but few of them leave compute
+// units idle through a long tile, and 1024 are in flight at once (four workgroups a unit): a few more end in
+// a nearly empty second round.  Histogram + gradient sweep in us at depth 2, 4, 8 by tiles (64 x 8 x 8):
+//   64: 36, 46, 62    192: 50, 53, 66    256: 56, 58, 69     320: 62, 63, 76    330: 68, 64, 78
+//   504: 86, 74, 79   640: 100, 84, 92   648: 98, 96, 92     720: 105, 100, 92  1008: 132, 118, 108
+//   1056: 136, 125, 141   1224: 155, 137, 149   1440: 175, 156, 157   1584: 187, 166, 171   1932: 217, 193, 188
 static int tile_depth(int across, int nz) {
     const long deep = (long)across * ((nz + kMaxDepth - 1) / kMaxDepth);
-    return deep <= 256 ? 2 : deep <= 1536 ? 4 : kMaxDepth;
+    if (deep <= 320) return 2;
+    return deep <= 640 || (deep > 1024 && deep <= 1600) ? 4 : kMaxDepth;
 }
 
 // The plan is kept beside the handle in a side table keyed by handle address.

@@ -1,7 +1,7 @@
 """The sweeps' tile depth: a pair's own sweeps take 2, 4 or 8 slices a tile by the image's size, a
-batch's always 8.  Objective, node gradient and length of a pair alone and in a batch are equal bit
-for bit whatever the depth; the sizes lie on both sides of the rule's lines (256 and 1536 tiles of
-64 x 8 x 8) and end in partial tiles."""
+batch's always 8.  Objective, node gradient and length of a pair alone and in a batch are equal
+bit for bit whatever the depth; the sizes lie on both sides of the rule's lines (320, 640, 1024 and 1600
+tiles of 64 x 8 x 8) and end in partial tiles."""
 import numpy as np
 import pytest
 
@@ -14,10 +14,14 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dims", [
     (65, 9, 3),        # one shallow tile past each edge
-    (128, 128, 61),    # 256 tiles: depth 2
-    (128, 128, 65),    # 288: depth 4, the last tile one slice
-    (190, 176, 183),   # 1518: depth 4
-    (190, 176, 187),   # 1584: depth 8
+    (128, 128, 77),    # 320 tiles: depth 2
+    (128, 128, 81),    # 352: depth 4, the last tile one slice
+    (128, 157, 121),   # 640: depth 4
+    (190, 143, 95),    # 648: depth 8
+    (250, 121, 125),   # 1024: depth 8
+    (190, 171, 123),   # 1056: depth 4
+    (190, 176, 187),   # 1584: depth 4
+    (190, 176, 193),   # 1650: depth 8, the last tile one slice
 ])
 @pytest.mark.parametrize("storage", [0, 1])
 def test_depths_agree(gpu, dims, storage):
