@@ -6,6 +6,7 @@
 // matrix kept in device memory:
 //   k_affine_warp   field = (A * ref.sto_xyz) * voxel in FP64, trilinear warp of the floating image
 //   k_block_match   five active 4x4x4 blocks a workgroup, a lane per (y, z) of their capture offsets
+//                   (few blocks: one, a lane per offset)
 //   k_lts           one workgroup: compaction, FP64 moment fits, radix-select trimming
 // Block variances for the active-block choice are computed on the device; their heap-sort
 // ranking runs on the host because its tie order is part of the reference's result.
@@ -180,125 +181,137 @@ k_affine_warp(const float *__restrict__ flo, int fnx, int fny, int fnz, Affine f
 }
 
 // ------------------------------------------------------------------ block matching
-// block_matching_method3D<float> (reg-lib/cpu/_reg_blockMatching.cpp:455-690).  A workgroup takes
-// kMatchBlocks active blocks (neighbours: the list is in block order, as undefined values come in clusters); a lane takes one (m, n) of a block's 7 x 7 capture
-// offsets along y and z and all 7 along x, so the 10 warped values of a row are read from LDS once for
-// the 28 products that they enter.  Each offset runs the reference's two float passes (means, then
-// variances and covariance) in voxel order; a wave per block then replays the sequential
-// "cc > best -> best = cc + 1e-7" rule with ballots, which gives the same winner as the reference's
-// scan over offsets (l, m, n) = (o % 7, o / 7 % 7, o / 49) - 3.
+// block_matching_method3D<float> (reg-lib/cpu/_reg_blockMatching.cpp:455-690).  A workgroup takes NB
+// active blocks (neighbours: the list is in block order, as undefined values come in clusters); a lane
+// takes one (m, n) of a block's 7 x 7 capture offsets along y and z and NX of the 7 along x: all 7, so
+// that the 10 warped values of a row are read from LDS once for the 28 products that they enter, or one.
+// Each offset runs the reference's two float passes (means, then variances and covariance) in voxel
+// order; a wave per block then replays the sequential "cc > best -> best = cc + 1e-7" rule with ballots,
+// which gives the same winner as the reference's scan over offsets (l, m, n) = (o % 7, o / 7 % 7, o / 49) - 3.
 //
 // Bound by vector instructions: 343 offsets x 64 voxels x 6 for a block whose values are all defined
 // (its mean and variance are the same for every offset and come from one lane), 16 with a check of
 // each value otherwise; a wave takes the short way when every block it works on allows.  One offset
 // a lane, both checks always and an atomic per block on the count of defined blocks: 254 us for the
-// 16384 blocks of 128^3; so, 93 us (in rank order, which scatters the blocks with undefined values, and
-// with the coordinates of each staged value found by division, 179 us).  5 blocks fill 245 of 256 lanes.
-constexpr int kMatchBlocks = 5;
-constexpr int kMatchThreads = 256;
+// 16384 blocks of 128^3; with NB = 5 (245 of 256 lanes) and NX = 7, 93 us (in rank order, which scatters
+// the blocks with undefined values, and with the coordinates of each staged value found by division, 179
+// us).  That many blocks keep the chip busy; few of them wait for one lane's seven offsets, 28 us however
+// few, and go a block a workgroup of 384, an offset a lane (NB = NX = 1).  us by active blocks, 5 / 7 and
+// 1 / 1: 256: 28, 10; 500: 28, 14; 1008: 28, 21; 1372: 28, 26; 2048: 30, 34; 4000: 39, 56.
+constexpr int kMatchFew = 1536;
 
+template<int NB, int NX>
+struct MatchShape {
+    static constexpr int kLanes = 49 * (7 / NX);  // of a block
+    static constexpr int kThreads = (NB * kLanes + 63) / 64 * 64;
+    static constexpr int kStage = NX == 7 ? 1 : 4;  // fifties of threads that stage a block
+    static_assert(7 % NX == 0 && 50 * kStage * NB <= kThreads, "threads of a block");
+};
+
+template<int NB>
 struct MatchShared {
-    float W[kMatchBlocks][1000];    // warped values, 3 voxels around the block
-    float R[kMatchBlocks][68];      // reference values (NaN: undefined or masked)
-    float rt[kMatchBlocks][64];     // reference values less their mean (blocks without NaN)
-    float rv[kMatchBlocks];         // and the sum of their squares
-    float cc[kMatchBlocks][343];
-    int rank[kMatchBlocks];
-    int org[kMatchBlocks][3];       // first voxel
-    int bad[kMatchBlocks];          // an undefined value among R or W
+    float W[NB][1000];    // warped values, 3 voxels around the block
+    float R[NB][68];      // reference values (NaN: undefined or masked)
+    float rt[NB][64];     // reference values less their mean (blocks without NaN)
+    float rv[NB];         // and the sum of their squares
+    float cc[NB][343];
+    int rank[NB];
+    int org[NB][3];       // first voxel
+    int bad[NB];          // an undefined value among R or W
     int defined;
 };
 
-// cc of the 7 offsets along x, every value of the block and its surroundings defined.
-__device__ __forceinline__ void match_defined(const MatchShared& S, int blk, int m, int n, float (&cc)[7]) {
-#pragma clang fp contract(off)
-    const float *w0 = S.W[blk] + n * 100 + m * 10;  // rows start on even indices: pairs are aligned
-    float wm[7] = {};
-    for (int z = 0; z < 4; ++z)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            float w[10];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                const float2 v = *reinterpret_cast<const float2 *>(w0 + z * 100 + y * 10 + 2 * k);
-                w[2 * k] = v.x;
-                w[2 * k + 1] = v.y;
-            }
-#pragma unroll
-            for (int x = 0; x < 4; ++x)
-#pragma unroll
-                for (int l = 0; l < 7; ++l) wm[l] += w[l + x];
-        }
-    float wv[7] = {}, c[7] = {};
-#pragma unroll
-    for (int l = 0; l < 7; ++l) wm[l] /= 64.f;
-    for (int z = 0; z < 4; ++z)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            float w[10];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                const float2 v = *reinterpret_cast<const float2 *>(w0 + z * 100 + y * 10 + 2 * k);
-                w[2 * k] = v.x;
-                w[2 * k + 1] = v.y;
-            }
-            const float4 r4 = *reinterpret_cast<const float4 *>(&S.rt[blk][z * 16 + y * 4]);
-            const float rt[4] = { r4.x, r4.y, r4.z, r4.w };
-#pragma unroll
-            for (int x = 0; x < 4; ++x)
-#pragma unroll
-                for (int l = 0; l < 7; ++l) {
-                    const float wt = w[l + x] - wm[l];
-                    wv[l] += wt * wt;
-                    c[l] += rt[x] * wt;
-                }
-        }
-    const float rv = S.rv[blk];
-#pragma unroll
-    for (int l = 0; l < 7; ++l) cc[l] = (rv * wv[l]) > 0.f ? fabsf(c[l] / sqrtf(rv * wv[l])) : 0.f;
-}
-
-// The same over the pairs whose two values are defined (an undefined one adds 0), more than 32 of them.
-__device__ __forceinline__ void match_checked(const MatchShared& S, int blk, int m, int n, float (&cc)[7]) {
-#pragma clang fp contract(off)
-    const float *w0 = S.W[blk] + n * 100 + m * 10;
-    // a row's values and which of them are defined: one comparison each, for all that they enter
-    float w[10], r[4];
-    bool wok[10], rok[4];
-    auto row = [&](int q) {
-        const float *p = w0 + (q >> 2) * 100 + (q & 3) * 10;
+// The NX + 3 warped values of a row that NX offsets of 4 voxels take; all seven offsets' rows start on
+// even indices: pairs are aligned.
+template<int NX>
+__device__ __forceinline__ void match_row(const float *p, float (&w)[NX + 3]) {
+    if constexpr (NX == 7) {
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
             const float2 v = *reinterpret_cast<const float2 *>(p + 2 * k);
             w[2 * k] = v.x;
             w[2 * k + 1] = v.y;
         }
-        const float4 v = *reinterpret_cast<const float4 *>(&S.R[blk][q * 4]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < NX + 3; ++k) w[k] = p[k];
+    }
+}
+
+// cc of NX offsets along x from w0 (the first offset's first voxel), every value of the block and its
+// surroundings defined.
+template<int NX>
+__device__ __forceinline__ void match_defined(const float *w0, const float *rts, float rv, float (&cc)[NX]) {
+#pragma clang fp contract(off)
+    float wm[NX] = {};
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            float w[NX + 3];
+            match_row<NX>(w0 + z * 100 + y * 10, w);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int l = 0; l < NX; ++l) wm[l] += w[l + x];
+        }
+    float wv[NX] = {}, c[NX] = {};
+#pragma unroll
+    for (int l = 0; l < NX; ++l) wm[l] /= 64.f;
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            float w[NX + 3];
+            match_row<NX>(w0 + z * 100 + y * 10, w);
+            const float4 r4 = *reinterpret_cast<const float4 *>(rts + z * 16 + y * 4);
+            const float rt[4] = { r4.x, r4.y, r4.z, r4.w };
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int l = 0; l < NX; ++l) {
+                    const float wt = w[l + x] - wm[l];
+                    wv[l] += wt * wt;
+                    c[l] += rt[x] * wt;
+                }
+        }
+#pragma unroll
+    for (int l = 0; l < NX; ++l) cc[l] = (rv * wv[l]) > 0.f ? fabsf(c[l] / sqrtf(rv * wv[l])) : 0.f;
+}
+
+// The same over the pairs whose two values are defined (an undefined one adds 0), more than 32 of them.
+template<int NX>
+__device__ __forceinline__ void match_checked(const float *w0, const float *R, float (&cc)[NX]) {
+#pragma clang fp contract(off)
+    // a row's values and which of them are defined: one comparison each, for all that they enter
+    float w[NX + 3], r[4];
+    bool wok[NX + 3], rok[4];
+    auto row = [&](int q) {
+        match_row<NX>(w0 + (q >> 2) * 100 + (q & 3) * 10, w);
+        const float4 v = *reinterpret_cast<const float4 *>(R + q * 4);
         r[0] = v.x;
         r[1] = v.y;
         r[2] = v.z;
         r[3] = v.w;
 #pragma unroll
-        for (int k = 0; k < 10; ++k) wok[k] = w[k] == w[k];
+        for (int k = 0; k < NX + 3; ++k) wok[k] = w[k] == w[k];
 #pragma unroll
         for (int x = 0; x < 4; ++x) rok[x] = r[x] == r[x];
     };
-    float rm[7] = {}, wm[7] = {}, cnt[7] = {};
+    float rm[NX] = {}, wm[NX] = {}, cnt[NX] = {};
     for (int q = 0; q < 16; ++q) {
         row(q);
 #pragma unroll
         for (int x = 0; x < 4; ++x)
 #pragma unroll
-            for (int l = 0; l < 7; ++l) {
+            for (int l = 0; l < NX; ++l) {
                 const bool ok = rok[x] && wok[l + x];
                 rm[l] += ok ? r[x] : 0.f;
                 wm[l] += ok ? w[l + x] : 0.f;
                 cnt[l] += ok ? 1.f : 0.f;
             }
     }
-    float rv[7] = {}, wv[7] = {}, c[7] = {};
+    float rv[NX] = {}, wv[NX] = {}, c[NX] = {};
 #pragma unroll
-    for (int l = 0; l < 7; ++l) {
+    for (int l = 0; l < NX; ++l) {
         rm[l] /= cnt[l];
         wm[l] /= cnt[l];
     }
@@ -307,7 +320,7 @@ __device__ __forceinline__ void match_checked(const MatchShared& S, int blk, int
 #pragma unroll
         for (int x = 0; x < 4; ++x)
 #pragma unroll
-            for (int l = 0; l < 7; ++l) {
+            for (int l = 0; l < NX; ++l) {
                 const bool ok = rok[x] && wok[l + x];
                 const float rt = ok ? r[x] - rm[l] : 0.f, wt = ok ? w[l + x] - wm[l] : 0.f;
                 rv[l] += rt * rt;
@@ -316,21 +329,24 @@ __device__ __forceinline__ void match_checked(const MatchShared& S, int blk, int
             }
     }
 #pragma unroll
-    for (int l = 0; l < 7; ++l) {
+    for (int l = 0; l < NX; ++l) {
         const float v = (rv[l] * wv[l]) > 0.f ? fabsf(c[l] / sqrtf(rv[l] * wv[l])) : 0.f;
         cc[l] = cnt[l] > 32.f ? v : -1.f;
     }
 }
 
-__global__ void __launch_bounds__(kMatchThreads)
+template<int NB, int NX>
+__global__ void __launch_bounds__((MatchShape<NB, NX>::kThreads))
 k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, const int *__restrict__ mask,
               int nx, int ny, int nz, int nbx, int nby, const int2 *__restrict__ activeList, int nActive, Affine xyz,
               float *__restrict__ refPos, float *__restrict__ warpPos, int *__restrict__ definedCount) {
 #pragma clang fp contract(off)
-    __shared__ __align__(16) MatchShared S;
-    const int t = threadIdx.x, first = blockIdx.x * kMatchBlocks, nb = min(kMatchBlocks, nActive - first);
+    using Shape = MatchShape<NB, NX>;
+    constexpr int kThreads = Shape::kThreads, kLanes = Shape::kLanes, kStage = Shape::kStage;
+    __shared__ __align__(16) MatchShared<NB> S;
+    const int t = threadIdx.x, first = blockIdx.x * NB, nb = min(NB, nActive - first);
     const float qnan = __builtin_nanf("");
-    if (t < kMatchBlocks) {
+    if (t < NB) {
         const int2 a = activeList[first + min(t, nb - 1)];  // blocks past the last repeat it, unused
         S.rank[t] = a.y;
         S.org[t][0] = 4 * (a.x % nbx);
@@ -341,24 +357,23 @@ k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, c
     if (t == 0) S.defined = 0;
     __syncthreads();
     {
-        // the warped values first, all loads in flight before the first is stored: 50 threads a block,
-        // each two columns (x, y) and (x, y + 5) of its 10 slices
-        const int wb = min(t / 50, kMatchBlocks - 1), p = t % 50;
+        // the warped values first, all loads in flight before the first is stored: fifty r of a block's
+        // threads takes the halves j kStage + r of its slices, columns (x, y) or (x, y + 5)
+        const int wb = min(t / (50 * kStage), NB - 1), p = t % 50, r = t / 50 % kStage;
         const int x = S.org[wb][0] - 3 + p % 10, y = S.org[wb][1] - 3 + p / 10, z0 = S.org[wb][2] - 3;
         const bool in0 = x > -1 && x < nx && y > -1 && y < ny, in1 = x > -1 && x < nx && y + 5 > -1 && y + 5 < ny;
         const float *c0 = warped + (in0 ? (size_t)y * nx + x : 0), *c1 = warped + (in1 ? (size_t)(y + 5) * nx + x : 0);
         const size_t slice = (size_t)nx * ny;
-        float v[20];
+        constexpr int kLoads = 20 / kStage;
+        float v[kLoads];
 #pragma unroll
-        for (int u = 0; u < 10; ++u) {
-            const int z = min(max(z0 + u, 0), nz - 1);
-            v[u] = c0[z * slice];
-            v[10 + u] = c1[z * slice];
-            const bool inz = z == z0 + u;
-            if (!in0 || !inz) v[u] = qnan;
-            if (!in1 || !inz) v[10 + u] = qnan;
+        for (int j = 0; j < kLoads; ++j) {
+            const int h = j * kStage + r, zj = z0 + (h >> 1);
+            const int z = min(max(zj, 0), nz - 1);
+            v[j] = (h & 1 ? c1 : c0)[z * slice];
+            if (!(h & 1 ? in1 : in0) || z != zj) v[j] = qnan;
         }
-        for (int i = t; i < kMatchBlocks * 64; i += kMatchThreads) {
+        for (int i = t; i < NB * 64; i += kThreads) {
             const int blk = i >> 6, a = i & 63;
             const int rx = S.org[blk][0] + (a & 3), ry = S.org[blk][1] + ((a >> 2) & 3), rz = S.org[blk][2] + (a >> 4);
             float r = qnan;
@@ -369,19 +384,18 @@ k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, c
             S.R[blk][a] = r;
             if (!(r == r)) S.bad[blk] = 1;
         }
-        if (t < 50 * kMatchBlocks) {
+        if (t < 50 * kStage * NB) {
             bool bad = false;
 #pragma unroll
-            for (int u = 0; u < 10; ++u) {
-                S.W[wb][u * 100 + p] = v[u];
-                S.W[wb][u * 100 + 50 + p] = v[10 + u];
-                bad = bad || !(v[u] == v[u]) || !(v[10 + u] == v[10 + u]);
+            for (int j = 0; j < kLoads; ++j) {
+                S.W[wb][(j * kStage + r) * 50 + p] = v[j];
+                bad = bad || !(v[j] == v[j]);
             }
             if (bad) S.bad[wb] = 1;
         }
     }
     __syncthreads();
-    if (t < kMatchBlocks && !S.bad[t]) {
+    if (t < NB && !S.bad[t]) {
         const float *R = S.R[t];
         float rm = 0.f, rv = 0.f;
 #pragma unroll 16
@@ -397,15 +411,18 @@ k_block_match(const float *__restrict__ ref, const float *__restrict__ warped, c
     }
     __syncthreads();
     {
-        const int blk = min(t / 49, kMatchBlocks - 1), o = t % 49, m = o % 7, n = o / 7;
-        float cc[7];
-        if (__any(S.bad[blk])) match_checked(S, blk, m, n, cc);
-        else match_defined(S, blk, m, n, cc);
-        if (t < kMatchBlocks * 49)
-            for (int l = 0; l < 7; ++l) S.cc[blk][n * 49 + m * 7 + l] = cc[l];
+        constexpr int kX = 7 / NX;  // lanes along x
+        const int blk = min(t / kLanes, NB - 1), o = t - t / kLanes * kLanes;
+        const int l0 = o % kX * NX, m = o / kX % 7, n = o / (7 * kX);
+        const float *w0 = S.W[blk] + n * 100 + m * 10 + l0;
+        float cc[NX];
+        if (__any(S.bad[blk])) match_checked<NX>(w0, S.R[blk], cc);
+        else match_defined<NX>(w0, S.rt[blk], S.rv[blk], cc);
+        if (t < NB * kLanes)
+            for (int l = 0; l < NX; ++l) S.cc[blk][n * 49 + m * 7 + l0 + l] = cc[l];
     }
     __syncthreads();
-    for (int blk = t >> 6; blk < nb; blk += kMatchThreads / 64) {
+    for (int blk = t >> 6; blk < nb; blk += kThreads / 64) {
         const int lane = t & 63;
         float best = 0.f;
         int win = -1;
@@ -1360,12 +1377,18 @@ void launch_warp(nrh_aladin *h) {
     NRH_HIP(hipGetLastError());
 }
 
-void launch_block_matching(nrh_aladin *h) {
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, h->stream, h->counters.p);
-    hipLaunchKernelGGL(k_block_match, dim3((h->activeBlocks + kMatchBlocks - 1) / kMatchBlocks), dim3(kMatchThreads), 0,
+template<int NB, int NX>
+void launch_match(nrh_aladin *h) {
+    hipLaunchKernelGGL((k_block_match<NB, NX>), dim3((h->activeBlocks + NB - 1) / NB), dim3(MatchShape<NB, NX>::kThreads), 0,
                        h->stream, h->refImg.p, h->warped.p, h->mask.p, h->ref.nx, h->ref.ny, h->ref.nz, h->nb[0], h->nb[1],
                        h->activeList.p, h->activeBlocks, to_affine(h->ref.xyz), h->refPos.p, h->warpPos.p, h->counters.p);
     NRH_HIP(hipGetLastError());
+}
+
+void launch_block_matching(nrh_aladin *h) {
+    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, h->stream, h->counters.p);
+    if (h->activeBlocks <= kMatchFew) launch_match<1, 1>(h);
+    else launch_match<5, 7>(h);
 }
 
 void launch_lts(nrh_aladin *h, bool affine) {

@@ -1,5 +1,6 @@
-"""Block matching at the edges of its work split: five active blocks a workgroup, the short way for
-blocks whose values are all defined and the checked one beside it, against the oracle, bit for bit.
+"""Block matching at the edges of its work split: one active block a workgroup to 1536 of them, five
+above (whole and partial last workgroups), the short way for blocks whose values are all defined and the
+checked one beside it, against the oracle, bit for bit.
 """
 import numpy as np
 import pytest
@@ -12,7 +13,8 @@ from niftyreg_amd.geometry import Geom
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dims", [(8, 8, 4), (12, 12, 8), (16, 20, 8), (17, 19, 9), (24, 20, 24), (40, 33, 31)])
+@pytest.mark.parametrize("dims", [(8, 8, 4), (12, 12, 8), (16, 20, 8), (17, 19, 9), (24, 20, 24), (40, 33, 31),
+                                  (64, 64, 48), (60, 60, 56), (61, 57, 55), (64, 61, 53)])
 @pytest.mark.parametrize("holes", [0, 1, 40, "half"])
 def test_block_matching(gpu, dims, holes):
     g = Geom.identity(dims)
