@@ -216,19 +216,17 @@ __device__ __forceinline__ bool lncc_gradient_terms(const LocalStats& s, float t
     return true;
 }
 
-// The value's terms from the six convolved arrays, reduced per block in a fixed order.
-__global__ void __launch_bounds__(kB)
-k_lncc_value(const float *__restrict__ C, const uint8_t *__restrict__ comb, size_t N, double *__restrict__ partSum,
-             unsigned long long *__restrict__ partCnt) {
-#pragma clang fp contract(off)
+// The value's terms (term(i, l): whether voxel i counts, and its l), reduced per block in a fixed order.
+template<class Term>
+__device__ __forceinline__ void value_partials(size_t N, Term term, double *__restrict__ partSum,
+                                               unsigned long long *__restrict__ partCnt) {
     __shared__ double sS[kB / 64];
     __shared__ unsigned long long sC[kB / 64];
     double sum = 0.0;
     unsigned long long cnt = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (size_t)gridDim.x * blockDim.x) {
-        if (!comb[i]) continue;
         double l;
-        if (lncc_value_term(local_stats(C[i], C[N + i], C[2 * N + i], C[3 * N + i], C[4 * N + i], C[5 * N + i]), l)) {
+        if (term(i, l)) {
             sum += l;
             ++cnt;
         }
@@ -253,6 +251,18 @@ k_lncc_value(const float *__restrict__ C, const uint8_t *__restrict__ comb, size
         partSum[blockIdx.x] = s;
         partCnt[blockIdx.x] = c;
     }
+}
+
+__global__ void __launch_bounds__(kB)
+k_lncc_value(const float *__restrict__ C, const uint8_t *__restrict__ comb, size_t N, double *__restrict__ partSum,
+             unsigned long long *__restrict__ partCnt) {
+    value_partials(
+        N,
+        [&](size_t i, double& l) {
+            return comb[i] &&
+                   lncc_value_term(local_stats(C[i], C[N + i], C[2 * N + i], C[3 * N + i], C[4 * N + i], C[5 * N + i]), l);
+        },
+        partSum, partCnt);
 }
 
 // Sum of the block partials in block order; out[0] = sum / count, out[1] = count.
@@ -341,8 +351,9 @@ k_lncc_apply(const float *__restrict__ T, const uint8_t *__restrict__ comb, cons
 // ------------------------------------------------------------------ evaluation passes
 // The evaluations' convolutions: the sums of the per-operation passes, product by product, in fewer
 // trips to memory.  The x pass forms the six numerators from the two images as it stages them, with a
-// sliding window of samples in registers for eight neighbouring outputs, and the z pass ends in the value
-// or the derivative terms, so that the six arrays cross memory four times instead of ten.
+// sliding window of samples in registers for eight neighbouring outputs, and the z pass ends in the value's
+// or the derivative's terms, so that the six arrays cross memory four times instead of ten.  The value's
+// terms, one array, are added in the per-operation order by a pass of their own (20 us).
 // At 256 x 256 x 160, sigma 5 voxels (31 taps): the x, y and z passes of the six sums take 225, 219 and
 // 278 us (with the derivative's terms 305), about 300 each by the per-operation passes, with a preparing
 // and a reducing pass of 52 and 70 us; the derivative's three arrays 109, 110 and 152 us.  A tap is a
@@ -553,15 +564,14 @@ k_eval_cols(const float *__restrict__ in, float *__restrict__ out, size_t N, Col
     }
 }
 
-// z pass of the six sums, ending in the value's terms (GRAD = false: their sum and number per block)
-// or the derivative's (GRAD = true: three arrays and the convolved density into T, and their number).
+// z pass of the six sums, ending in the value's terms (GRAD = false: in T, NaN where there is none) or the
+// derivative's (GRAD = true: three arrays and the convolved density into T, and their number per block).
 template<bool GRAD>
 __global__ void __launch_bounds__(kB)
 k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, size_t N, Columns c,
-             const float *__restrict__ kern, int radius, float *__restrict__ T, double *__restrict__ partSum,
+             const float *__restrict__ kern, int radius, float *__restrict__ T,
              unsigned long long *__restrict__ partCnt) {
     extern __shared__ float tileF[];
-    __shared__ double sS[kB / 64];
     __shared__ unsigned long long sC[kB / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const size_t colIdx = (size_t)blockIdx.x * 64 + lane;
@@ -584,7 +594,6 @@ k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, siz
     array(std::integral_constant<int, 3>{});
     array(std::integral_constant<int, 4>{});
     array(std::integral_constant<int, 5>{});
-    double s = 0.0;
     unsigned long long cnt = 0;
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
@@ -602,30 +611,29 @@ k_eval_stats(const float *__restrict__ in, const uint8_t *__restrict__ comb, siz
             T[3 * N + i] = sum[5][o];
         } else {
             double l;
-            if (used && lncc_value_term(st, l)) {
-                s += l;
-                ++cnt;
-            }
+            T[i] = used && lncc_value_term(st, l) ? (float)l : __builtin_nanf("");  // l is a float's value
         }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        s += __shfl_down(s, off, 64);
-        cnt += __shfl_down(cnt, off, 64);
-    }
-    if (lane == 0) {
-        sS[w] = s;
-        sC[w] = cnt;
-    }
+    if (!GRAD) return;
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_down(cnt, off, 64);
+    if (lane == 0) sC[w] = cnt;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const size_t b = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
-        for (int k = 1; k < kB / 64; ++k) {
-            s += sS[k];
-            cnt += sC[k];
-        }
-        partSum[b] = s;
-        partCnt[b] = cnt;
+        for (int k = 1; k < kB / 64; ++k) cnt += sC[k];
+        partCnt[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = cnt;
     }
+}
+
+// The value's partials from the z pass's terms, in k_lncc_value's order.
+__global__ void __launch_bounds__(kB)
+k_eval_value(const float *__restrict__ T, size_t N, double *__restrict__ partSum, unsigned long long *__restrict__ partCnt) {
+    value_partials(
+        N,
+        [&](size_t i, double& l) {
+            l = (double)T[i];
+            return l == l;
+        },
+        partSum, partCnt);
 }
 
 // z pass of the three derivative arrays, ending in k_lncc_apply's voxel gradient, which is written
@@ -674,23 +682,14 @@ k_eval_apply(const float *__restrict__ in, const uint8_t *__restrict__ comb, con
     }
 }
 
-// Sums of the block partials, one workgroup of 1024 in a fixed order; the value (out[0] = sum /
-// count, out[1] = count) or the gradient's weight (out[0] = weight / count).
+// The gradient's weight over the number of terms, one workgroup of 1024.
 __global__ void __launch_bounds__(1024)
-k_eval_finish(const double *__restrict__ partSum, const unsigned long long *__restrict__ partCnt, int nb, int grad,
-              double weight, double *__restrict__ out) {
+k_eval_weight(const unsigned long long *__restrict__ partCnt, int nb, double weight, double *__restrict__ out) {
     __shared__ double red[16];
-    double s = 0.0, n = 0.0;  // counts below 2^53 add exactly
-    for (int b = threadIdx.x; b < nb; b += 1024) {
-        if (!grad) s += partSum[b];
-        n += (double)partCnt[b];
-    }
-    s = block_sum_double(s, red);
+    double n = 0.0;  // counts below 2^53 add exactly
+    for (int b = threadIdx.x; b < nb; b += 1024) n += (double)partCnt[b];
     n = block_sum_double(n, red);
-    if (threadIdx.x == 0) {
-        out[0] = grad ? weight / n : s / n;
-        if (!grad) out[1] = n;
-    }
+    if (threadIdx.x == 0) out[0] = weight / n;
 }
 
 // Gaussian kernel of reg_tools_kernelConvolution (:866-901); returns the radius.
@@ -840,13 +839,15 @@ void op_lncc_eval_value(nrh_f3d *h, double *out_device) {
     const int r = eval_axis(h, 2, &kern);
     const Columns c = z_columns(h);
     const dim3 grid = column_grid(c, 1);
-    const int nb = (int)eval_blocks(h);
-    double *ps = h->lnccPart.p;
-    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p + nb);
     hipLaunchKernelGGL(k_eval_stats<false>, grid, dim3(kB), eval_lds_cols(r), h->stream, h->lnccB.p, h->lnccComb.p, h->N, c,
-                       kern, r, nullptr, ps, pc);
+                       kern, r, h->lnccA.p, nullptr);
     NRH_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_eval_finish, dim3(1), dim3(1024), 0, h->stream, ps, pc, nb, 0, 0.0, out_device);
+    const unsigned nb = std::min<unsigned>(blocks_of(h->N), kRedBlocks);
+    double *ps = h->lnccPart.p;
+    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p + kRedBlocks);
+    hipLaunchKernelGGL(k_eval_value, dim3(nb), dim3(kB), 0, h->stream, h->lnccA.p, h->N, ps, pc);
+    NRH_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_lncc_finish, dim3(1), dim3(64), 0, h->stream, ps, pc, (int)nb, out_device);
     NRH_HIP(hipGetLastError());
 }
 
@@ -865,13 +866,12 @@ void op_lncc_eval_voxel_gradient(nrh_f3d *h, double weight) {
     const Columns c = z_columns(h);
     const dim3 grid = column_grid(c, 1);
     const int nb = (int)eval_blocks(h);
-    double *ps = h->lnccPart.p;
-    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p + nb);
+    auto *pc = reinterpret_cast<unsigned long long *>(h->lnccPart.p);
     float *T = h->lnccA.p, *dens = h->lnccA.p + 3 * h->N;
     hipLaunchKernelGGL(k_eval_stats<true>, grid, dim3(kB), eval_lds_cols(r), h->stream, h->lnccB.p, h->lnccComb.p, h->N, c,
-                       kern, r, T, ps, pc);
+                       kern, r, T, pc);
     NRH_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_eval_finish, dim3(1), dim3(1024), 0, h->stream, ps, pc, nb, 1, weight, h->lnccScalars.p);
+    hipLaunchKernelGGL(k_eval_weight, dim3(1), dim3(1024), 0, h->stream, pc, nb, weight, h->lnccScalars.p);
     NRH_HIP(hipGetLastError());
     // the six sums are done with: their buffer takes the terms' x and y passes
     eval_xy(h, T, h->lnccB.p, h->lnccB.p + 3 * h->N, 3);
