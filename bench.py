@@ -104,7 +104,9 @@ def bench_aladin(torch, steps, with_cpu):
     it_s = warp_s + bm_s + lts_s
     N = g.nvox
     active = h.active_blocks
-    flops = active * 343 * 64 * 11.0  # pass 1: 3 adds; pass 2: 2 sub, 3 mul, 3 add (per offset and voxel)
+    # per offset and voxel: pass 1 an add; pass 2 a subtraction, two products, two adds (the block's own
+    # mean and variance are the same for every offset)
+    flops = active * 343 * 64 * 6.0
     out = {
         "metric": "Aladin iterations/s at 128^3 (warp + block matching + LTS)",
         "value": 1.0 / it_s, "unit": "iterations/s",
@@ -140,8 +142,7 @@ def bench_aladin(torch, steps, with_cpu):
 
 
 def bench_lncc(torch, ref, flo, geom, cppg, cpp, steps, with_cpu):
-    """F3D with LNCC (Gaussian sigma 5 voxels): one objective value + one gradient at 256x256x160
-    through the per-operation chain."""
+    """F3D with LNCC (Gaussian sigma 5 voxels): one objective value + one gradient at 256x256x160."""
     from niftyreg_amd import _lib
     from niftyreg_amd.f3d import F3dContent, default_params
     h = F3dContent(geom, ref, geom, flo, cppg, cpp,
@@ -155,10 +156,12 @@ def bench_lncc(torch, ref, flo, geom, cppg, cpp, steps, with_cpu):
     h.close()
     N = geom.nvox
     # algorithmic bytes: the reference and floating images read once per sweep, two sweeps per
-    # obj+grad eval (8 B per voxel each); the design's traffic (the two statistics sets, 6 + 4
-    # planar arrays through 3 axis passes, read + write) is reported beside it
+    # obj+grad eval (8 B per voxel each); the traffic of the convolution passes is reported beside it,
+    # in planar float arrays: the six sums' x (2 in, 6 out) and y passes, their z pass for the value (6
+    # in, its terms out and in) and for the gradient (6 in, 4 out), the three terms' x and y passes, and
+    # their z pass with what it forms the voxel gradient from (3 + 6 in, 3 out)
     algo_bytes = 2 * 8 * N
-    conv_bytes = (6 + 6 + 4) * 2 * 4 * 3 * N
+    conv_bytes = (8 + 12 + 8 + 10 + 6 + 6 + 12) * 4 * N
     out = {
         "metric": "F3D LNCC obj+grad evals/s at 256x256x160", "value": 1.0 / step_s, "unit": "evals/s",
         "ms_per_step": step_s * 1e3, "lncc": terms[0] / (1.0 - BE),

@@ -870,7 +870,9 @@ __device__ __forceinline__ void lts_add_listed(const float *__restrict__ P, cons
 // fit each, so its cost is the instructions and barriers of one compute unit.  The kept points' sums
 // are carried from one iteration to the next: only points that enter or leave the set are added or
 // subtracted, gathered in a list per wave so that 64 at a time fill the lanes (all kept points summed
-// anew took as long as the residuals).  19 iterations over 16384 points 470 -> 426 us, of which the
+// anew took as long as the residuals).  What that loses in FP64 is far below the matrix's floats; but a
+// point with an infinite coordinate that is in the set once leaves its sums NaN to the end of the fit,
+// where sums formed anew would be numbers again after it left.  19 iterations over 16384 points 470 -> 426 us, of which the
 // residuals are 40 % (their conversions to and from double run at a quarter of the rate) and the digits
 // 25 %; the 1000 points of a coarse level, 4 iterations, 57 -> 42 us.
 template<int NT, bool LDS>

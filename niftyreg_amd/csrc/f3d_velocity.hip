@@ -988,8 +988,10 @@ inline dim3 blocks8_for(size_t n) { return dim3((unsigned)(((n + kBlock - 1) / k
 
 inline dim3 blocks8(size_t blocks) { return dim3((unsigned)((blocks + 7) / 8 * 8)); }
 
-// Tiles of the gathers through LDS.  Four voxels a thread read the least around a tile; a launch of
-// fewer than kTileMinimum such tiles (two a compute unit are resident) takes a voxel a thread.
+// Tiles of the gathers through LDS.  Two voxels a thread read less around a tile than one; a launch of
+// fewer than kTileMinimum such tiles, two a compute unit where four fit, takes a voxel a thread.  us a
+// launch (both directions' overlapping) with two voxels and with one, by tiles of two: 64: 10, 7;
+// 256: 10, 9; 384: 12, 11; 540: 15.0, 15.1; 576: 15, 16; 726: 16, 19; 2048: 40, 43.
 template<int VPT>
 size_t tiles_of(int nx, int ny, int nz) {
     return (size_t)((nx + kTileX - 1) / kTileX) * ((ny + kTileY - 1) / kTileY) * ((nz + 2 * VPT - 1) / (2 * VPT));

@@ -1,5 +1,5 @@
 """The gradient resampling through LDS (and the field composition) at the edges of their tiles: sizes
-below, on and past a tile of 32 x 8 x 2 or 8 voxels, fields that are the identity, whose boxes fit,
+below, on and past a tile of 32 x 8 x 2 or 4 voxels, fields that are the identity, whose boxes fit,
 whose boxes do not, that leave the image, and single undefined positions; against the oracle, bit for
 bit.
 """
